@@ -10,6 +10,7 @@
 // re-read from the caches (k+-1 is the next lane; j+-1 and i+-1 rows and planes are in
 // L2 from the neighbouring threads).  HBM-bound: per step the H update reads e and h and
 // writes h, the E update reads h and e (and eps) and writes e.
+#include <algorithm>
 #include <cstdlib>
 #include <string>
 
@@ -37,6 +38,57 @@ __device__ __forceinline__ double width_u(const double* w, int n) {
   return w ? ((const MX_CONST double*)w)[n] : 1.0;
 }
 
+// x / d given rd = 1 / d: one product, its exact residual and one correction, then the
+// divide fix-up instruction for zeros, infinities and NaN.  The value rounded at the end
+// is within 2^-20 ulp of the quotient (2^-50 in float64), so the result is the correctly
+// rounded quotient in all but about one of 10^6 (10^15) near-ties.  4 instructions at full
+// rate; the compiler's divide takes 9 (float32) or 13 (float64) of that issue time.
+__device__ __forceinline__ double div_by(double x, double d, double rd) {
+  const double q = x * rd;
+  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-q, d, x), rd, q), d, x);
+}
+__device__ __forceinline__ float div_by(float x, float d, float rd) {
+  const float q = x * rd;
+  return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-q, d, x), rd, q), d, x);
+}
+
+// 1 / d to within an ulp, for div_by: the hardware's reciprocal and Newton steps
+__device__ __forceinline__ double recip(double d) {
+  double r = __builtin_amdgcn_rcp(d);
+  r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+  return __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+}
+__device__ __forceinline__ float recip(float d) {
+  const float r = __builtin_amdgcn_rcpf(d);
+  return __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
+}
+
+// value of the next / previous lane of the wave (DPP wave shifts; the end lanes get 0)
+template <int CTRL> __device__ __forceinline__ float lane_shift(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL> __device__ __forceinline__ double lane_shift(double v) {
+  typedef int __attribute__((ext_vector_type(2))) I2;
+  const I2 w = __builtin_bit_cast(I2, v);
+  I2 r;
+  r.x = __builtin_amdgcn_update_dpp(0, w.x, CTRL, 0xf, 0xf, true);
+  r.y = __builtin_amdgcn_update_dpp(0, w.y, CTRL, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, r);
+}
+// a value that is the same in every lane, as a scalar (SGPRs)
+__device__ __forceinline__ float wave_value(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+}
+__device__ __forceinline__ double wave_value(double v) {
+  typedef int __attribute__((ext_vector_type(2))) I2;
+  I2 w = __builtin_bit_cast(I2, v);
+  w.x = __builtin_amdgcn_readfirstlane(w.x);
+  w.y = __builtin_amdgcn_readfirstlane(w.y);
+  return __builtin_bit_cast(double, w);
+}
+template <typename T> __device__ __forceinline__ T lane_next(T v) { return lane_shift<0x130>(v); }
+template <typename T> __device__ __forceinline__ T lane_prev(T v) { return lane_shift<0x138>(v); }
+
 template <typename T>
 __global__ __launch_bounds__(kFB) void k_fdtd_h(RGrid g, T dt, const T* __restrict__ e, T* __restrict__ h,
                                                 const T* __restrict__ mu, T mu_s) {
@@ -47,15 +99,16 @@ __global__ __launch_bounds__(kFB) void k_fdtd_h(RGrid g, T dt, const T* __restri
     const int sy = (j + 1 == g.ny ? -j : 1) * g.nz;
     const int sz = (k + 1 == g.nz ? -k : 1);
     const T dx = (T)width(g.dxe[0], i), dy = (T)width(g.dxe[1], j), dz = (T)width(g.dxe[2], k);
+    const T rx = T(1) / dx, ry = T(1) / dy, rz = T(1) / dz;
     const T ex = e[cell], ey = e[nc + cell], ez = e[2 * nc + cell];
-    const T cx = (e[2 * nc + cell + sy] - ez) / dy - (e[nc + cell + sz] - ey) / dz;
-    const T cy = (e[cell + sz] - ex) / dz - (e[2 * nc + cell + sx] - ez) / dx;
-    const T cz = (e[nc + cell + sx] - ey) / dx - (e[cell + sy] - ex) / dy;
+    const T cx = div_by(e[2 * nc + cell + sy] - ez, dy, ry) - div_by(e[nc + cell + sz] - ey, dz, rz);
+    const T cy = div_by(e[cell + sz] - ex, dz, rz) - div_by(e[2 * nc + cell + sx] - ez, dx, rx);
+    const T cz = div_by(e[nc + cell + sx] - ey, dx, rx) - div_by(e[cell + sy] - ex, dy, ry);
     const T c[3] = {cx, cy, cz};
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
       const T m = mu ? mu[q * nc + cell] : mu_s;
-      h[q * nc + cell] -= dt * c[q] / m;
+      h[q * nc + cell] -= div_by(dt * c[q], m, recip(m));
     }
   }
 }
@@ -70,247 +123,256 @@ __global__ __launch_bounds__(kFB) void k_fdtd_e(RGrid g, T dt, T* __restrict__ e
     const int sy = (j == 0 ? g.ny - 1 : -1) * g.nz;
     const int sz = (k == 0 ? g.nz - 1 : -1);
     const T dx = (T)width(g.dxh[0], i), dy = (T)width(g.dxh[1], j), dz = (T)width(g.dxh[2], k);
+    const T rx = T(1) / dx, ry = T(1) / dy, rz = T(1) / dz;
     const T hx = h[cell], hy = h[nc + cell], hz = h[2 * nc + cell];
-    const T cx = (hz - h[2 * nc + cell + sy]) / dy - (hy - h[nc + cell + sz]) / dz;
-    const T cy = (hx - h[cell + sz]) / dz - (hz - h[2 * nc + cell + sx]) / dx;
-    const T cz = (hy - h[nc + cell + sx]) / dx - (hx - h[cell + sy]) / dy;
+    const T cx = div_by(hz - h[2 * nc + cell + sy], dy, ry) - div_by(hy - h[nc + cell + sz], dz, rz);
+    const T cy = div_by(hx - h[cell + sz], dz, rz) - div_by(hz - h[2 * nc + cell + sx], dx, rx);
+    const T cz = div_by(hy - h[nc + cell + sx], dx, rx) - div_by(hx - h[cell + sy], dy, ry);
     const T c[3] = {cx, cy, cz};
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
       const T m = eps ? eps[q * nc + cell] : eps_s;
-      e[q * nc + cell] += dt * c[q] / m;
+      e[q * nc + cell] += div_by(dt * c[q], m, recip(m));
     }
   }
 }
-
-// ---- fused leapfrog step (mx_fdtd_run) ----------------------------------------------
-// One pass per step: H' = H - dt curl_f(E) / mu, then E' = E + dt curl_b(H') / eps, read
-// from (e0, h0) and written to (e1, h1).  The two buffer pairs alternate between steps,
-// so no block ever reads a half-updated field: 5 field streams per step instead of the
-// 7 of two separate updates.  A block owns a TY x 64 (y, z) tile and marches along x
-// over `slab` planes.  Per plane i:
-//   - E(i) of the tile plus a one-cell halo sits in LDS; plane i+1 comes from the
-//     registers of the threads that loaded it: each thread loads exactly the plane-i+1
-//     values its own H computations need (own cell; wave 0 the row j0-1 whose H it forms;
-//     lanes 0..TY-1 of wave TY-1 the column k0-1 whose H they form);
-//   - H'(i) is formed on the tile, the -y row and the -z column (the halo cells
-//     redundantly with the neighbouring blocks, by the same expressions) into LDS;
-//   - E'(i) takes H'(i) from LDS and H'(i-1) of its own cell from registers.
-// The expressions are those of k_fdtd_h and k_fdtd_e, so a run equals the step-by-step
-// updates bit for bit.  Partial tiles wrap their row and column indices (periodic grid),
-// so every load is in bounds and every neighbour read is the periodic one.
-// Tile rows (waves per block) of the fused step.  At 256^3: 8 rows 429 us (float64) /
-// 263 us (float32) per step, 4 rows 433 / 282 us, 2 rows 452 / 291 us (fewer re-read
-// halo rows per computed row).
-#ifndef MX_FDTD_TY
-#define MX_FDTD_TY 8
-#endif
-constexpr int kStepTY = MX_FDTD_TY;
-constexpr int kStepSlab = 16;
 
 __device__ __forceinline__ int wrap(int v, int n) {
   const int r = v % n;
   return r < 0 ? r + n : r;
 }
 
-template <typename T>
-__global__ __launch_bounds__(64 * kStepTY) void k_fdtd_step(RGrid g, T dt, const T* __restrict__ e0,
-                                                            const T* __restrict__ h0, T* __restrict__ e1,
-                                                            T* __restrict__ h1, const T* __restrict__ eps, T eps_s,
-                                                            const T* __restrict__ mu, T mu_s, int slab) {
-  constexpr int TY = kStepTY, TZ = 64, LY = TY + 2, LZ = TZ + 2;
-  static_assert(2 * TY + 2 <= 64, "the z-halo loads take 2 TY + 2 lanes of one wave");
-  __shared__ T sE[3][LY][LZ];
-  __shared__ T sH[3][TY + 1][TZ + 1];
+// ---- leapfrog steps (mx_fdtd_run) ----------------------------------------------------
+// One pass does S steps (1 or 2): E_0, H_0 and the materials are read once, E_S and H_S
+// written once into a second buffer pair (the pairs alternate between passes, so no block
+// ever reads a half-updated field).  Two steps a pass halve the bytes per step.
+//
+// A block is W waves; its lanes are 64 consecutive z cells and its rows W consecutive y
+// cells, S of each on every side being halo that the neighbouring blocks compute as well
+// (all indices wrap, so every lane holds a cell of the periodic grid).  It marches along x
+// over `slab` planes: in iteration i, stage s (1..S) forms H_s and E_s, the fields after s
+// steps, of plane i - 2 (s - 1):
+//   phase 1:  H_s = H_{s-1} - dt curl_f(E_{s-1}) / mu     (all stages)
+//   phase 2:  E_s = E_{s-1} + dt curl_b(H_s) / eps        (all stages)
+// z neighbours come from the next lane, y neighbours through LDS (two components of E and
+// of H per stage, one barrier per phase); x neighbours and the planes on their way from
+// one stage to the next stay in the thread's registers.  E_0, H_0 and the materials are
+// loaded one iteration ahead into alternating register sets, so nothing waits for a load
+// in the iteration that issues it.  Only the last stage is stored, by the lanes and rows
+// that are not halo: each stage's fields are valid one cell further in than those of the
+// stage before.  The expressions are those of k_fdtd_h and k_fdtd_e without contraction,
+// so a run equals the step-by-step updates bit for bit.
+//
+// Bound by the divisions' issue (58% of the time at 256^3 in float64) together with the
+// reads, 1.36 times the algorithmic ones with the halos.  Per step of a run (in brackets
+// with passes of one step and compiler divides): 256^3 float64 281 us (435), 256^3 float32
+// 148 us (266), 190 x 160 x 201 float32 57 us (129).  12 rows: 8 rows recompute half of
+// theirs (330 / 170 us at 256^3), 16 rows leave float64 128 VGPRs of the 142 it needs
+// (396 / 155 us).  Three steps a pass spill in float64 and gain nothing in float32 (159
+// us), since the halo grows with each.  Two rows per thread measured 285 / 161 us.
+constexpr int kStepRows = 12;
+constexpr int kStepMaxSlab = 128;
+constexpr int kStepTab = 136;    // planes of the x table: the slab and the pipeline's run-in
+enum : int { MU_ONE = 0, MU_SCALAR = 1, MU_FIELD = 2 };
+
+template <typename T, int S, bool EPS, int MU>
+__global__ __launch_bounds__(64 * kStepRows) void k_fdtd_steps(RGrid g, T dt, const T* __restrict__ e0,
+                                                               const T* __restrict__ h0, T* __restrict__ e1,
+                                                               T* __restrict__ h1, const T* __restrict__ eps,
+                                                               T eps_s, const T* __restrict__ mu, T mu_s, int slab) {
+#pragma clang fp contract(off)
+  constexpr int W = kStepRows, OY = W - 2 * S, OZ = 64 - 2 * S;
+  __shared__ T sE[S][2][W + 1][64];   // E_{s-1} x, z by row
+  __shared__ T sH[S][2][W + 1][64];   // H_s x, z by row + 1
+  __shared__ T sX[kStepTab][4];       // dx_e, 1 / dx_e, dx_h, 1 / dx_h by plane
   const int nx = g.nx, ny = g.ny, nz = g.nz;
   const int nc = nx * ny * nz, plane = ny * nz;
-  const int ntj = (ny + TY - 1) / TY, ntk = (nz + TZ - 1) / TZ, tiles = ntj * ntk;
+  const int ntj = (ny + OY - 1) / OY, ntk = (nz + OZ - 1) / OZ, tiles = ntj * ntk;
   const int nwork = ((nx + slab - 1) / slab) * tiles;
-  // workgroups are dealt round-robin to the 8 XCDs: XCD x takes work items
-  // [x * per, (x + 1) * per), neighbouring tiles of one slab, so halos hit its own L2
+  // workgroups are dealt round-robin to the 8 XCDs: XCD x takes a contiguous run of work
+  // items, neighbouring tiles of one slab, so that the halos they share are in its own L2
   const int per = (nwork + 7) / 8;
   const int w = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
   if (w >= nwork) return;
   const int slab_id = w / tiles, tile = w - slab_id * tiles;
-  const int j0 = (tile / ntk) * TY, k0 = (tile % ntk) * TZ;
+  const int j0 = (tile / ntk) * OY, k0 = (tile % ntk) * OZ;
   const int ib = slab_id * slab, ie = min(ib + slab, nx);
   const int tz = threadIdx.x, ty = __builtin_amdgcn_readfirstlane(threadIdx.y);
-  const int j = j0 + ty, k = k0 + tz;
-  const bool valid = j < ny && k < nz;
+  const int j = j0 + ty - S, k = k0 + tz - S;
+  const bool valid = ty >= S && ty < W - S && tz >= S && tz < 64 - S && j < ny && k < nz;
   const int jw = wrap(j, ny), kw = wrap(k, nz);
-
-  // load sites: own cell; y-halo row (wave 0: row j0-1, wave TY-1: row j0+TY); z-halo
-  // cells (wave TY-1: lanes 0..TY column k0-1 at LDS rows 1..TY+1, lanes TY+1..2TY+1
-  // column k0+TZ at LDS rows 0..TY)
-  const int own_off = jw * nz + kw;
-  const bool has_row = ty == 0 || ty == TY - 1;
-  const int row_j = wrap(ty == 0 ? j0 - 1 : j0 + TY, ny);
-  const int row_off = row_j * nz + kw;
-  const int row_r = ty == 0 ? 0 : TY + 1;
-  const bool has_col = ty == TY - 1 && tz < 2 * TY + 2;
-  const int col_r = tz < TY + 1 ? tz + 1 : tz - (TY + 1);
-  const int col_q = tz < TY + 1 ? 0 : TZ + 1;
-  const int col_j = wrap(j0 - 1 + col_r, ny), col_k = wrap(col_q ? k0 + TZ : k0 - 1, nz);
-  const int col_off = col_j * nz + col_k;
-  const bool row_h = ty == 0;                    // forms H' of row j0-1 (x, z components)
-  const bool col_h = ty == TY - 1 && tz < TY;    // forms H' of column k0-1, row j0+tz (x, y)
-
-  // widths of the cells this thread forms H' / E' at
-  const T dye = (T)width(g.dxe[1], jw), dze = (T)width(g.dxe[2], kw);
-  const T dyh = (T)width(g.dxh[1], jw), dzh = (T)width(g.dxh[2], kw);
-  const T dye_r = (T)width(g.dxe[1], row_j);
-  const T dye_c = (T)width(g.dxe[1], col_j), dze_c = (T)width(g.dxe[2], col_k);
-
-  // What step i needs besides LDS: E(i+1) at the load sites, H(i) and mu(i) where this
-  // thread forms H', eps(i) at its own cell.
-  struct Bundle {
-    T eo[3], er[3], ec[3];   // E(i+1): own, row, column site
-    T ho[3], hr[2], hc[2];   // H(i): own; row site (x, z); column site (x, y)
-    T mo[3], mr[2], mc[2];   // mu(i) at the same cells
-    T ep[3];                 // eps(i), own cell
+  // byte offsets within one component are 32-bit (the host keeps it below 4 GiB): an SGPR
+  // base per component and one VGPR offset per plane
+  const unsigned own = (unsigned)(jw * nz + kw) * (unsigned)sizeof(T);
+  const unsigned pbytes = (unsigned)plane * (unsigned)sizeof(T);
+  auto ld = [&](const T* f, int c, unsigned off) -> T {
+    return *(const MX_GLOBAL T*)((const MX_GLOBAL char*)(f + (size_t)c * nc) + off);
   };
-  auto mat = [&](const T* m, T ms, int idx) -> T { return m ? m[idx] : ms; };
-  auto fetch = [&](Bundle& B, int i) {   // plane i+1 of E, plane i of H, mu and eps
-    const int pn = wrap(i + 1, nx) * plane, pi = i * plane;
+  auto st = [&](T* f, int c, unsigned off, T v) {
+    *(MX_GLOBAL T*)((MX_GLOBAL char*)(f + (size_t)c * nc) + off) = v;
+  };
+
+  // iterations t = 0..nt-1 hold plane first + t in stage 1; stage s trails by 2 (s - 1)
+  const int first = ib - S, nt = (ie - ib) + 3 * S - 2;
+  constexpr int kLag = 2 * (S - 1);
+  for (int t = ty * 64 + tz; t < nt + kLag; t += 64 * W) {
+    const int n = wrap(first - kLag + t, nx);
+    const T de = (T)width(g.dxe[0], n), dh = (T)width(g.dxh[0], n);
+    sX[t][0] = de;
+    sX[t][1] = T(1) / de;
+    sX[t][2] = dh;
+    sX[t][3] = T(1) / dh;
+  }
+  const T dye = (T)width_u(g.dxe[1], jw), dyh = (T)width_u(g.dxh[1], jw);
+  const T rye = wave_value(T(1) / dye), ryh = wave_value(T(1) / dyh);
+  const T dze = (T)width(g.dxe[2], kw), dzh = (T)width(g.dxh[2], kw);
+  const T rze = T(1) / dze, rzh = T(1) / dzh;
+  const T rmu = wave_value(recip(mu_s)), reps = wave_value(recip(eps_s));
+
+  struct In { T e[3], h[3], ep[3], m[3]; };   // E_0 of plane i+1; H_0, eps, mu of plane i
+  In A, B;
+  T Ec[S][3];                  // E_{s-1} of the stage's plane
+  T En[S][3];                  // and of the next one (stage 1 has it in the In)
+  T H1[S][3], H2[S][3];        // H_s of the plane before, and of the one before that
+  T ep[2 * S - 1][3], er[2 * S - 1][3];   // eps of plane i, i-1, ... and its reciprocal
+  T mm[2 * S - 1][3], mr[2 * S - 1][3];   // mu likewise
 #pragma unroll
-    for (int c = 0; c < 3; ++c) B.eo[c] = e0[c * nc + pn + own_off];
-    if (has_row) {
+  for (int c = 0; c < 3; ++c) {
 #pragma unroll
-      for (int c = 0; c < 3; ++c) B.er[c] = e0[c * nc + pn + row_off];
-    }
-    if (has_col) {
+    for (int s = 0; s < S; ++s) Ec[s][c] = En[s][c] = H1[s][c] = H2[s][c] = T(0);
 #pragma unroll
-      for (int c = 0; c < 3; ++c) B.ec[c] = e0[c * nc + pn + col_off];
-    }
+    for (int q = 0; q < 2 * S - 1; ++q) ep[q][c] = er[q][c] = mm[q][c] = mr[q][c] = T(1);
+  }
+  int pn = wrap(first, nx);    // the plane of H_0 and the materials in the next fetch
+  auto fetch = [&](In& I) {
+    const int p1 = pn + 1 == nx ? 0 : pn + 1;
+    const unsigned o1 = (unsigned)p1 * pbytes + own, o0 = (unsigned)pn * pbytes + own;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      B.ho[c] = h0[c * nc + pi + own_off];
-      B.mo[c] = mat(mu, mu_s, c * nc + pi + own_off);
-      B.ep[c] = mat(eps, eps_s, c * nc + pi + own_off);
+      I.e[c] = ld(e0, c, o1);
+      I.h[c] = ld(h0, c, o0);
+      if constexpr (EPS) I.ep[c] = ld(eps, c, o0);
+      if constexpr (MU == MU_FIELD) I.m[c] = ld(mu, c, o0);
     }
-    if (row_h) {
-      B.hr[0] = h0[pi + row_off];
-      B.hr[1] = h0[2 * nc + pi + row_off];
-      B.mr[0] = mat(mu, mu_s, pi + row_off);
-      B.mr[1] = mat(mu, mu_s, 2 * nc + pi + row_off);
-    }
-    if (col_h) {
-      B.hc[0] = h0[pi + col_off];
-      B.hc[1] = h0[nc + pi + col_off];
-      B.mc[0] = mat(mu, mu_s, pi + col_off);
-      B.mc[1] = mat(mu, mu_s, nc + pi + col_off);
+    pn = p1;
+  };
+#pragma unroll
+  for (int c = 0; c < 3; ++c) Ec[0][c] = ld(e0, c, (unsigned)pn * pbytes + own);
+  fetch(A);
+  auto put_e = [&]() {
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      sE[s][0][ty][tz] = Ec[s][0];
+      sE[s][1][ty][tz] = Ec[s][2];
     }
   };
-  auto put_e = [&](int i) {   // E(i) at the load sites into LDS (plane-i values of the bundle)
-    const int p = i * plane;
+  // rows that no wave writes, read only for halo values that are never used
+  if (ty == 0) {
 #pragma unroll
-    for (int c = 0; c < 3; ++c) sE[c][ty + 1][tz + 1] = e0[c * nc + p + own_off];
-    if (has_row) {
-#pragma unroll
-      for (int c = 0; c < 3; ++c) sE[c][row_r][tz + 1] = e0[c * nc + p + row_off];
-    }
-    if (has_col) {
-#pragma unroll
-      for (int c = 0; c < 3; ++c) sE[c][col_r][col_q] = e0[c * nc + p + col_off];
-    }
-  };
-  auto commit = [&](const Bundle& B) {   // E(i+1) from the bundle into LDS
-#pragma unroll
-    for (int c = 0; c < 3; ++c) sE[c][ty + 1][tz + 1] = B.eo[c];
-    if (has_row) {
-#pragma unroll
-      for (int c = 0; c < 3; ++c) sE[c][row_r][tz + 1] = B.er[c];
-    }
-    if (has_col) {
-#pragma unroll
-      for (int c = 0; c < 3; ++c) sE[c][col_r][col_q] = B.ec[c];
-    }
-  };
-
-  Bundle B;
-  T hpy, hpz;   // H'(i-1) y, z at the own cell
-  const int r = ty + 1, q = tz + 1;
-  // ---- prologue: H'(ib-1) at the own cell (y, z), plane ib into LDS
-  {
-    const int im1 = wrap(ib - 1, nx);
-    put_e(im1);
-    fetch(B, im1);   // E(ib), H(ib-1), mu(ib-1)
-    __syncthreads();
-    const T dx = (T)width(g.dxe[0], im1);
-    const T cy = (sE[0][r][q + 1] - sE[0][r][q]) / dze - (B.eo[2] - sE[2][r][q]) / dx;
-    const T cz = (B.eo[1] - sE[1][r][q]) / dx - (sE[0][r + 1][q] - sE[0][r][q]) / dye;
-    hpy = B.ho[1] - dt * cy / B.mo[1];
-    hpz = B.ho[2] - dt * cz / B.mo[2];
-    __syncthreads();
-    commit(B);       // plane ib
-    fetch(B, ib);    // E(ib+1), H(ib), mu(ib), eps(ib)
+    for (int s = 0; s < S; ++s) sE[s][0][W][tz] = sE[s][1][W][tz] = sH[s][0][0][tz] = sH[s][1][0][tz] = T(0);
   }
+  put_e();
+  __syncthreads();
 
-  // float32: the x widths of the next plane are read one step ahead with scalar loads
-  // (as vector loads at the top of the step they are waited for right there, a memory
-  // round trip per plane): 246 against 255-257 us per 256^3 step.  float64 keeps the
-  // vector loads: ahead of time its step measured 432 against 427 us, and carried in the
-  // prefetch bundle the widths took it over 128 VGPRs (a wave per SIMD less, 504 us).
-  constexpr bool kAheadWidths = sizeof(T) == 4;
-  double wxe_n = kAheadWidths ? width_u(g.dxe[0], ib) : 0.0, wxh_n = kAheadWidths ? width_u(g.dxh[0], ib) : 0.0;
-#pragma unroll 1
-  for (int i = ib; i < ie; ++i) {
-    __syncthreads();   // E(i) is in LDS; the previous step's reads of sH are done
-    const T dxe_i = (T)(kAheadWidths ? wxe_n : width(g.dxe[0], i));
-    const T dxh_i = (T)(kAheadWidths ? wxh_n : width(g.dxh[0], i));
-    const T e_own[3] = {sE[0][r][q], sE[1][r][q], sE[2][r][q]};
-    const T epsv[3] = {B.ep[0], B.ep[1], B.ep[2]};
-    // H'(i): own cell
-    {
-      const T cx = (sE[2][r + 1][q] - e_own[2]) / dye - (sE[1][r][q + 1] - e_own[1]) / dze;
-      const T cy = (sE[0][r][q + 1] - e_own[0]) / dze - (B.eo[2] - e_own[2]) / dxe_i;
-      const T cz = (B.eo[1] - e_own[1]) / dxe_i - (sE[0][r + 1][q] - e_own[0]) / dye;
-      const T hn[3] = {B.ho[0] - dt * cx / B.mo[0], B.ho[1] - dt * cy / B.mo[1], B.ho[2] - dt * cz / B.mo[2]};
+  auto step = [&](const int t, In& cur, In& nxt) {
+    fetch(nxt);
+    // phase 1
+    T hs[S][3];
+    if constexpr (MU == MU_FIELD) {
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
-        sH[c][r][q] = hn[c];
-        if (valid) h1[c * nc + i * plane + own_off] = hn[c];
+        mm[0][c] = cur.m[c];
+        mr[0][c] = recip(cur.m[c]);
       }
     }
-    if (row_h) {   // row j0-1 (LDS row 0): x and z
-      const T cx = (sE[2][1][q] - sE[2][0][q]) / dye_r - (sE[1][0][q + 1] - sE[1][0][q]) / dze;
-      const T cz = (B.er[1] - sE[1][0][q]) / dxe_i - (sE[0][1][q] - sE[0][0][q]) / dye_r;
-      sH[0][0][q] = B.hr[0] - dt * cx / B.mr[0];
-      sH[2][0][q] = B.hr[1] - dt * cz / B.mr[1];
-    }
-    if (col_h) {   // column k0-1 (LDS column 0), row j0+tz: x and y
-      const int rr = tz + 1;
-      const T cx = (sE[2][rr + 1][0] - sE[2][rr][0]) / dye_c - (sE[1][rr][1] - sE[1][rr][0]) / dze_c;
-      const T cy = (sE[0][rr][1] - sE[0][rr][0]) / dze_c - (B.ec[2] - sE[2][rr][0]) / dxe_i;
-      sH[0][rr][0] = B.hc[0] - dt * cx / B.mc[0];
-      sH[1][rr][0] = B.hc[1] - dt * cy / B.mc[1];
-    }
-    __syncthreads();   // H'(i) is in LDS; every read of E(i) is done
-    if (i + 1 < ie) {
-      commit(B);          // E(i+1) replaces E(i)
-      fetch(B, i + 1);    // E(i+2), H(i+1), mu(i+1), eps(i+1)
-    }
-    // E'(i): own cell
-    {
-      const T hx = sH[0][r][q], hy = sH[1][r][q], hz = sH[2][r][q];
-      const T cx = (hz - sH[2][r - 1][q]) / dyh - (hy - sH[1][r][q - 1]) / dzh;
-      const T cy = (hx - sH[0][r][q - 1]) / dzh - (hz - hpz) / dxh_i;
-      const T cz = (hy - hpy) / dxh_i - (hx - sH[0][r - 1][q]) / dyh;
-      const T c3[3] = {cx, cy, cz};
-      if (valid) {
 #pragma unroll
-        for (int c = 0; c < 3; ++c) e1[c * nc + i * plane + own_off] = e_own[c] + dt * c3[c] / epsv[c];
+    for (int s = 0; s < S; ++s) {
+      const T* xt = sX[t + kLag - 2 * s];
+      const T dx = xt[0], rx = xt[1];
+      const T (&ec)[3] = Ec[s];
+      const T (&en)[3] = s == 0 ? cur.e : En[s];
+      const T ex_y = sE[s][0][ty + 1][tz], ez_y = sE[s][1][ty + 1][tz];
+      const T ex_z = lane_next(ec[0]), ey_z = lane_next(ec[1]);
+      const T cc[3] = {div_by(ez_y - ec[2], dye, rye) - div_by(ey_z - ec[1], dze, rze),
+                       div_by(ex_z - ec[0], dze, rze) - div_by(en[2] - ec[2], dx, rx),
+                       div_by(en[1] - ec[1], dx, rx) - div_by(ex_y - ec[0], dye, rye)};
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const T hb = s == 0 ? cur.h[c] : H2[s > 0 ? s - 1 : 0][c];
+        T up = dt * cc[c];   // mu = 1: the quotient is the dividend
+        if constexpr (MU == MU_FIELD) up = div_by(up, mm[2 * s][c], mr[2 * s][c]);
+        if constexpr (MU == MU_SCALAR) up = div_by(up, mu_s, rmu);
+        hs[s][c] = hb - up;
       }
-      hpy = hy;
-      hpz = hz;
+      sH[s][0][ty + 1][tz] = hs[s][0];
+      sH[s][1][ty + 1][tz] = hs[s][2];
     }
-    // the next plane's widths, at the end of the step: scalar loads share the wait
-    // counter of LDS reads, so issued at the top they made its first LDS read wait
-    if (kAheadWidths && i + 1 < ie) {
-      wxe_n = width_u(g.dxe[0], i + 1);
-      wxh_n = width_u(g.dxh[0], i + 1);
+    __syncthreads();
+    // phase 2
+    T es[S][3];
+    if constexpr (EPS) {
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        ep[0][c] = cur.ep[c];
+        er[0][c] = recip(cur.ep[c]);
+      }
     }
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const T* xt = sX[t + kLag - 2 * s];
+      const T dx = xt[2], rx = xt[3];
+      const T hx = hs[s][0], hy = hs[s][1], hz = hs[s][2];
+      const T hx_y = sH[s][0][ty][tz], hz_y = sH[s][1][ty][tz];
+      const T hx_z = lane_prev(hx), hy_z = lane_prev(hy);
+      const T cc[3] = {div_by(hz - hz_y, dyh, ryh) - div_by(hy - hy_z, dzh, rzh),
+                       div_by(hx - hx_z, dzh, rzh) - div_by(hz - H1[s][2], dx, rx),
+                       div_by(hy - H1[s][1], dx, rx) - div_by(hx - hx_y, dyh, ryh)};
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const T up = EPS ? div_by(dt * cc[c], ep[2 * s][c], er[2 * s][c]) : div_by(dt * cc[c], eps_s, reps);
+        es[s][c] = Ec[s][c] + up;
+      }
+    }
+    const int out = first + t - kLag;   // plane of the last stage
+    if (valid && out >= ib && out < ie) {
+      const unsigned o = (unsigned)out * pbytes + own;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        st(e1, c, o, es[S - 1][c]);
+        st(h1, c, o, hs[S - 1][c]);
+      }
+    }
+    // hand the planes on
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        H2[s][c] = H1[s][c];
+        H1[s][c] = hs[s][c];
+        Ec[s][c] = s == 0 ? cur.e[c] : En[s][c];
+        if (s > 0) En[s][c] = es[s > 0 ? s - 1 : 0][c];
+      }
+#pragma unroll
+      for (int q = 2 * S - 2; q > 0; --q) {
+        ep[q][c] = ep[q - 1][c];
+        er[q][c] = er[q - 1][c];
+        mm[q][c] = mm[q - 1][c];
+        mr[q][c] = mr[q - 1][c];
+      }
+    }
+    put_e();
+    // the barrier ends the step: as the first instruction of the loop it came without the
+    // wait for the LDS writes of the step before (read in the assembly of this build), and
+    // a row's old values were read now and then
+    __syncthreads();
+  };
+  int t = 0;
+#pragma unroll 1
+  for (; t + 1 < nt; t += 2) {
+    step(t, A, B);
+    step(t + 1, B, A);
   }
+  if (t < nt) step(t, A, B);
 }
 
 // ---- convolutional PML (fdtd/pml.py:96-230) ---------------------------------------
@@ -659,32 +721,73 @@ hipError_t launch_cpml(const RGrid& v, int prec, int psi_prec, double dt, const 
   return hipGetLastError();
 }
 
-// `steps` fused steps, (e, h) -> (e2, h2) -> (e, h) -> ...
-hipError_t launch_steps(const RGrid& v, int prec, double dt, void* e, void* h, void* e2, void* h2, const void* eps,
-                        double eps_s, const void* mu, double mu_s, int steps, hipStream_t s) {
+// Slab depth of a pass: the one with the least modelled time.  A block takes slab + 3 S - 2
+// iterations; per iteration the n blocks that a CU gets (256 CUs) cost n, plus a fifth of
+// one where two blocks share it (float32) that a lone block cannot hide.  Measured at
+// 256^3 float64, two steps: slabs 16/24/32/48/64/128 model 200/196/180/208/204/264, time
+// 611/576/542/595/572/696 us.
+int step_slab(const RGrid& v, int steps, size_t elem) {
   static const int forced = [] {   // MEANAS_AMD_FDTD_SLAB overrides the slab depth (tuning runs)
     const char* env = getenv("MEANAS_AMD_FDTD_SLAB");
     return env ? atoi(env) : 0;
   }();
-  const int want = forced > 0 ? forced : kStepSlab;
-  const int slab = v.nx < want ? v.nx : want;
-  const long long tiles = (long long)((v.ny + kStepTY - 1) / kStepTY) * ((v.nz + 63) / 64);
-  const long long nwork = (long long)((v.nx + slab - 1) / slab) * tiles;
+  if (forced > 0) return std::min(std::min(forced, kStepMaxSlab), v.nx);
+  const long long tiles = (long long)((v.ny + kStepRows - 2 * steps - 1) / (kStepRows - 2 * steps)) *
+                          ((v.nz + 63 - 2 * steps) / (64 - 2 * steps));
+  int best = 1;
+  double best_cost = 0.0;
+  for (int want : {4, 6, 8, 12, 16, 24, 32, 48, 64, 96, kStepMaxSlab}) {
+    const int slab = std::min(want, v.nx);
+    const long long blocks = tiles * ((v.nx + slab - 1) / slab);
+    const double n = (double)((blocks + 255) / 256) + (elem == 4 ? 0.2 : 0.0);
+    const double cost = n * (slab + 3 * steps - 2);
+    if (best_cost == 0.0 || cost < best_cost) {
+      best_cost = cost;
+      best = slab;
+    }
+  }
+  return best;
+}
+
+template <typename T, int S>
+hipError_t launch_pass(const RGrid& v, T dt, const void* ei, const void* hi, void* eo, void* ho, const void* eps,
+                       double eps_s, const void* mu, double mu_s, hipStream_t s) {
+  static_assert(kStepMaxSlab + 5 * S - 4 <= kStepTab, "x table");
+  const int slab = step_slab(v, S, sizeof(T));
+  const long long tiles =
+      (long long)((v.ny + kStepRows - 2 * S - 1) / (kStepRows - 2 * S)) * ((v.nz + 63 - 2 * S) / (64 - 2 * S));
+  const long long nwork = tiles * ((v.nx + slab - 1) / slab);
   const unsigned nb = (unsigned)(((nwork + 7) / 8) * 8);
-  for (int t = 0; t < steps; ++t) {
+#define MX_STEP_CASE(EPS, MU)                                                                                   \
+  hipLaunchKernelGGL((k_fdtd_steps<T, S, EPS, MU>), dim3(nb), dim3(64, kStepRows), 0, s, v, dt, (const T*)ei,   \
+                     (const T*)hi, (T*)eo, (T*)ho, (const T*)eps, (T)eps_s, (const T*)mu, (T)mu_s, slab)
+  if (mu) { if (eps) MX_STEP_CASE(true, MU_FIELD); else MX_STEP_CASE(false, MU_FIELD); }
+  else if (mu_s == 1.0) { if (eps) MX_STEP_CASE(true, MU_ONE); else MX_STEP_CASE(false, MU_ONE); }
+  else { if (eps) MX_STEP_CASE(true, MU_SCALAR); else MX_STEP_CASE(false, MU_SCALAR); }
+#undef MX_STEP_CASE
+  return hipGetLastError();
+}
+
+// passes of a run: two steps each, a last single step if their number is odd
+int step_passes(int steps) { return steps / 2 + steps % 2; }
+
+// `steps` steps, (e, h) -> (e2, h2) -> (e, h) -> ... by passes
+hipError_t launch_steps(const RGrid& v, int prec, double dt, void* e, void* h, void* e2, void* h2, const void* eps,
+                        double eps_s, const void* mu, double mu_s, int steps, hipStream_t s) {
+  const int passes = step_passes(steps);
+  for (int t = 0; t < passes; ++t) {
     void* ei = (t & 1) ? e2 : e;
     void* hi = (t & 1) ? h2 : h;
     void* eo = (t & 1) ? e : e2;
     void* ho = (t & 1) ? h : h2;
+    const bool two = 2 * t + 2 <= steps;
+    hipError_t err;
     if (prec == MX_REAL64)
-      hipLaunchKernelGGL(k_fdtd_step<double>, dim3(nb), dim3(64, kStepTY), 0, s, v, dt, (const double*)ei,
-                         (const double*)hi, (double*)eo, (double*)ho, (const double*)eps, eps_s, (const double*)mu,
-                         mu_s, slab);
+      err = two ? launch_pass<double, 2>(v, dt, ei, hi, eo, ho, eps, eps_s, mu, mu_s, s)
+                : launch_pass<double, 1>(v, dt, ei, hi, eo, ho, eps, eps_s, mu, mu_s, s);
     else
-      hipLaunchKernelGGL(k_fdtd_step<float>, dim3(nb), dim3(64, kStepTY), 0, s, v, (float)dt, (const float*)ei,
-                         (const float*)hi, (float*)eo, (float*)ho, (const float*)eps, (float)eps_s, (const float*)mu,
-                         (float)mu_s, slab);
-    const hipError_t err = hipGetLastError();
+      err = two ? launch_pass<float, 2>(v, (float)dt, ei, hi, eo, ho, eps, eps_s, mu, mu_s, s)
+                : launch_pass<float, 1>(v, (float)dt, ei, hi, eo, ho, eps, eps_s, mu, mu_s, s);
     if (err != hipSuccess) return err;
   }
   return hipSuccess;
@@ -726,14 +829,22 @@ int mx_fdtd_run(const mx_fdtd_grid* g, int32_t prec, double dt, void* e, void* h
   if (steps < 0) return mx::set_error("mx_fdtd_run: steps < 0");
   if (steps == 0) return 0;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  // fused steps alternate between (e, h) and a second pair, allocated in stream order
-  const size_t bytes = (size_t)3 * v.nx * v.ny * v.nz * (prec == MX_REAL64 ? 8 : 4);
+  const size_t comp = (size_t)v.nx * v.ny * v.nz * (prec == MX_REAL64 ? 8 : 4), bytes = 3 * comp;
+  if (comp >= (size_t)1 << 32) {   // beyond the passes' 32-bit offsets: the separate updates
+    for (int t = 0; t < steps; ++t) {
+      hipError_t err = mx::launch_h(v, prec, dt, e, h, mu, mu_scalar, s);
+      if (err == hipSuccess) err = mx::launch_e(v, prec, dt, e, h, eps, eps_scalar, s);
+      if (err != hipSuccess) return mx::set_error(std::string("mx_fdtd_run: ") + hipGetErrorString(err));
+    }
+    return 0;
+  }
+  // passes alternate between (e, h) and a second pair, allocated in stream order
   void* e2 = nullptr;
   void* h2 = nullptr;
   hipError_t err = hipMallocAsync(&e2, bytes, s);
   if (err == hipSuccess) err = hipMallocAsync(&h2, bytes, s);
   if (err == hipSuccess) err = mx::launch_steps(v, prec, dt, e, h, e2, h2, eps, eps_scalar, mu, mu_scalar, steps, s);
-  if (err == hipSuccess && (steps & 1)) {   // the last step wrote the second pair
+  if (err == hipSuccess && (mx::step_passes(steps) & 1)) {   // the last pass wrote the second pair
     err = hipMemcpyAsync(e, e2, bytes, hipMemcpyDeviceToDevice, s);
     if (err == hipSuccess) err = hipMemcpyAsync(h, h2, bytes, hipMemcpyDeviceToDevice, s);
   }

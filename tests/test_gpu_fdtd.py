@@ -66,6 +66,55 @@ def test_run_matches_steps_and_oracle(shape, steps, dtype):
     numpy.testing.assert_allclose(h2, h3, rtol=1e-11, atol=1e-12)
 
 
+@pytest.mark.parametrize('shape', [(2, 8, 60), (5, 9, 61), (1, 7, 59), (130, 16, 121), (3, 2, 2), (6, 25, 1)])
+@pytest.mark.parametrize('eps_kind,mu_kind', [('field', None), ('field', 'field'), ('field', 'scalar'), ('scalar', None),
+                                              ('scalar', 'field')])
+@pytest.mark.parametrize('dtype', [numpy.float64, numpy.float32])
+@pytest.mark.parametrize('steps', [1, 2, 3])
+def test_run_passes_at_tile_edges(shape, eps_kind, mu_kind, dtype, steps):
+    """Passes of two steps and a last one of one: tiles of 8 (one step: 10) rows and 60 (62)
+    cells with remainders 0 and 1, several slabs, and every material form, against the
+    separate updates bit for bit."""
+    from meanas_amd import fdtd
+    e, h, eps, mu, dxes = _fields(shape, 3, dtype)
+    eps = eps if eps_kind == 'field' else 2.5
+    mu = mu if mu_kind == 'field' else 1.7 if mu_kind == 'scalar' else None
+    dt = 0.2
+    et, ht = torch.from_numpy(e.copy()).cuda(), torch.from_numpy(h.copy()).cuda()
+    fdtd.run(et, ht, eps, dt, dxes, steps=steps, mu=mu)
+    me, mh = fdtd.maxwell_e(dt, dxes), fdtd.maxwell_h(dt, dxes)
+    e2, h2 = torch.from_numpy(e.copy()).cuda(), torch.from_numpy(h.copy()).cuda()
+    for _ in range(steps):
+        mh(e2, h2, mu)
+        me(e2, h2, eps)
+    assert torch.equal(et, e2) and torch.equal(ht, h2)
+
+
+@pytest.mark.parametrize('dtype', [numpy.float64, numpy.float32])
+def test_updates_keep_infinities_zeros_and_nan(dtype):
+    """Infinite fields and materials, zero and NaN values divide as numpy divides them."""
+    from meanas_amd import fdtd
+    shape = (6, 12, 70)
+    e, h, eps, mu, dxes = _fields(shape, 5, dtype)
+    e[1, 2, 3, 4] = numpy.inf
+    e[2, 4, 9, 65] = numpy.nan
+    h[0, 1, 1, 1] = -numpy.inf
+    eps[:, 3, 5, 20] = numpy.inf
+    eps[0, 5, 11, 30] = 0.0
+    mu[2, 1, 10, 40] = numpy.inf
+    # float32 numpy updates keep the float64 widths' precision, so they round differently
+    tol = 1e-12 if dtype == numpy.float64 else 1e-4
+    with numpy.errstate(all='ignore'):
+        e1, h1 = e.copy(), h.copy()
+        for _ in range(2):
+            ref.maxwell_h(0.2, dxes)(e1, h1, mu)
+            ref.maxwell_e(0.2, dxes)(e1, h1, eps)
+    et, ht = torch.from_numpy(e.copy()).cuda(), torch.from_numpy(h.copy()).cuda()
+    fdtd.run(et, ht, eps, 0.2, dxes, steps=2, mu=mu)
+    numpy.testing.assert_allclose(et.cpu().numpy(), e1, rtol=tol, atol=tol)
+    numpy.testing.assert_allclose(ht.cpu().numpy(), h1, rtol=tol, atol=tol)
+
+
 def test_unit_widths_scalar_materials_and_float32():
     from meanas_amd import fdtd
     shape = (8, 6, 66)
