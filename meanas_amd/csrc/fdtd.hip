@@ -38,6 +38,47 @@ __device__ __forceinline__ double width_u(const double* w, int n) {
   return w ? ((const MX_CONST double*)w)[n] : 1.0;
 }
 
+// A thread's column of a kernel that marches along x: cell t = j nz + k of the (y, z)
+// plane and the planes [ib, ie) of one slab.  Consecutive threads take consecutive cells
+// of the flattened plane (no lanes lost on short or odd rows), and the work items (plane
+// pieces of kFB cells, slab by slab) are dealt so that each XCD -- workgroups go round the
+// 8 of them -- has a contiguous run, whose neighbouring rows and planes meet in its L2.
+struct Column {
+  int j, k, t, ib, ie;
+  bool ok;
+};
+__device__ __forceinline__ Column column(const RGrid& g, int slab) {
+  const int plane = g.ny * g.nz, pieces = (plane + kFB - 1) / kFB;
+  const int nwork = pieces * ((g.nx + slab - 1) / slab), per = (nwork + 7) / 8;
+  const int w = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+  const int s = w / pieces, piece = w - s * pieces;
+  Column c;
+  c.t = piece * kFB + (int)threadIdx.x;
+  c.ok = (int)(blockIdx.x / 8) < per && w < nwork && c.t < plane;
+  c.j = c.t / g.nz;
+  c.k = c.t - c.j * g.nz;
+  c.ib = s * slab;
+  c.ie = min(c.ib + slab, g.nx);
+  return c;
+}
+// element of `f` at a uniform element offset plus a thread's byte offset: with a 32-bit OFF
+// one load from an SGPR base and a VGPR offset
+template <typename T, typename OFF>
+__device__ __forceinline__ T at(const T* f, size_t base, OFF off) {
+  return *(const MX_GLOBAL T*)((const MX_GLOBAL char*)(f + base) + off);
+}
+// A thread offset that does not change in a loop, as if it did: otherwise its extension to
+// 64 bits is hoisted, and the loads take per-thread 64-bit addresses (two registers and an
+// addition each) instead of an SGPR base and the offset.
+template <typename OFF> __device__ __forceinline__ OFF in_loop(OFF off) {
+  asm volatile("" : "+v"(off));
+  return off;
+}
+template <typename T, typename OFF>
+__device__ __forceinline__ void put(T* f, size_t base, OFF off, T v) {
+  *(MX_GLOBAL T*)((MX_GLOBAL char*)(f + base) + off) = v;
+}
+
 // x / d given rd = 1 / d: one product, its exact residual and one correction, then the
 // divide fix-up instruction for zeros, infinities and NaN.  The value rounded at the end
 // is within 2^-20 ulp of the quotient (2^-50 in float64), so the result is the correctly
@@ -385,77 +426,165 @@ __global__ __launch_bounds__(64 * kStepRows) void k_fdtd_steps(RGrid g, T dt, co
 // float64 widths: differences of field values in the field precision, divided by the
 // float64 width, so derivatives, psi updates and the final sum are double; dt / material
 // is taken in the material's (field) precision, dt / scalar in double.
-struct CpmlLayer {
-  int axis, start, thickness;
-  const double* pe;
-  const double* ph;
-  void* psie;
-  void* psih;
+//
+// A thread owns one (y, z) column and marches along x over `slab` planes (see Column): the
+// index divisions, the neighbour offsets, the y and z widths and the layer positions are
+// per thread, the plane's are uniform, and the x neighbour comes from the thread's own
+// registers.  Every array index of the derivatives is a constant (the layers are visited
+// by face; a layer loop with run-time indexes put them into LDS), and the psi values and
+// profiles a thread needs are loaded with the fields, not one dependent load after another
+// in the layer's branch.  The widths divide through their reciprocals.
+// Bound by latency at 4-5 waves per SIMD and by the traffic (48 and 36 B a cell in float32
+// for the E and H updates, psi aside).  E + H update, 8-cell layers on all faces, per step:
+// 150 x 141 x 130 float32 63 us (106 with a thread per cell), float64 85 us (120); 256^3
+// float32 364 us (506), float64 622 us (666).
+struct CpmlFace {
+  int start, thickness;   // thickness 0: no layer on this face
+  const double* p;        // p0, p1, p2, `thickness` values each
+  void* psi;
 };
-struct CpmlTable {
-  int n;
-  CpmlLayer l[MX_CPML_MAX_LAYERS];
-};
+struct CpmlTable { CpmlFace f[MX_CPML_MAX_LAYERS]; };   // by 2 axis + (polarity > 0)
 
-template <typename T, typename TP, bool EUPD>
-__global__ __launch_bounds__(kFB) void k_cpml(RGrid g, T dt, T* __restrict__ e, T* __restrict__ h,
-                                              const T* __restrict__ mat, double mat_s, double dt64, CpmlTable tab) {
-  const int nc = g.nx * g.ny * g.nz;
-  const int dims[3] = {g.nx, g.ny, g.nz};
-  const int strides[3] = {g.ny * g.nz, g.nz, 1};
-  const T* f = EUPD ? h : e;
-  T* out = EUPD ? e : h;
-  for (int cell = blockIdx.x * kFB + threadIdx.x; cell < nc; cell += gridDim.x * kFB) {
-    const int k = cell % g.nz, t = cell / g.nz, j = t % g.ny, i = t / g.ny;
-    const int idx[3] = {i, j, k};
-    // d[a][c]: derivative along a of component c (E update: backward of h; H: forward of e)
-    double d[3][3];
+// One layer along axis A at its cell, with profiles p and psi values (u, v) in q.
+template <int A, typename TP>
+__device__ __forceinline__ void cpml_layer(const double (&p)[3], TP (&q)[2], double (&d)[3][3], TP (&aux)[3]) {
+  constexpr int u = A == 0 ? 1 : 0, v = A == 2 ? 1 : 2;
+  d[A][u] *= p[2];
+  d[A][v] *= p[2];
+  q[0] = (TP)((double)q[0] * p[0]);
+  q[1] = (TP)((double)q[1] * p[0]);
+  q[0] = (TP)((double)q[0] + p[1] * d[A][v]);
+  q[1] = (TP)((double)q[1] + p[1] * d[A][u]);
+  const TP sg = A == 1 ? TP(1) : TP(-1);
+  aux[u] = aux[u] + sg * q[0];
+  aux[v] = aux[v] + (-sg) * q[1];
+}
+
+template <typename T, typename TP, bool EUPD, typename OFF>
+__global__ __launch_bounds__(kFB) void k_cpml(RGrid g, T dt, const T* __restrict__ f, T* __restrict__ out,
+                                              const T* __restrict__ mat, double const_scale, CpmlTable tab, int slab) {
+  const Column c = column(g, slab);
+  if (!c.ok) return;
+  const int nx = g.nx, ny = g.ny, nz = g.nz, plane = ny * nz;
+  const size_t nc = (size_t)nx * plane;
+  // neighbours of the difference: the cell before (E update) or after (H update)
+  const int jn = EUPD ? (c.j == 0 ? ny - 1 : c.j - 1) : (c.j + 1 == ny ? 0 : c.j + 1);
+  const int kn = EUPD ? (c.k == 0 ? nz - 1 : c.k - 1) : (c.k + 1 == nz ? 0 : c.k + 1);
+  const OFF own0 = (OFF)c.t * (OFF)sizeof(T);
+  const OFF oy0 = ((OFF)jn * (OFF)nz + (OFF)c.k) * (OFF)sizeof(T), oz0 = ((OFF)c.j * (OFF)nz + (OFF)kn) * (OFF)sizeof(T);
+  const double wy = width(g.dxh[1], c.j), wz = width(g.dxh[2], c.k);
+  const double ry = 1.0 / wy, rz = 1.0 / wz;
+  // the thread's place in the y and z layers: whether it lies in one, its profiles, its
+  // byte offset in a plane of the layer's psi
+  bool in_y[2], in_z[2];
+  OFF fy0[2], fz0[2];
+  double ly[2][3], lz[2][3];
 #pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      const double w = width(g.dxh[a], idx[a]);
-      const int s = EUPD ? (idx[a] == 0 ? (dims[a] - 1) * strides[a] : -strides[a])
-                         : (idx[a] + 1 == dims[a] ? -idx[a] * strides[a] : strides[a]);
+  for (int q = 0; q < 2; ++q) {
+    const CpmlFace &Y = tab.f[2 + q], &Z = tab.f[4 + q];
+    const int py = c.j - Y.start, pz = c.k - Z.start;
+    in_y[q] = (unsigned)py < (unsigned)Y.thickness;
+    in_z[q] = (unsigned)pz < (unsigned)Z.thickness;
+    fy0[q] = ((OFF)py * (OFF)nz + (OFF)c.k) * (OFF)sizeof(TP);
+    fz0[q] = ((OFF)c.j * (OFF)Z.thickness + (OFF)pz) * (OFF)sizeof(TP);
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        if (c == a) continue;
-        const T here = f[c * nc + cell], there = f[c * nc + cell + s];
-        d[a][c] = (double)(EUPD ? here - there : there - here) / w;
+    for (int n = 0; n < 3; ++n) {
+      ly[q][n] = in_y[q] ? Y.p[n * Y.thickness + py] : 0.0;
+      lz[q][n] = in_z[q] ? Z.p[n * Z.thickness + pz] : 0.0;
+    }
+  }
+
+  // x: the plane carried along is i - 1 of y, z (E update) or i of all (H update)
+  T car[3];
+  {
+    const int ip = EUPD ? (c.ib == 0 ? nx - 1 : c.ib - 1) : c.ib;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) car[q] = at(f, q * nc + (size_t)ip * plane, own0);
+  }
+#pragma unroll 1
+  for (int i = c.ib; i < c.ie; ++i) {
+    const OFF own = in_loop(own0), oy = in_loop(oy0), oz = in_loop(oz0), op = in_loop((OFF)c.t * (OFF)sizeof(TP));
+    const OFF fy[2] = {in_loop(fy0[0]), in_loop(fy0[1])}, fz[2] = {in_loop(fz0[0]), in_loop(fz0[1])};
+    const size_t pi = (size_t)i * plane;
+    const size_t pl = EUPD ? pi : (size_t)(i + 1 == nx ? 0 : i + 1) * plane;
+    T ld[3], o[3], m[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) ld[q] = at(f, q * nc + pl, own);
+    const T y0 = at(f, pi, oy), y2 = at(f, 2 * nc + pi, oy), z0 = at(f, pi, oz), z1 = at(f, nc + pi, oz);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      o[q] = at((const T*)out, q * nc + pi, own);
+      m[q] = mat ? at(mat, q * nc + pi, own) : T(1);
+    }
+    // psi of the layers the cell lies in, loaded with the fields
+    TP sx[2][2], sy[2][2], sz[2][2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const CpmlFace &X = tab.f[q], &Y = tab.f[2 + q], &Z = tab.f[4 + q];
+      if ((unsigned)(i - X.start) < (unsigned)X.thickness) {
+        const size_t r = (size_t)(i - X.start) * plane;
+        sx[q][0] = at((const TP*)X.psi, r, op);
+        sx[q][1] = at((const TP*)X.psi, r + (size_t)X.thickness * plane, op);
+      }
+      if (in_y[q]) {
+        sy[q][0] = at((const TP*)Y.psi, (size_t)i * Y.thickness * nz, fy[q]);
+        sy[q][1] = at((const TP*)Y.psi, (size_t)(nx + i) * Y.thickness * nz, fy[q]);
+      }
+      if (in_z[q]) {
+        sz[q][0] = at((const TP*)Z.psi, (size_t)i * ny * Z.thickness, fz[q]);
+        sz[q][1] = at((const TP*)Z.psi, (size_t)(nx + i) * ny * Z.thickness, fz[q]);
       }
     }
+    const double wx = width_u(g.dxh[0], i), rx = recip(wx);
+    const T (&here)[3] = EUPD ? ld : car;
+    const T (&xn)[3] = EUPD ? car : ld;
+    auto dif = [](T a, T b, double w, double r) { return div_by((double)(EUPD ? a - b : b - a), w, r); };
+    double d[3][3];
+    d[0][1] = dif(here[1], xn[1], wx, rx);
+    d[0][2] = dif(here[2], xn[2], wx, rx);
+    d[1][0] = dif(here[0], y0, wy, ry);
+    d[1][2] = dif(here[2], y2, wy, ry);
+    d[2][0] = dif(here[0], z0, wz, rz);
+    d[2][1] = dif(here[1], z1, wz, rz);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) car[q] = ld[q];
     TP aux[3] = {TP(0), TP(0), TP(0)};
-    for (int q = 0; q < tab.n; ++q) {
-      const CpmlLayer& L = tab.l[q];
-      const int a = L.axis;
-      const int pos = idx[a] - L.start;
-      if (pos < 0 || pos >= L.thickness) continue;
-      const int u = a == 0 ? 1 : 0, v = a == 2 ? 1 : 2;
-      const double* p = EUPD ? L.pe : L.ph;
-      const double p0 = p[pos], p1 = p[L.thickness + pos], p2 = p[2 * L.thickness + pos];
-      d[a][u] *= p2;
-      d[a][v] *= p2;
-      // index in the layer's C-order sub-grid (its axis `thickness` cells long)
-      int sub[3] = {i, j, k}, sd[3] = {g.nx, g.ny, g.nz};
-      sub[a] = pos;
-      sd[a] = L.thickness;
-      const int r = (sub[0] * sd[1] + sub[1]) * sd[2] + sub[2];
-      const int rn = sd[0] * sd[1] * sd[2];
-      TP* psi = reinterpret_cast<TP*>(EUPD ? L.psie : L.psih);
-      TP pu = (TP)((double)psi[r] * p0), pv = (TP)((double)psi[rn + r] * p0);
-      pu = (TP)((double)pu + p1 * d[a][v]);
-      pv = (TP)((double)pv + p1 * d[a][u]);
-      psi[r] = pu;
-      psi[rn + r] = pv;
-      const TP sg = a == 1 ? TP(1) : TP(-1);
-      aux[u] = aux[u] + sg * pu;
-      aux[v] = aux[v] + (-sg) * pv;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const CpmlFace& X = tab.f[q];
+      const int pos = i - X.start;
+      if ((unsigned)pos < (unsigned)X.thickness) {
+        const double p[3] = {width_u(X.p, pos), width_u(X.p, X.thickness + pos), width_u(X.p, 2 * X.thickness + pos)};
+        cpml_layer<0, TP>(p, sx[q], d, aux);
+        const size_t r = (size_t)pos * plane;
+        put((TP*)X.psi, r, op, sx[q][0]);
+        put((TP*)X.psi, r + (size_t)X.thickness * plane, op, sx[q][1]);
+      }
     }
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      const int c1 = (c + 1) % 3, c2 = (c + 2) % 3;
-      const double curl = (d[c1][c2] - d[c2][c1]) + (double)aux[c];
-      const double scale = mat ? (double)(dt / mat[c * nc + cell]) : dt64 / mat_s;
-      const double o = (double)out[c * nc + cell];
-      out[c * nc + cell] = (T)(EUPD ? o + scale * curl : o - scale * curl);
+    for (int q = 0; q < 2; ++q) {
+      const CpmlFace& Y = tab.f[2 + q];
+      if (in_y[q]) {
+        cpml_layer<1, TP>(ly[q], sy[q], d, aux);
+        put((TP*)Y.psi, (size_t)i * Y.thickness * nz, fy[q], sy[q][0]);
+        put((TP*)Y.psi, (size_t)(nx + i) * Y.thickness * nz, fy[q], sy[q][1]);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const CpmlFace& Z = tab.f[4 + q];
+      if (in_z[q]) {
+        cpml_layer<2, TP>(lz[q], sz[q], d, aux);
+        put((TP*)Z.psi, (size_t)i * ny * Z.thickness, fz[q], sz[q][0]);
+        put((TP*)Z.psi, (size_t)(nx + i) * ny * Z.thickness, fz[q], sz[q][1]);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const int c1 = (q + 1) % 3, c2 = (q + 2) % 3;
+      const double curl = (d[c1][c2] - d[c2][c1]) + (double)aux[q];
+      const double scale = mat ? (double)div_by(dt, m[q], recip(m[q])) : const_scale;
+      put(out, q * nc + pi, own, (T)(EUPD ? (double)o[q] + scale * curl : (double)o[q] - scale * curl));
     }
   }
 }
@@ -683,11 +812,11 @@ hipError_t launch_poynting_div(const RGrid& v, int prec, const void* sv, void* d
 
 // Layer table of a CPML update: faces in increasing (axis, polarity) order (the order
 // the reference accumulates in), each inside the grid, with its arrays.
-bool cpml_table(const RGrid& v, const mx_cpml_layer* layers, int n, CpmlTable* tab, std::string* why) {
+bool cpml_table(const RGrid& v, const mx_cpml_layer* layers, int n, bool eupd, CpmlTable* tab, std::string* why) {
   if (n < 0 || n > MX_CPML_MAX_LAYERS) { *why = "nlayers must be 0..6"; return false; }
   if (n > 0 && !layers) { *why = "null layer table"; return false; }
   const int dims[3] = {v.nx, v.ny, v.nz};
-  tab->n = n;
+  for (CpmlFace& f : tab->f) f = CpmlFace{0, 0, nullptr, nullptr};
   int prev = -1;
   for (int q = 0; q < n; ++q) {
     const mx_cpml_layer& L = layers[q];
@@ -698,24 +827,42 @@ bool cpml_table(const RGrid& v, const mx_cpml_layer* layers, int n, CpmlTable* t
     if (key <= prev) { *why = "layers must be in increasing (axis, polarity) order, one per face"; return false; }
     prev = key;
     if (!L.p_e || !L.p_h || !L.psi_e || !L.psi_h) { *why = "null layer array"; return false; }
-    tab->l[q] = CpmlLayer{L.axis, L.polarity < 0 ? 0 : dims[L.axis] - L.thickness, L.thickness, L.p_e, L.p_h,
-                          L.psi_e, L.psi_h};
+    tab->f[key] = CpmlFace{L.polarity < 0 ? 0 : dims[L.axis] - L.thickness, L.thickness, eupd ? L.p_e : L.p_h,
+                           eupd ? L.psi_e : L.psi_h};
   }
   return true;
 }
 
+// Launch of a column kernel: slabs of 16 planes, shallower (down to 4) while the chip has
+// fewer than 8 blocks per CU.
+struct ColumnGrid { int slab; unsigned blocks; };
+ColumnGrid column_grid(const RGrid& v) {
+  const long long pieces = ((long long)v.ny * v.nz + kFB - 1) / kFB;
+  int slab = 16;
+  while (slab > 4 && pieces * ((v.nx + slab - 1) / slab) < 2048) slab /= 2;
+  slab = std::min(slab, v.nx);
+  const long long nwork = pieces * ((v.nx + slab - 1) / slab);
+  return {slab, (unsigned)((nwork + 7) / 8 * 8)};
+}
+// whether the byte offsets of a plane fit 32 bits (beyond: kernels with 64-bit offsets)
+bool small_plane(const RGrid& v, int prec) {
+  return (unsigned long long)v.ny * v.nz * (prec == MX_REAL64 ? 8 : 4) < (1ull << 32);
+}
+
 template <bool EUPD>
-hipError_t launch_cpml(const RGrid& v, int prec, int psi_prec, double dt, const void* e, const void* h,
+hipError_t launch_cpml(const RGrid& v, int prec, int psi_prec, double dt, const void* f, void* out,
                        const void* mat, double mat_s, const CpmlTable& tab, hipStream_t s) {
-#define MX_CPML_CASE(T, TP)                                                                                  \
-  hipLaunchKernelGGL((k_cpml<T, TP, EUPD>), dim3(blocks(v)), dim3(kFB), 0, s, v, (T)dt, (T*)e, (T*)h,       \
-                     (const T*)mat, mat_s, dt, tab)
+  const ColumnGrid cg = column_grid(v);
+#define MX_CPML_CASE(T, TP, OFF)                                                                              \
+  hipLaunchKernelGGL((k_cpml<T, TP, EUPD, OFF>), dim3(cg.blocks), dim3(kFB), 0, s, v, (T)dt, (const T*)f, (T*)out, \
+                     (const T*)mat, dt / mat_s, tab, cg.slab)
+  const bool small = small_plane(v, prec);
   if (prec == MX_REAL64) {
-    if (psi_prec == MX_REAL64) MX_CPML_CASE(double, double);
-    else MX_CPML_CASE(double, float);
-  } else {
-    if (psi_prec == MX_REAL64) MX_CPML_CASE(float, double);
-    else MX_CPML_CASE(float, float);
+    if (psi_prec == MX_REAL64) { if (small) MX_CPML_CASE(double, double, unsigned); else MX_CPML_CASE(double, double, size_t); }
+    else { if (small) MX_CPML_CASE(double, float, unsigned); else MX_CPML_CASE(double, float, size_t); }
+  } else {   // a float32 plane is always below 4 GiB (3 N < 2^31)
+    if (psi_prec == MX_REAL64) MX_CPML_CASE(float, double, unsigned);
+    else MX_CPML_CASE(float, float, unsigned);
   }
 #undef MX_CPML_CASE
   return hipGetLastError();
@@ -860,8 +1007,8 @@ int mx_fdtd_cpml_e(const mx_fdtd_grid* g, int32_t prec, int32_t psi_prec, double
   if (psi_prec != MX_REAL32 && psi_prec != MX_REAL64) return mx::set_error("mx_fdtd_cpml_e: psi_prec must be MX_REAL32 or MX_REAL64");
   mx::CpmlTable tab;
   std::string why;
-  if (!mx::cpml_table(v, layers, nlayers, &tab, &why)) return mx::set_error("mx_fdtd_cpml_e: " + why);
-  const hipError_t err = mx::launch_cpml<true>(v, prec, psi_prec, dt, e, h, eps, eps_scalar, tab,
+  if (!mx::cpml_table(v, layers, nlayers, true, &tab, &why)) return mx::set_error("mx_fdtd_cpml_e: " + why);
+  const hipError_t err = mx::launch_cpml<true>(v, prec, psi_prec, dt, h, e, eps, eps_scalar, tab,
                                                reinterpret_cast<hipStream_t>(stream));
   return err == hipSuccess ? 0 : mx::set_error(std::string("mx_fdtd_cpml_e: ") + hipGetErrorString(err));
 }
@@ -873,7 +1020,7 @@ int mx_fdtd_cpml_h(const mx_fdtd_grid* g, int32_t prec, int32_t psi_prec, double
   if (psi_prec != MX_REAL32 && psi_prec != MX_REAL64) return mx::set_error("mx_fdtd_cpml_h: psi_prec must be MX_REAL32 or MX_REAL64");
   mx::CpmlTable tab;
   std::string why;
-  if (!mx::cpml_table(v, layers, nlayers, &tab, &why)) return mx::set_error("mx_fdtd_cpml_h: " + why);
+  if (!mx::cpml_table(v, layers, nlayers, false, &tab, &why)) return mx::set_error("mx_fdtd_cpml_h: " + why);
   const hipError_t err = mx::launch_cpml<false>(v, prec, psi_prec, dt, e, h, mu, mu_scalar, tab,
                                                 reinterpret_cast<hipStream_t>(stream));
   return err == hipSuccess ? 0 : mx::set_error(std::string("mx_fdtd_cpml_h: ") + hipGetErrorString(err));

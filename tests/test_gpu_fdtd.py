@@ -187,6 +187,50 @@ def test_cpml_updates_match_oracle(fdt, pdt, tol, shape, faces, thickness, with_
     numpy.testing.assert_allclose(ht.cpu().numpy(), h, rtol=tol, atol=tol * scale)
 
 
+@pytest.mark.parametrize('fdt,pdt,tol', [(numpy.float64, numpy.float64, 1e-11), (numpy.float32, numpy.float32, 1e-4)])
+@pytest.mark.parametrize('shape', [(4, 16, 16), (5, 16, 17), (67, 5, 51), (18, 3, 6)])
+def test_cpml_columns_and_slabs(fdt, pdt, tol, shape):
+    """(y, z) planes of exactly one 256-thread block, one cell more, and less than one; x
+    axes of one slab, of whole slabs and of a remainder; layers on every face that fits."""
+    from meanas_amd import fdtd
+    dt, thick = 0.2, 3
+    rng = numpy.random.default_rng(11)
+    e = rng.standard_normal((3, *shape)).astype(fdt)
+    h = rng.standard_normal((3, *shape)).astype(fdt)
+    eps = (1 + rng.random((3, *shape))).astype(fdt)
+    dxes = [[0.8 + 0.4 * rng.random(n) for n in shape] for _ in range(2)]
+    make = [[mod.cpml_params(a, p, dt, thickness=thick) if shape[a] > thick else None for p in (-1, 1)] for mod in (fdtd, ref)
+            for a in range(3)]
+    uE, uH = fdtd.updates_with_cpml(make[:3], dt, dxes, eps, dtype=pdt)
+    rE, rH = ref.updates_with_cpml(make[3:], dt, dxes, eps, dtype=pdt)
+    et, ht = torch.from_numpy(e.copy()).cuda(), torch.from_numpy(h.copy()).cuda()
+    for _ in range(4):
+        uE(et, ht, eps)
+        uH(et, ht)
+        rE(e, h, eps)
+        rH(e, h)
+    numpy.testing.assert_allclose(et.cpu().numpy(), e, rtol=tol, atol=tol)
+    numpy.testing.assert_allclose(ht.cpu().numpy(), h, rtol=tol, atol=tol)
+
+
+def test_cpml_plane_beyond_32_bit_offsets():
+    """A float64 (y, z) plane of more than 4 GiB (one x plane; about 30 GB in all): rows at
+    both ends and in the middle against the same differences in torch."""
+    from meanas_amd import fdtd
+    shape = (1, 23200, 23200)
+    e = torch.empty((3, *shape), dtype=torch.float64, device='cuda').uniform_(-1, 1)
+    h = torch.zeros_like(e)
+    n = shape[1]
+    dxes = [[numpy.ones(k) for k in shape] for _ in range(2)]
+    _, uH = fdtd.updates_with_cpml([[None, None]] * 3, 0.25, dxes, e)
+    uH(e, h)
+    for j in (0, n // 2, n - 1):
+        here, up = e[:, 0, j], e[:, 0, (j + 1) % n]
+        dz = [torch.roll(here[c], -1, 0) - here[c] for c in range(3)]
+        want = torch.stack([(up[2] - here[2]) - dz[1], dz[0], -(up[0] - here[0])]) * -0.25
+        torch.testing.assert_close(h[:, 0, j], want, rtol=1e-14, atol=1e-14)
+
+
 @pytest.mark.parametrize('axis,comp', [(0, 1), (1, 2), (2, 0)])
 def test_cpml_absorbs_a_pulse_on_gpu(axis, comp):
     from meanas_amd import fdtd
