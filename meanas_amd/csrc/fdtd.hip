@@ -6,10 +6,8 @@
 // differences (f[n+1] - f[n]) / dx_e[n] and backward differences (f[n] - f[n-1]) / dx_h[n],
 // unit widths when the grid gives none.  Materials divide, as the reference does.
 //
-// One thread per cell updates its three components; the neighbours one cell away are
-// re-read from the caches (k+-1 is the next lane; j+-1 and i+-1 rows and planes are in
-// L2 from the neighbouring threads).  HBM-bound: per step the H update reads e and h and
-// writes h, the E update reads h and e (and eps) and writes e.
+// The updates, the CPML and the energy kernels march along x, a thread per (y, z) column
+// (see Column); runs of several steps pipeline two steps per pass (k_fdtd_steps).
 #include <algorithm>
 #include <cstdlib>
 #include <string>
@@ -130,50 +128,63 @@ __device__ __forceinline__ double wave_value(double v) {
 template <typename T> __device__ __forceinline__ T lane_next(T v) { return lane_shift<0x130>(v); }
 template <typename T> __device__ __forceinline__ T lane_prev(T v) { return lane_shift<0x138>(v); }
 
-template <typename T>
-__global__ __launch_bounds__(kFB) void k_fdtd_h(RGrid g, T dt, const T* __restrict__ e, T* __restrict__ h,
-                                                const T* __restrict__ mu, T mu_s) {
-  const int nc = g.nx * g.ny * g.nz;
-  for (int cell = blockIdx.x * kFB + threadIdx.x; cell < nc; cell += gridDim.x * kFB) {
-    const int k = cell % g.nz, t = cell / g.nz, j = t % g.ny, i = t / g.ny;
-    const int sx = (i + 1 == g.nx ? -i : 1) * g.ny * g.nz;   // i+1 (periodic)
-    const int sy = (j + 1 == g.ny ? -j : 1) * g.nz;
-    const int sz = (k + 1 == g.nz ? -k : 1);
-    const T dx = (T)width(g.dxe[0], i), dy = (T)width(g.dxe[1], j), dz = (T)width(g.dxe[2], k);
-    const T rx = T(1) / dx, ry = T(1) / dy, rz = T(1) / dz;
-    const T ex = e[cell], ey = e[nc + cell], ez = e[2 * nc + cell];
-    const T cx = div_by(e[2 * nc + cell + sy] - ez, dy, ry) - div_by(e[nc + cell + sz] - ey, dz, rz);
-    const T cy = div_by(e[cell + sz] - ex, dz, rz) - div_by(e[2 * nc + cell + sx] - ez, dx, rx);
-    const T cz = div_by(e[nc + cell + sx] - ey, dx, rx) - div_by(e[cell + sy] - ex, dy, ry);
-    const T c[3] = {cx, cy, cz};
+// One leapfrog half step, HBM-bound: 36 (H) and 48 (E) bytes a cell in float32.  Marching
+// with the x neighbour in registers, no index division per cell and each XCD on its own
+// run of the grid reads each value about once (a thread per cell read 1.3 times as much).
+// E / H update: 256^3 float32 158 / 121 us (180 / 171 before), that is 5.1 / 5.0 TB/s, a
+// large copy's rate; float64 314 / 239 us (313 / 249); 150 x 141 x 130, in cache, float32
+// 21 / 17 us (28 / 24), float64 39 / 31 us (44 / 37).
+// H' = H - dt curl_f(E) / mu (EUPD false) or E' = E + dt curl_b(H) / eps (EUPD true), in
+// place: f is the field differenced, out the one updated.
+template <typename T, bool EUPD, typename OFF>
+__global__ __launch_bounds__(kFB) void k_fdtd_update(RGrid g, T dt, const T* __restrict__ f, T* __restrict__ out,
+                                                     const T* __restrict__ mat, T mat_s, int slab) {
+  const Column c = column(g, slab);
+  if (!c.ok) return;
+  const int nx = g.nx, ny = g.ny, nz = g.nz, plane = ny * nz;
+  const size_t nc = (size_t)nx * plane;
+  // neighbours of the difference: the cell before (E update) or after (H update)
+  const int jn = EUPD ? (c.j == 0 ? ny - 1 : c.j - 1) : (c.j + 1 == ny ? 0 : c.j + 1);
+  const int kn = EUPD ? (c.k == 0 ? nz - 1 : c.k - 1) : (c.k + 1 == nz ? 0 : c.k + 1);
+  const OFF own0 = (OFF)c.t * (OFF)sizeof(T);
+  const OFF oy0 = ((OFF)jn * (OFF)nz + (OFF)c.k) * (OFF)sizeof(T), oz0 = ((OFF)c.j * (OFF)nz + (OFF)kn) * (OFF)sizeof(T);
+  const double* const* wd = EUPD ? g.dxh : g.dxe;
+  const T dy = (T)width(wd[1], c.j), dz = (T)width(wd[2], c.k);
+  const T ry = T(1) / dy, rz = T(1) / dz;
+  const T rs = recip(mat_s);
+  // x: the plane carried along is i - 1 (E update) or i (H update)
+  T car[3];
+  {
+    const int ip = EUPD ? (c.ib == 0 ? nx - 1 : c.ib - 1) : c.ib;
 #pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      const T m = mu ? mu[q * nc + cell] : mu_s;
-      h[q * nc + cell] -= div_by(dt * c[q], m, recip(m));
-    }
+    for (int q = 0; q < 3; ++q) car[q] = at(f, q * nc + (size_t)ip * plane, own0);
   }
-}
-
-template <typename T>
-__global__ __launch_bounds__(kFB) void k_fdtd_e(RGrid g, T dt, T* __restrict__ e, const T* __restrict__ h,
-                                                const T* __restrict__ eps, T eps_s) {
-  const int nc = g.nx * g.ny * g.nz;
-  for (int cell = blockIdx.x * kFB + threadIdx.x; cell < nc; cell += gridDim.x * kFB) {
-    const int k = cell % g.nz, t = cell / g.nz, j = t % g.ny, i = t / g.ny;
-    const int sx = (i == 0 ? g.nx - 1 : -1) * g.ny * g.nz;   // i-1 (periodic)
-    const int sy = (j == 0 ? g.ny - 1 : -1) * g.nz;
-    const int sz = (k == 0 ? g.nz - 1 : -1);
-    const T dx = (T)width(g.dxh[0], i), dy = (T)width(g.dxh[1], j), dz = (T)width(g.dxh[2], k);
-    const T rx = T(1) / dx, ry = T(1) / dy, rz = T(1) / dz;
-    const T hx = h[cell], hy = h[nc + cell], hz = h[2 * nc + cell];
-    const T cx = div_by(hz - h[2 * nc + cell + sy], dy, ry) - div_by(hy - h[nc + cell + sz], dz, rz);
-    const T cy = div_by(hx - h[cell + sz], dz, rz) - div_by(hz - h[2 * nc + cell + sx], dx, rx);
-    const T cz = div_by(hy - h[nc + cell + sx], dx, rx) - div_by(hx - h[cell + sy], dy, ry);
-    const T c[3] = {cx, cy, cz};
+#pragma unroll 1
+  for (int i = c.ib; i < c.ie; ++i) {
+    const OFF own = in_loop(own0), oy = in_loop(oy0), oz = in_loop(oz0);
+    const size_t pi = (size_t)i * plane;
+    const size_t pl = EUPD ? pi : (size_t)(i + 1 == nx ? 0 : i + 1) * plane;
+    T ld[3], o[3], m[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) ld[q] = at(f, q * nc + pl, own);
+    const T y0 = at(f, pi, oy), y2 = at(f, 2 * nc + pi, oy), z0 = at(f, pi, oz), z1 = at(f, nc + pi, oz);
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
-      const T m = eps ? eps[q * nc + cell] : eps_s;
-      e[q * nc + cell] += div_by(dt * c[q], m, recip(m));
+      o[q] = at((const T*)out, q * nc + pi, own);
+      m[q] = mat ? at(mat, q * nc + pi, own) : mat_s;
+    }
+    const T dx = (T)width_u(wd[0], i), rx = recip(dx);
+    const T (&here)[3] = EUPD ? ld : car;
+    const T (&xn)[3] = EUPD ? car : ld;
+    auto dif = [](T a, T b, T w, T r) { return div_by(EUPD ? a - b : b - a, w, r); };
+    const T cc[3] = {dif(here[2], y2, dy, ry) - dif(here[1], z1, dz, rz),
+                     dif(here[0], z0, dz, rz) - dif(here[2], xn[2], dx, rx),
+                     dif(here[1], xn[1], dx, rx) - dif(here[0], y0, dy, ry)};
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const T up = div_by(dt * cc[q], m[q], mat ? recip(m[q]) : rs);
+      put(out, q * nc + pi, own, EUPD ? o[q] + up : o[q] - up);
+      car[q] = ld[q];
     }
   }
 }
@@ -649,80 +660,118 @@ __global__ __launch_bounds__(kFB) void k_conducting(int nx, int ny, int nz, int 
 // component sum in the field precision (in component order, starting from the x term),
 // the widths in double (the float64 width arrays promote) multiplied one axis at a time,
 // and nothing contracted into fused multiply-adds.  `form` is one of MX_ENERGY_*.
+// Column kernels, HBM-bound.  256^3: energy_hstep float64 270 us (307 with a thread per cell
+// and each component's loads behind the one before), 6.5 TB/s with part of it in cache,
+// float32 146 us (189); poynting 231 / 120 us (246 / 136), divergence 102 / 38 us (107 / 45).
 
-template <typename T>
+template <typename T, typename OFF>
 __global__ __launch_bounds__(kFB) void k_energy(RGrid g, int form, T dt, const T* __restrict__ f0,
                                                 const T* __restrict__ f1, const T* __restrict__ f2,
                                                 const T* __restrict__ f3, const T* __restrict__ eps, T eps_s,
-                                                const T* __restrict__ mu, T mu_s, double* __restrict__ out) {
+                                                const T* __restrict__ mu, T mu_s, double* __restrict__ out, int slab) {
 #pragma clang fp contract(off)
-  const int nc = g.nx * g.ny * g.nz;
-  for (int cell = blockIdx.x * kFB + threadIdx.x; cell < nc; cell += gridDim.x * kFB) {
-    const int k = cell % g.nz, t = cell / g.nz, j = t % g.ny, i = t / g.ny;
+  const Column col = column(g, slab);
+  if (!col.ok) return;
+  const size_t plane = (size_t)g.ny * g.nz, nc = g.nx * plane;
+  const OFF own0 = (OFF)col.t * (OFF)sizeof(T), oout0 = (OFF)col.t * (OFF)sizeof(double);
+  const double wey = width(g.dxe[1], col.j), wez = width(g.dxe[2], col.k);
+  const double why = width(g.dxh[1], col.j), whz = width(g.dxh[2], col.k);
+#pragma unroll 1
+  for (int i = col.ib; i < col.ie; ++i) {
+    const OFF own = in_loop(own0), oout = in_loop(oout0);
+    // every load of the cell before any is used (f2, f3 and the materials only if given)
+    T a0[3], a1[3], a2[3], a3[3], me[3], mh[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const size_t q = c * nc + i * plane;
+      a0[c] = at(f0, q, own);
+      a1[c] = at(f1, q, own);
+      a2[c] = f2 ? at(f2, q, own) : T(0);
+      a3[c] = f3 ? at(f3, q, own) : T(0);
+      me[c] = eps ? at(eps, q, own) : eps_s;
+      mh[c] = mu ? at(mu, q, own) : mu_s;
+    }
     T se = T(0), sh = T(0);
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      const int q = c * nc + cell;
       T ee, hh = T(0);
       switch (form) {
-        case MX_ENERGY_DXMUL: ee = f0[q]; hh = f1[q]; break;
-        case MX_ENERGY_HSTEP: ee = f0[q] * f2[q]; hh = f1[q] * f1[q]; break;
-        case MX_ENERGY_ESTEP: ee = f1[q] * f1[q]; hh = f0[q] * f2[q]; break;
-        case MX_ENERGY_H2E: ee = f2[q] * (f2[q] - f0[q]) / dt; hh = f1[q] * (f3[q] - f1[q]) / dt; break;
-        case MX_ENERGY_E2H: ee = f1[q] * (f3[q] - f1[q]) / dt; hh = f2[q] * (f2[q] - f0[q]) / dt; break;
-        default: ee = f0[q] * f1[q]; break;   // j0 . e1, no material
+        case MX_ENERGY_DXMUL: ee = a0[c]; hh = a1[c]; break;
+        case MX_ENERGY_HSTEP: ee = a0[c] * a2[c]; hh = a1[c] * a1[c]; break;
+        case MX_ENERGY_ESTEP: ee = a1[c] * a1[c]; hh = a0[c] * a2[c]; break;
+        case MX_ENERGY_H2E: ee = a2[c] * (a2[c] - a0[c]) / dt; hh = a1[c] * (a3[c] - a1[c]) / dt; break;
+        case MX_ENERGY_E2H: ee = a1[c] * (a3[c] - a1[c]) / dt; hh = a2[c] * (a2[c] - a0[c]) / dt; break;
+        default: ee = a0[c] * a1[c]; break;   // j0 . e1, no material
       }
-      const T we = form == MX_ENERGY_J ? ee : ee * (eps ? eps[q] : eps_s);
-      const T wh = hh * (mu ? mu[q] : mu_s);
+      const T we = form == MX_ENERGY_J ? ee : ee * me[c];
+      const T wh = hh * mh[c];
       se = c == 0 ? we : se + we;
       sh = c == 0 ? wh : sh + wh;
     }
-    const double ue = (double)se * width(g.dxe[0], i) * width(g.dxe[1], j) * width(g.dxe[2], k);
-    out[cell] = form == MX_ENERGY_J ? ue : ue + (double)sh * width(g.dxh[0], i) * width(g.dxh[1], j) * width(g.dxh[2], k);
+    const double ue = (double)se * width_u(g.dxe[0], i) * wey * wez;
+    put(out, i * plane, oout, form == MX_ENERGY_J ? ue : ue + (double)sh * width_u(g.dxh[0], i) * why * whz);
   }
 }
 
 // s = E(+1) x H with both width-weighted (fdtd/energy.py:10-87): s_x = ey(i+1) hz - ez(i+1) hy
 // and cyclically, E taken at the next cell along the component's axis (periodic), in
 // double, stored in the field precision.
-template <typename T>
+template <typename T, typename OFF>
 __global__ __launch_bounds__(kFB) void k_poynting(RGrid g, const T* __restrict__ e, const T* __restrict__ h,
-                                                  T* __restrict__ s) {
+                                                  T* __restrict__ s, int slab) {
 #pragma clang fp contract(off)
-  const int nc = g.nx * g.ny * g.nz;
-  for (int cell = blockIdx.x * kFB + threadIdx.x; cell < nc; cell += gridDim.x * kFB) {
-    const int k = cell % g.nz, t = cell / g.nz, j = t % g.ny, i = t / g.ny;
-    const int sx = (i + 1 == g.nx ? -i : 1) * g.ny * g.nz;
-    const int sy = (j + 1 == g.ny ? -j : 1) * g.nz;
-    const int sz = (k + 1 == g.nz ? -k : 1);
-    const double wex = width(g.dxe[0], i), wey = width(g.dxe[1], j), wez = width(g.dxe[2], k);
-    const double hx = (double)h[cell] * width(g.dxh[0], i);
-    const double hy = (double)h[nc + cell] * width(g.dxh[1], j);
-    const double hz = (double)h[2 * nc + cell] * width(g.dxh[2], k);
-    const double s0 = ((double)e[nc + cell + sx] * wey) * hz - ((double)e[2 * nc + cell + sx] * wez) * hy;
-    const double s1 = ((double)e[2 * nc + cell + sy] * wez) * hx - ((double)e[cell + sy] * wex) * hz;
-    const double s2 = ((double)e[cell + sz] * wex) * hy - ((double)e[nc + cell + sz] * wey) * hx;
-    s[cell] = (T)s0;
-    s[nc + cell] = (T)s1;
-    s[2 * nc + cell] = (T)s2;
+  const Column col = column(g, slab);
+  if (!col.ok) return;
+  const int nx = g.nx, ny = g.ny, nz = g.nz;
+  const size_t plane = (size_t)ny * nz, nc = nx * plane;
+  const int jn = col.j + 1 == ny ? 0 : col.j + 1, kn = col.k + 1 == nz ? 0 : col.k + 1;
+  const OFF own0 = (OFF)col.t * (OFF)sizeof(T);
+  const OFF oy0 = ((OFF)jn * (OFF)nz + (OFF)col.k) * (OFF)sizeof(T);
+  const OFF oz0 = ((OFF)col.j * (OFF)nz + (OFF)kn) * (OFF)sizeof(T);
+  const double wey = width(g.dxe[1], col.j), wez = width(g.dxe[2], col.k);
+  const double why = width(g.dxh[1], col.j), whz = width(g.dxh[2], col.k);
+#pragma unroll 1
+  for (int i = col.ib; i < col.ie; ++i) {
+    const OFF own = in_loop(own0), oy = in_loop(oy0), oz = in_loop(oz0);
+    const size_t pi = i * plane, pn = (size_t)(i + 1 == nx ? 0 : i + 1) * plane;
+    const T h0 = at(h, pi, own), h1 = at(h, nc + pi, own), h2 = at(h, 2 * nc + pi, own);
+    const T eyx = at(e, nc + pn, own), ezx = at(e, 2 * nc + pn, own), ezy = at(e, 2 * nc + pi, oy), exy = at(e, pi, oy);
+    const T exz = at(e, pi, oz), eyz = at(e, nc + pi, oz);
+    const double wex = width_u(g.dxe[0], i);
+    const double hx = (double)h0 * width_u(g.dxh[0], i), hy = (double)h1 * why, hz = (double)h2 * whz;
+    const double s0 = ((double)eyx * wey) * hz - ((double)ezx * wez) * hy;
+    const double s1 = ((double)ezy * wez) * hx - ((double)exy * wex) * hz;
+    const double s2 = ((double)exz * wex) * hy - ((double)eyz * wey) * hx;
+    put(s, pi, own, (T)s0);
+    put(s, nc + pi, own, (T)s1);
+    put(s, 2 * nc + pi, own, (T)s2);
   }
 }
 
 // ds = sum_a (s_a - s_a(previous cell along a)), unit spacing (deriv_back() without
 // widths, fdtd/energy.py:90-125), in the field precision.
-template <typename T>
-__global__ __launch_bounds__(kFB) void k_poynting_div(RGrid g, const T* __restrict__ s, T* __restrict__ ds) {
+template <typename T, typename OFF>
+__global__ __launch_bounds__(kFB) void k_poynting_div(RGrid g, const T* __restrict__ s, T* __restrict__ ds, int slab) {
 #pragma clang fp contract(off)
-  const int nc = g.nx * g.ny * g.nz;
-  for (int cell = blockIdx.x * kFB + threadIdx.x; cell < nc; cell += gridDim.x * kFB) {
-    const int k = cell % g.nz, t = cell / g.nz, j = t % g.ny, i = t / g.ny;
-    const int sx = (i == 0 ? g.nx - 1 : -1) * g.ny * g.nz;   // i-1 (periodic)
-    const int sy = (j == 0 ? g.ny - 1 : -1) * g.nz;
-    const int sz = (k == 0 ? g.nz - 1 : -1);
-    const T dx = s[cell] - s[cell + sx];
-    const T dy = s[nc + cell] - s[nc + cell + sy];
-    const T dz = s[2 * nc + cell] - s[2 * nc + cell + sz];
-    ds[cell] = dx + dy + dz;
+  const Column col = column(g, slab);
+  if (!col.ok) return;
+  const int nx = g.nx, ny = g.ny, nz = g.nz;
+  const size_t plane = (size_t)ny * nz, nc = nx * plane;
+  const int jp = col.j == 0 ? ny - 1 : col.j - 1, kp = col.k == 0 ? nz - 1 : col.k - 1;
+  const OFF own0 = (OFF)col.t * (OFF)sizeof(T);
+  const OFF oy0 = ((OFF)jp * (OFF)nz + (OFF)col.k) * (OFF)sizeof(T);
+  const OFF oz0 = ((OFF)col.j * (OFF)nz + (OFF)kp) * (OFF)sizeof(T);
+  T sx = at(s, (size_t)(col.ib == 0 ? nx - 1 : col.ib - 1) * plane, own0);
+#pragma unroll 1
+  for (int i = col.ib; i < col.ie; ++i) {
+    const OFF own = in_loop(own0), oy = in_loop(oy0), oz = in_loop(oz0);
+    const size_t pi = i * plane;
+    const T s0 = at(s, pi, own);
+    const T dx = s0 - sx;
+    const T dy = at(s, nc + pi, own) - at(s, nc + pi, oy);
+    const T dz = at(s, 2 * nc + pi, own) - at(s, 2 * nc + pi, oz);
+    put(ds, pi, own, dx + dy + dz);
+    sx = s0;
   }
 }
 
@@ -737,32 +786,45 @@ bool rgrid(const mx_fdtd_grid* g, RGrid* v, std::string* why) {
   return true;
 }
 
-unsigned blocks(const RGrid& v) {
-  const long long nc = (long long)v.nx * v.ny * v.nz;
-  const long long nb = (nc + kFB - 1) / kFB;
-  return (unsigned)(nb > 16384 ? 16384 : nb);
+// Launch of a column kernel: slabs of 6 planes, of 4 and then 2 while the chip has fewer
+// than 8 blocks per CU.  Slabs of 2/4/6/8/16/64 planes, E update of float64 at 256^3: 327,
+// 320, 314, 317, 323, 326 us; of float32 at 228 x 100 x 180: 28.7, 29.1, 30.0, 31.3, 34.0,
+// 42.1 us, with CPML 50.2, 43.2, 42.8, 43.5, 52.8, 107.7 us.
+struct ColumnGrid { int slab; unsigned blocks; };
+ColumnGrid column_grid(const RGrid& v) {
+  const long long pieces = ((long long)v.ny * v.nz + kFB - 1) / kFB;
+  int slab = 0;
+  for (int want : {6, 4, 2}) {
+    slab = std::min(want, v.nx);
+    if (pieces * ((v.nx + slab - 1) / slab) >= 2048) break;
+  }
+  const long long nwork = pieces * ((v.nx + slab - 1) / slab);
+  return {slab, (unsigned)((nwork + 7) / 8 * 8)};
+}
+// whether the byte offsets of a plane fit 32 bits (beyond: kernels with 64-bit offsets)
+bool small_plane(const RGrid& v, int prec) {
+  return (unsigned long long)v.ny * v.nz * (prec == MX_REAL64 ? 8 : 4) < (1ull << 32);
 }
 
+template <bool EUPD>
+hipError_t launch_update(const RGrid& v, int prec, double dt, const void* f, void* out, const void* mat, double mat_s,
+                         hipStream_t s) {
+  const ColumnGrid cg = column_grid(v);
+#define MX_UPDATE_CASE(T, OFF)                                                                                      \
+  hipLaunchKernelGGL((k_fdtd_update<T, EUPD, OFF>), dim3(cg.blocks), dim3(kFB), 0, s, v, (T)dt, (const T*)f, (T*)out, \
+                     (const T*)mat, (T)mat_s, cg.slab)
+  if (prec == MX_REAL64) { if (small_plane(v, prec)) MX_UPDATE_CASE(double, unsigned); else MX_UPDATE_CASE(double, size_t); }
+  else MX_UPDATE_CASE(float, unsigned);   // a float32 plane is always below 4 GiB (3 N < 2^31)
+#undef MX_UPDATE_CASE
+  return hipGetLastError();
+}
 hipError_t launch_h(const RGrid& v, int prec, double dt, const void* e, void* h, const void* mu, double mu_s,
                     hipStream_t s) {
-  if (prec == MX_REAL64)
-    hipLaunchKernelGGL(k_fdtd_h<double>, dim3(blocks(v)), dim3(kFB), 0, s, v, dt, (const double*)e, (double*)h,
-                       (const double*)mu, mu_s);
-  else
-    hipLaunchKernelGGL(k_fdtd_h<float>, dim3(blocks(v)), dim3(kFB), 0, s, v, (float)dt, (const float*)e, (float*)h,
-                       (const float*)mu, (float)mu_s);
-  return hipGetLastError();
+  return launch_update<false>(v, prec, dt, e, h, mu, mu_s, s);
 }
-
 hipError_t launch_e(const RGrid& v, int prec, double dt, void* e, const void* h, const void* eps, double eps_s,
                     hipStream_t s) {
-  if (prec == MX_REAL64)
-    hipLaunchKernelGGL(k_fdtd_e<double>, dim3(blocks(v)), dim3(kFB), 0, s, v, dt, (double*)e, (const double*)h,
-                       (const double*)eps, eps_s);
-  else
-    hipLaunchKernelGGL(k_fdtd_e<float>, dim3(blocks(v)), dim3(kFB), 0, s, v, (float)dt, (float*)e, (const float*)h,
-                       (const float*)eps, (float)eps_s);
-  return hipGetLastError();
+  return launch_update<true>(v, prec, dt, h, e, eps, eps_s, s);
 }
 
 hipError_t launch_conducting(const RGrid& v, int prec, int dir, int pol, int is_h, void* f, hipStream_t s) {
@@ -779,36 +841,39 @@ hipError_t launch_conducting(const RGrid& v, int prec, int dir, int pol, int is_
   return hipGetLastError();
 }
 
+// a column kernel in the field precision, with 32-bit byte offsets where the widest plane it
+// addresses allows (a float32 plane always does: 3 N < 2^31)
+#define MX_COLUMN_LAUNCH(kern, small, ...)                                                             \
+  do {                                                                                                 \
+    const ColumnGrid cg = column_grid(v);                                                              \
+    if (prec == MX_REAL64) {                                                                           \
+      typedef double T;                                                                                \
+      if (small) hipLaunchKernelGGL((kern<T, unsigned>), dim3(cg.blocks), dim3(kFB), 0, s, v, __VA_ARGS__, cg.slab); \
+      else hipLaunchKernelGGL((kern<T, size_t>), dim3(cg.blocks), dim3(kFB), 0, s, v, __VA_ARGS__, cg.slab);         \
+    } else {                                                                                           \
+      typedef float T;                                                                                 \
+      if (small) hipLaunchKernelGGL((kern<T, unsigned>), dim3(cg.blocks), dim3(kFB), 0, s, v, __VA_ARGS__, cg.slab); \
+      else hipLaunchKernelGGL((kern<T, size_t>), dim3(cg.blocks), dim3(kFB), 0, s, v, __VA_ARGS__, cg.slab);         \
+    }                                                                                                  \
+  } while (0)
+
 hipError_t launch_energy(const RGrid& v, int prec, int form, double dt, const void* const* f, const void* eps,
                          double eps_s, const void* mu, double mu_s, double* out, hipStream_t s) {
-  if (prec == MX_REAL64)
-    hipLaunchKernelGGL(k_energy<double>, dim3(blocks(v)), dim3(kFB), 0, s, v, form, dt, (const double*)f[0],
-                       (const double*)f[1], (const double*)f[2], (const double*)f[3], (const double*)eps, eps_s,
-                       (const double*)mu, mu_s, out);
-  else
-    hipLaunchKernelGGL(k_energy<float>, dim3(blocks(v)), dim3(kFB), 0, s, v, form, (float)dt, (const float*)f[0],
-                       (const float*)f[1], (const float*)f[2], (const float*)f[3], (const float*)eps, (float)eps_s,
-                       (const float*)mu, (float)mu_s, out);
+  MX_COLUMN_LAUNCH(k_energy, small_plane(v, MX_REAL64), form, (T)dt, (const T*)f[0], (const T*)f[1], (const T*)f[2],
+                   (const T*)f[3], (const T*)eps, (T)eps_s, (const T*)mu, (T)mu_s, out);
   return hipGetLastError();
 }
 
 hipError_t launch_poynting(const RGrid& v, int prec, const void* e, const void* h, void* out, hipStream_t s) {
-  if (prec == MX_REAL64)
-    hipLaunchKernelGGL(k_poynting<double>, dim3(blocks(v)), dim3(kFB), 0, s, v, (const double*)e, (const double*)h,
-                       (double*)out);
-  else
-    hipLaunchKernelGGL(k_poynting<float>, dim3(blocks(v)), dim3(kFB), 0, s, v, (const float*)e, (const float*)h,
-                       (float*)out);
+  MX_COLUMN_LAUNCH(k_poynting, small_plane(v, prec), (const T*)e, (const T*)h, (T*)out);
   return hipGetLastError();
 }
 
 hipError_t launch_poynting_div(const RGrid& v, int prec, const void* sv, void* ds, hipStream_t s) {
-  if (prec == MX_REAL64)
-    hipLaunchKernelGGL(k_poynting_div<double>, dim3(blocks(v)), dim3(kFB), 0, s, v, (const double*)sv, (double*)ds);
-  else
-    hipLaunchKernelGGL(k_poynting_div<float>, dim3(blocks(v)), dim3(kFB), 0, s, v, (const float*)sv, (float*)ds);
+  MX_COLUMN_LAUNCH(k_poynting_div, small_plane(v, prec), (const T*)sv, (T*)ds);
   return hipGetLastError();
 }
+#undef MX_COLUMN_LAUNCH
 
 // Layer table of a CPML update: faces in increasing (axis, polarity) order (the order
 // the reference accumulates in), each inside the grid, with its arrays.
@@ -831,22 +896,6 @@ bool cpml_table(const RGrid& v, const mx_cpml_layer* layers, int n, bool eupd, C
                            eupd ? L.psi_e : L.psi_h};
   }
   return true;
-}
-
-// Launch of a column kernel: slabs of 16 planes, shallower (down to 4) while the chip has
-// fewer than 8 blocks per CU.
-struct ColumnGrid { int slab; unsigned blocks; };
-ColumnGrid column_grid(const RGrid& v) {
-  const long long pieces = ((long long)v.ny * v.nz + kFB - 1) / kFB;
-  int slab = 16;
-  while (slab > 4 && pieces * ((v.nx + slab - 1) / slab) < 2048) slab /= 2;
-  slab = std::min(slab, v.nx);
-  const long long nwork = pieces * ((v.nx + slab - 1) / slab);
-  return {slab, (unsigned)((nwork + 7) / 8 * 8)};
-}
-// whether the byte offsets of a plane fit 32 bits (beyond: kernels with 64-bit offsets)
-bool small_plane(const RGrid& v, int prec) {
-  return (unsigned long long)v.ny * v.nz * (prec == MX_REAL64 ? 8 : 4) < (1ull << 32);
 }
 
 template <bool EUPD>

@@ -416,3 +416,57 @@ def test_energy_functions_on_device_tensors():
         fdtd.energy_estep(e, h.astype(numpy.float32), e2)
     with pytest.raises(AssertionError):     # as the reference: e, h and dxes, or s
         fdtd.poynting_divergence(e=e, h=h)
+
+
+@pytest.mark.parametrize('dtype', [numpy.float64, numpy.float32])
+@pytest.mark.parametrize('shape', [(4, 16, 16), (5, 16, 17), (13, 5, 60), (1, 1, 300)])
+def test_column_kernels_at_block_and_slab_edges(dtype, shape):
+    """Updates, energy, Poynting vector and divergence on (y, z) planes of one 256-thread
+    block, one cell more, less, and several, with whole and partial slabs."""
+    from meanas_amd import fdtd
+    e, h, eps, mu, dxes = _fields(shape, 17, dtype)
+    tol = 1e-13 if dtype == numpy.float64 else 2e-5
+    kw = dict(rtol=tol, atol=tol)
+    e2, h2 = numpy.roll(e, 1, axis=2), numpy.roll(h, 1, axis=3)
+    numpy.testing.assert_allclose(fdtd.energy_hstep(e, h, e2, eps, mu, dxes), ref.energy_hstep(e, h, e2, eps, mu, dxes), **kw)
+    numpy.testing.assert_allclose(fdtd.delta_energy_e2h(0.2, h, e, h2, e2, eps, mu, dxes),
+                                  ref.delta_energy_e2h(0.2, h, e, h2, e2, eps, mu, dxes), rtol=tol, atol=20 * tol)
+    s = ref.fdtd_poynting(e, h, dxes)
+    numpy.testing.assert_allclose(fdtd.poynting(e, h, dxes), s, **kw)
+    numpy.testing.assert_allclose(fdtd.poynting_divergence(s.astype(dtype)), ref.poynting_divergence(s.astype(dtype)), **kw)
+    e1, h1 = e.copy(), h.copy()
+    ref.maxwell_h(0.2, dxes)(h=h1, e=e1, mu=mu)
+    ref.maxwell_e(0.2, dxes)(e1, h1, eps)
+    fdtd.maxwell_h(0.2, dxes)(e, h, mu)
+    fdtd.maxwell_e(0.2, dxes)(e, h, eps)
+    numpy.testing.assert_allclose(h, h1, **kw)
+    numpy.testing.assert_allclose(e, e1, **kw)
+
+
+@pytest.mark.parametrize('name', ['update', 'energy', 'poynting'])
+def test_planes_beyond_32_bit_offsets(name):
+    """One float64 x plane of more than 4 GiB: rows at both ends and in the middle."""
+    from meanas_amd import fdtd
+    n = 23200
+    e = torch.empty((3, 1, n, n), dtype=torch.float64, device='cuda').uniform_(-1, 1)
+    rows = (0, n // 2, n - 1)
+    if name == 'energy':
+        got = fdtd.dxmul(e, e)
+        for j in rows:
+            torch.testing.assert_close(got[0, j], 2 * (e[:, 0, j] ** 2).sum(0), rtol=1e-13, atol=1e-13)
+        return
+    if name == 'poynting':
+        got = fdtd.poynting(e, e)
+        for j in rows:
+            x, y = e[:, 0, j], e[:, 0, (j + 1) % n]
+            z = torch.roll(x, -1, 1)
+            want = torch.stack([x[1] * x[2] - x[2] * x[1], y[2] * x[0] - y[0] * x[2], z[0] * x[1] - z[1] * x[0]])
+            torch.testing.assert_close(got[:, 0, j], want, rtol=1e-13, atol=1e-13)
+        return
+    out = torch.zeros_like(e)
+    fdtd.maxwell_e(0.25)(out, e, 2.0)
+    for j in rows:
+        x, y = e[:, 0, j], e[:, 0, j - 1]
+        z = torch.roll(x, 1, 1)
+        want = torch.stack([(x[2] - y[2]) - (x[1] - z[1]), x[0] - z[0], -(x[0] - y[0])]) * 0.125
+        torch.testing.assert_close(out[:, 0, j], want, rtol=1e-13, atol=1e-13)
