@@ -232,6 +232,20 @@ int mx_poynting_e_cross_h(const mx_grid* g, const void* e, const void* h, int32_
  * conjugated first when conj_e is nonzero.  h, e, s: 3N complex128 in vec() order. */
 int mx_poynting_h_cross_e(const mx_grid* g, const void* h, const void* e, int32_t conj_e, void* s, void* stream);
 
+/* y = A0 x, A0 = e_full with the operator's materials and masks (fdfd/operators.py:40-96;
+ * the unscaled operator: A = P A0 P^-1 is what mx_apply applies).  g holds the operator's
+ * cell widths.  With `reversed` nonzero every cell index of x and y is reversed, which
+ * makes the e_full of a reversed dual operator h_full (fdfd/operators.py:126-180).  x, y:
+ * 3N complex128 in vec() order, not overlapping. */
+int mx_wave(const mx_operator* op, const mx_grid* g, int32_t reversed, const void* x, void* y, void* stream);
+
+/* y = c k (A0 (q x) - q (A0 x)): the total-field / scattered-field source of region q
+ * (fdfd/operators.py:366-394) with c = 1 / (-i omega), kept only where k says (the boundary
+ * source, fdfd/operators.py:397-450).  region, keep: 3N float64; keep may be NULL.  x, y:
+ * 3N complex128, not overlapping. */
+int mx_wave_source(const mx_operator* op, const mx_grid* g, const double* region, const double* keep, double c_re,
+                   double c_im, const void* x, void* y, void* stream);
+
 /* ---- time domain (FDTD) ------------------------------------------------------------
  * Real fields (3, nx, ny, nz) in vec() order, float32 (MX_REAL32) or float64 (MX_REAL64).
  * Grid: real cell widths dxes[0] (E grid) and dxes[1] (H grid), float64 device arrays of

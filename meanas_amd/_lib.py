@@ -136,6 +136,10 @@ PROTOTYPES = {
                                              c_void_p]),
     'mx_poynting_e_cross_h': (ctypes.c_int, [ctypes.POINTER(MxGrid), c_void_p, c_void_p, ctypes.c_int32, c_void_p,
                                              c_void_p]),
+    'mx_wave': (ctypes.c_int, [ctypes.POINTER(MxOperator), ctypes.POINTER(MxGrid), ctypes.c_int32, c_void_p, c_void_p,
+                               c_void_p]),
+    'mx_wave_source': (ctypes.c_int, [ctypes.POINTER(MxOperator), ctypes.POINTER(MxGrid), c_void_p, c_void_p,
+                                      ctypes.c_double, ctypes.c_double, c_void_p, c_void_p, c_void_p]),
     'mx_fdtd_h': (ctypes.c_int, [ctypes.POINTER(MxFdtdGrid), ctypes.c_int32, ctypes.c_double, c_void_p, c_void_p,
                                  c_void_p, ctypes.c_double, c_void_p]),
     'mx_fdtd_e': (ctypes.c_int, [ctypes.POINTER(MxFdtdGrid), ctypes.c_int32, ctypes.c_double, c_void_p, c_void_p,

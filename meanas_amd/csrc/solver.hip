@@ -722,6 +722,13 @@ mx_options defaults(const mx_options* opt) {
 namespace mx {
 // error reporting for the other translation units of the library (mx_last_error)
 int set_error(const std::string& msg) { return fail(msg); }
+
+// the checked complex128 view of an operator, for the other translation units
+bool wave_op(const mx_operator& op, OpView<double>* v, std::string* why) {
+  if (!valid_op(op, MX_FP64, why)) return false;
+  *v = view_of<double>(op);
+  return true;
+}
 }  // namespace mx
 
 extern "C" {

@@ -30,7 +30,7 @@ It also gives the wave operators as callables:
   shift turns backward differences into negated forward ones);
 - `e_full(omega, dxes, epsilon, mu, pec, pmc)`: the sparse `meanas/fdfd/operators.py:40-96`
   operator (1/mu divides, as on the solve path; the reference's functional form multiplies
-  by mu instead), applied as (1/p) A (p E) with the solver's symmetrised FP64 apply;
+  by mu instead), one pass over the field (`mx_wave`);
 - `h_full(...)` (`meanas/fdfd/operators.py:126-180`) through the exact duality
   h_full(omega, dxes, eps, mu, pec, pmc) = R e_full(omega, [rev dxh, rev dxe], rev mu,
   rev eps, pec = rev pmc, pmc = rev pec) R;
@@ -40,7 +40,7 @@ It also gives the wave operators as callables:
 Fields may be given as `(3, nx, ny, nz)` arrays (the functional layout) or as `vec()`
 vectors of length 3N.  numpy inputs give numpy outputs of the same shape; torch tensors
 stay on the device.  The kernels run through the C ABI (`mx_e2h`, `mx_m2j`,
-`mx_poynting_e_cross_h`, `mx_poynting_h_cross_e`, `mx_map`, `mx_apply`).
+`mx_poynting_e_cross_h`, `mx_poynting_h_cross_e`, `mx_wave`).
 """
 from __future__ import annotations
 
@@ -62,7 +62,7 @@ class _Grid:
         if tuple(len(d) for d in dxes[1]) != self.shape:
             raise ValueError('dxes[0] and dxes[1] describe different grids')
         self.device = torch.device(device)
-        self.arrays = [torch.from_numpy(numpy.ascontiguousarray(d, dtype=numpy.complex128)).to(self.device)
+        self.arrays = [torch.from_numpy(numpy.array(d, dtype=numpy.complex128, order='C')).to(self.device)
                        for d in (*dxes[0], *dxes[1])]
         nx, ny, nz = self.shape
         self.desc = _lib.MxGrid(nx, ny, nz, 0,
@@ -241,15 +241,20 @@ def _rev_vec(v, shape):
 
 
 class _A0:
-    """E -> e_full(omega, dxes, epsilon, mu, pec, pmc) @ E on the GPU: (1/p) A (p E)."""
+    """E -> e_full(omega, dxes, epsilon, mu, pec, pmc) @ E on the GPU; with `reversed` the
+    cells of E and of the result are taken in reversed order (R e_full R)."""
 
-    def __init__(self, omega, dxes, epsilon, mu, pec, pmc, device):
+    def __init__(self, omega, dxes, epsilon, mu, pec, pmc, device, reversed: bool = False):
         self.op = DeviceOperator(omega, dxes, numpy.asarray(epsilon).reshape(-1), mu=_vec_or_none(mu),
                                  pec=_vec_or_none(pec), pmc=_vec_or_none(pmc), device=device)
+        self.grid = _Grid(dxes, device)
+        self.reversed = 1 if reversed else 0
 
     def __call__(self, x: torch.Tensor) -> torch.Tensor:
-        px = self.op.map(_lib.MX_MAP_RHS, x, coef=1.0)
-        return self.op.map(_lib.MX_MAP_E, self.op.apply(px))
+        y = torch.empty_like(x)
+        _lib.check(_lib.lib().mx_wave(ctypes.byref(self.op.desc), ctypes.byref(self.grid.desc), self.reversed,
+                                      x.data_ptr(), y.data_ptr(), torch_stream_handle()), 'mx_wave')
+        return y
 
 
 def _dev_field(f, op: DeviceOperator):
@@ -283,11 +288,12 @@ def h_full(omega: complex, dxes, epsilon, mu=None, pec=None, pmc=None,
     eps = numpy.asarray(epsilon).reshape(-1)
     dual_dxes = [[numpy.asarray(d)[::-1] for d in dxes[1]], [numpy.asarray(d)[::-1] for d in dxes[0]]]
     dual_eps = _rev_vec(mu, shape) if mu is not None else numpy.ones_like(eps)
-    A0 = _A0(omega, dual_dxes, dual_eps, _rev_vec(eps, shape), _rev_vec(pmc, shape), _rev_vec(pec, shape), device)
+    A0 = _A0(omega, dual_dxes, dual_eps, _rev_vec(eps, shape), _rev_vec(pmc, shape), _rev_vec(pec, shape), device,
+             reversed=True)
 
     def f(h):
         ht, like = _dev_field(h, A0.op)
-        return _from_device(_flip(A0(_flip(ht, shape)), shape), like)
+        return _from_device(A0(ht), like)
     return f
 
 

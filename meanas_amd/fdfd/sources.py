@@ -13,20 +13,20 @@ The step before the solve: these turn a desired E field into the current J that
 - `expand_e` and `compute_source` build the one-way source of a mode field
   (`meanas/fdfd/waveguide_3d.py:113-156,206-252`).
 
-A0 is applied on the GPU through the symmetrised operator: with the factored p of the
-device operator, A = P A0 P^-1, so A0 v = (1/p) A (p v) -- two diagonal maps around one
-FP64 apply (`mx_map`, `mx_apply`).  The masks are computed on the host (a few byte
-arrays); the fields and the applies stay on the device.
+Both products with A0 are formed in one pass over the field (`mx_wave_source`).  The masks
+are computed on the host (a few byte arrays); the fields stay on the device.
 """
 from __future__ import annotations
 
+import ctypes
 from typing import Callable, Sequence
 
 import numpy
 import torch
 
 from .. import _lib
-from .device import DeviceOperator
+from .device import DeviceOperator, grid_shape, torch_stream_handle
+from .functional import _Grid
 
 
 def _field_mask(mask, n3: int, ncell: int) -> numpy.ndarray:
@@ -43,20 +43,9 @@ def _field_mask(mask, n3: int, ncell: int) -> numpy.ndarray:
     raise ValueError(f'mask must have N = {ncell} or 3N = {n3} entries')
 
 
-class _A0:
-    """y = e_full(omega, dxes, epsilon, mu) @ x on the GPU (complex128)."""
-
-    def __init__(self, omega, dxes, epsilon, mu, device):
-        self.op = DeviceOperator(omega, dxes, epsilon, mu=mu, device=device)
-
-    def __call__(self, x: torch.Tensor) -> torch.Tensor:
-        px = self.op.map(_lib.MX_MAP_RHS, x, coef=1.0)          # p x
-        return self.op.map(_lib.MX_MAP_E, self.op.apply(px))    # (1/p) A (p x)
-
-
 def _to_dev(e, op: DeviceOperator) -> tuple[torch.Tensor, object]:
     if isinstance(e, torch.Tensor):
-        t = e.to(device=op.device, dtype=torch.complex128).reshape(-1).contiguous()
+        t = e.to(device=op.device, dtype=torch.complex128).reshape(-1).contiguous().resolve_conj()
         like = ('torch', tuple(e.shape))
     else:
         a = numpy.asarray(e)
@@ -72,14 +61,21 @@ def _from_dev(t: torch.Tensor, like):
     return t.reshape(shape) if kind == 'torch' else t.cpu().numpy().reshape(shape)
 
 
-def _masked_source(A0: _A0, q: torch.Tensor, keep: torch.Tensor | None, omega: complex) -> Callable:
+def _masked_source(omega, dxes, epsilon, mu, device, q, keep) -> Callable:
+    """`f(E) -> keep (A0 q E - q A0 E) / (-i omega)` for the 3N host masks q and keep (or
+    None), one pass over the field."""
+    op = DeviceOperator(omega, dxes, epsilon, mu=mu, device=device)
+    grid = _Grid(dxes, device)
+    q = torch.from_numpy(q).to(op.device)
+    keep = None if keep is None else torch.from_numpy(keep).to(op.device)
     c = 1.0 / (-1j * complex(omega))
 
     def f(e):
-        et, like = _to_dev(e, A0.op)
-        j = (A0(q * et) - q * A0(et)) * c
-        if keep is not None:
-            j = j * keep
+        et, like = _to_dev(e, op)
+        j = torch.empty_like(et)
+        _lib.check(_lib.lib().mx_wave_source(ctypes.byref(op.desc), ctypes.byref(grid.desc), q.data_ptr(),
+                                             None if keep is None else keep.data_ptr(), c.real, c.imag,
+                                             et.data_ptr(), j.data_ptr(), torch_stream_handle()), 'mx_wave_source')
         return _from_dev(j, like)
     return f
 
@@ -87,9 +83,8 @@ def _masked_source(A0: _A0, q: torch.Tensor, keep: torch.Tensor | None, omega: c
 def e_tfsf_source(TF_region, omega: complex, dxes, epsilon, mu=None,
                   device: str | torch.device = 'cuda') -> Callable:
     """`f(E) -> J = (A0 Q E - Q A0 E) / (-i omega)` (total-field / scattered-field source)."""
-    A0 = _A0(omega, dxes, epsilon, mu, device)
-    q = _field_mask(TF_region, A0.op.n3, A0.op.ncell)
-    return _masked_source(A0, torch.from_numpy(q).to(A0.op.device), None, omega)
+    ncell = int(numpy.prod(grid_shape(dxes)))
+    return _masked_source(omega, dxes, epsilon, mu, device, _field_mask(TF_region, 3 * ncell, ncell), None)
 
 
 def boundary_mask(mask, shape: Sequence[int], periodic_mask_edges: bool = False) -> numpy.ndarray:
@@ -117,12 +112,10 @@ def boundary_mask(mask, shape: Sequence[int], periodic_mask_edges: bool = False)
 def e_boundary_source(mask, omega: complex, dxes, epsilon, mu=None, periodic_mask_edges: bool = False,
                       device: str | torch.device = 'cuda') -> Callable:
     """`f(E) -> J`: the TFSF current of `mask`, kept only on the mask's edges."""
-    A0 = _A0(omega, dxes, epsilon, mu, device)
-    shape = A0.op.shape
-    q = _field_mask(mask, A0.op.n3, A0.op.ncell)
-    keep = boundary_mask(q, shape, periodic_mask_edges)
-    dev = A0.op.device
-    return _masked_source(A0, torch.from_numpy(q).to(dev), torch.from_numpy(keep).to(dev), omega)
+    shape = grid_shape(dxes)
+    ncell = int(numpy.prod(shape))
+    q = _field_mask(mask, 3 * ncell, ncell)
+    return _masked_source(omega, dxes, epsilon, mu, device, q, boundary_mask(q, shape, periodic_mask_edges))
 
 
 def expand_e(E, wavenumber: complex, dxes, axis: int, polarity: int, slices: Sequence[slice]) -> numpy.ndarray:
