@@ -44,26 +44,6 @@ __device__ __forceinline__ cplx<T> load_mat(const T* base, bool is_complex, bool
   return cplx<T>{gload1<T>(base, idx), T(0)};
 }
 
-// fa x1 - fb x0 with complex coefficients.  (Real-coefficient variants for axes outside
-// the PML, selected per plane and per wave, made the kernel 1.46x larger and measured 3%
-// slower in the 128^3 solve, so there is one form.)
-template <typename T>
-__device__ __forceinline__ cplx<T> dif(const cplx<T>& fa, const cplx<T>& x1, const cplx<T>& fb, const cplx<T>& x0) {
-  return fa * x1 - fb * x0;
-}
-
-// forward-difference coefficients (fa, fb) of entry n of a per-axis table; coef_u for
-// an n that is uniform over the wave (scalar loads, SGPRs)
-template <typename T> struct FaFb { cplx<T> fa, fb; };
-template <typename T>
-__device__ __forceinline__ FaFb<T> coef_at(const AxisCoef<T>* tab, int n) {
-  return FaFb<T>{gload<T>(tab, 4 * n), gload<T>(tab, 4 * n + 1)};
-}
-template <typename T>
-__device__ __forceinline__ FaFb<T> coef_u(const AxisCoef<T>* tab, int n) {
-  return FaFb<T>{cload<T>(tab, 4 * n), cload<T>(tab, 4 * n + 1)};
-}
-
 // Occupancy target (the second launch-bounds argument is the minimum number of waves
 // per SIMD): complex64 fits 4 waves (<= 128 VGPRs); complex128 needs 214 VGPRs, and
 // holding it to 3 waves (168) spills 117 of them to scratch, so it runs 2.
@@ -117,10 +97,12 @@ __global__ __launch_bounds__(64 * TY, (kWavesPerSimd<T, MK>)) void k_apply(const
   SysState* st = S.st;
   bool mr = false;     // rescue step: accumulate ||q||^2 instead of p^T q, q^T q
   bool keep_p = false;  // residual replacement that keeps the search direction
+  int cur = 0;          // state flags (which buffers hold r and p)
   if (EPI != EPI_PLAIN) {
     const int f = gload1<int>(&st->flags, 0);
     if ((f & skip_flags) || (need_flags && !(f & need_flags))) return;
     mr = (f & SF_MR) != 0;
+    cur = f;
     // fused iteration form only: the classic form rebuilds p in k_pupdate
     keep_p = EPI == EPI_RESID && (f & SF_FUSED) && !(f & (SF_MR | SF_RESTART)) && S.vec[VS_P] != nullptr;
   }
@@ -303,8 +285,12 @@ __global__ __launch_bounds__(64 * TY, (kWavesPerSimd<T, MK>)) void k_apply(const
   const cplx<T> w2 = op.w2;
   const bool diag_real = !eps_cplx && w2.im == T(0);
   const double* __restrict__ bvec = reinterpret_cast<const double*>(S.vec[VS_B]);
-  RT* __restrict__ rout = reinterpret_cast<RT*>(S.vec[out_slot]);
-  RT* __restrict__ pdir = reinterpret_cast<RT*>(S.vec[VS_P]);
+  // a replacement reads r and p where the one-launch iteration left them and writes both to
+  // their first buffers
+  RT* rout = reinterpret_cast<RT*>(S.vec[out_slot]);
+  RT* pdir = reinterpret_cast<RT*>(S.vec[VS_P]);
+  const RT* rcur = reinterpret_cast<const RT*>(S.vec[current_slot(VS_R, EPI == EPI_RESID ? cur : 0)]);
+  const RT* pcur = reinterpret_cast<const RT*>(S.vec[current_slot(VS_P, EPI == EPI_RESID ? cur : 0)]);
 
   // step i: Rn holds plane i+1; epsn holds eps of plane i, loaded during step i-1 ahead
   // of that step's plane prefetch (so waiting for it never waits for the prefetch)
@@ -410,8 +396,8 @@ __global__ __launch_bounds__(64 * TY, (kWavesPerSimd<T, MK>)) void k_apply(const
           if (keep_p) {
             // p was built from the recursive residual: p += r_true - r_recursive keeps
             // its direction component and swaps in the true residual
-            const cplx<RT> rold = gload<RT>(rout, idx);
-            gstore<RT>(pdir, idx, gload<RT>(pdir, idx) + (rs - rold));
+            const cplx<RT> rold = gload<RT>(rcur, idx);
+            gstore<RT>(pdir, idx, gload<RT>(pcur, idx) + (rs - rold));
           }
           gstore<RT>(rout, idx, rs);
           const cplx<double> rd = cast<double>(rs);

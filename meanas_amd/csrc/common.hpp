@@ -162,6 +162,26 @@ __device__ __forceinline__ void pstore_nt(void* base, long long i, typename Pack
 // scaling p used to map J -> b and x -> E.
 template <typename T> struct AxisCoef { cplx<T> fa, fb, se, sh; };
 
+// fa x1 - fb x0 with complex coefficients.  (Real-coefficient variants for axes outside
+// the PML, selected per plane and per wave, made the kernel 1.46x larger and measured 3%
+// slower in the 128^3 solve, so there is one form.)
+template <typename T>
+__device__ __forceinline__ cplx<T> dif(const cplx<T>& fa, const cplx<T>& x1, const cplx<T>& fb, const cplx<T>& x0) {
+  return fa * x1 - fb * x0;
+}
+
+// forward-difference coefficients (fa, fb) of entry n of a per-axis table; coef_u for
+// an n that is uniform over the wave (scalar loads, SGPRs)
+template <typename T> struct FaFb { cplx<T> fa, fb; };
+template <typename T>
+__device__ __forceinline__ FaFb<T> coef_at(const AxisCoef<T>* tab, int n) {
+  return FaFb<T>{gload<T>(tab, 4 * n), gload<T>(tab, 4 * n + 1)};
+}
+template <typename T>
+__device__ __forceinline__ FaFb<T> coef_u(const AxisCoef<T>* tab, int n) {
+  return FaFb<T>{cload<T>(tab, 4 * n), cload<T>(tab, 4 * n + 1)};
+}
+
 // Material / mask format flags of an operator.
 enum : int {
   OPF_EPS_COMPLEX = 1,   // eps interleaved complex, else real
@@ -213,6 +233,8 @@ enum : int {
   SF_UPD_PENDING = 16384, // the update ran; its partials await the post-update finishing step
   SF_XPEND     = 32768, // fused form: x_lo still lacks the last alpha p, kept as xa (p - r)
   SF_XSKIP     = 65536, // fused form: the coming update pass leaves x_lo alone (it defers alpha p)
+  SF_ALT       = 131072, // one-launch iteration: the r and p of this paused system are in VS_R2, VS_P2
+  SF_QVALID    = 262144, // one-launch iteration: q and its sums belong to the current p
 };
 
 // Deferred solution update of the fused form: an update pass may leave x_lo alone when
@@ -261,7 +283,12 @@ struct SysState {
 enum : int { FIN_APPLY = 0, FIN_UPDATE = 1, FIN_RESID = 2, FIN_BNORM = 3, FIN_APPLY_MERGED = 4 };
 
 // One linear system of a batch.  Vector slots name the vectors a kernel reads/writes.
-enum : int { VS_X = 0, VS_R, VS_P, VS_Q, VS_XLO, VS_B, VS_XBEST, VS_COUNT };
+// (VS_R2.. are the second buffers of the one-launch iteration, iter.hip; null without it.)
+enum : int { VS_X = 0, VS_R, VS_P, VS_Q, VS_XLO, VS_B, VS_XBEST, VS_R2, VS_P2, VS_Q2, VS_COUNT };
+// slot of the current r or p of a paused system with state flags f
+__host__ __device__ __forceinline__ constexpr int current_slot(int slot, int f) {
+  return (f & SF_ALT) ? slot + (VS_R2 - VS_R) : slot;
+}
 
 struct SysDesc {
   int op;                     // operator index
@@ -274,6 +301,10 @@ struct SysDesc {
   double* partial;            // >= 4 * max(nblk_apply, nblk_vec) doubles
   double* partial_vec;        // >= 3 * nblk_vec doubles: the update's partials, kept apart
                               // so the next apply can run before they are summed
+  // one-launch iteration (nblk_iter > 0): state and partials alternate between two copies
+  int nblk_iter;              // its blocks
+  SysState* st2;              // the state's second copy (st is the first)
+  double* part_it[2];         // 7 * nblk_iter doubles each
 };
 
 // Work assignment of one block: system index and block index within that system.

@@ -37,6 +37,12 @@ hipError_t launch_save_best(const SysDesc*, const BlockMap*, int, hipStream_t);
 hipError_t launch_zero_slot(int prec64, const SysDesc*, const BlockMap*, int, int, hipStream_t);
 hipError_t launch_fin(int kind, const SysDesc*, const int* syslist, int nsys, hipStream_t);
 hipError_t launch_diag(const AxisCoef<double>*, int, int, int, const void*, void*, double, double, int, hipStream_t);
+// iter.hip
+int iter_blocks(int nx, int ny, int nz);
+constexpr int kIterTileCells = 512;   // cells of a tile
+hipError_t launch_iterations(int kind, const SysDesc* one_sys, const OpView<double>* one_op, const OpView<double>* ops,
+                             const SysDesc* sys, const BlockMap* bmap, int nb, const int* syslist, int nsys, int n,
+                             hipStream_t s);
 }  // namespace mx
 
 using namespace mx;
@@ -139,6 +145,27 @@ int refresh_iters(int stall_iters) {
 // Material kind of an operator (common.hpp): the apply kernel its launches use.
 int op_kind(const mx_operator& op) { return mat_kind(view_of<double>(op).flags); }
 
+// Which systems run the one-launch iteration (iter.hip) in the fused form: complex128 grids of
+// few tiles that fill those tiles well.  A system's own grid decides, never the batch, so that
+// its bits do not depend on the batch.  Alone, one launch wins far beyond this line
+// (microseconds per iteration, three launches / one: 16^3 22.7 / 10.7, 48^3 29.8 / 14.4,
+// 64^3 38.5 / 22.4), but in a batch that fills the GPU its per-tile work decides: it costs
+// about the same per tile at every size while the three launches get cheaper per cell.
+// Batches of about 1.2 million cells, three launches / one:
+//   tiles used well: 20^3 183 / 148, 40x44x36 123 / 113, 48^3 118.3 / 118.6, 48^3 with mu
+//   faster, 56^3 120 / 129, 64^3 162 / 181: the line is at 216 tiles (48^3);
+//   partly empty tiles (padded / cells): 12^3 (2.4) 168 / 115, 25^3 (2.1) 157 / 154,
+//   33^3 (1.8) 133 / 137, 41^3 (1.6) 116 / 126, 43^3 (1.4) 115 / 117, 37^3 (1.3) 127 / 121:
+//   above 72 tiles at most 1.4.
+constexpr int kIterTiles = 216, kIterAnyFill = 72;
+bool one_launch(const mx_operator& op, int mode) {
+  if (mode != MX_FP64) return false;
+  const long long tiles = iter_blocks(op.nx, op.ny, op.nz);
+  return tiles <= kIterAnyFill || (tiles <= kIterTiles && tiles * kIterTileCells * 10 <= ncell_of(op) * 14);
+}
+// Iterations per chunk of a batch of such systems
+constexpr int kOneLaunchChunk = 32;
+
 // One finishing launch per fused iteration (default); MEANAS_AMD_MERGED_FIN=0 launches
 // the post-apply and post-update finishing kernels separately (same results).
 bool merged_fin_enabled() {
@@ -188,7 +215,10 @@ size_t elem_bytes(int mode) { return mode == MX_MIXED ? 8 : 16; }
 // workspace layout per system: r, p, q, x_lo (inner precision), x_best (FP64), state,
 // partials (apply and reductions), the update's partials
 struct WorkLayout {
-  size_t off_r, off_p, off_q, off_xlo, off_xbest, off_state, off_partial, off_partial_vec, total;
+  size_t off_r, off_p, off_q, off_xlo, off_xbest, off_state, off_partial, off_partial_vec;
+  size_t off_r2, off_p2, off_q2, off_state2, off_part_it[2];   // one-launch iteration only
+  int nblk_iter;                                               // 0: not that form
+  size_t total;
 };
 
 WorkLayout work_layout(const mx_operator& op, int mode) {
@@ -205,7 +235,39 @@ WorkLayout work_layout(const mx_operator& op, int mode) {
   const size_t nbmax = (size_t)std::max(apply_blocks_upper(op), kVecMaxBlocks);
   w.off_partial_vec = w.off_partial + align_up(4 * nbmax * sizeof(double));
   w.total = w.off_partial_vec + align_up(3 * (size_t)kVecMaxBlocks * sizeof(double));
+  w.nblk_iter = 0;
+  if (one_launch(op, mode)) {   // the second buffers of r, p, q and of the state; two sets of partials
+    w.nblk_iter = iter_blocks(op.nx, op.ny, op.nz);
+    const size_t pb = align_up(7 * (size_t)w.nblk_iter * sizeof(double));
+    w.off_r2 = w.total;
+    w.off_p2 = w.off_r2 + vb;
+    w.off_q2 = w.off_p2 + vb;
+    w.off_state2 = w.off_q2 + vb;
+    w.off_part_it[0] = w.off_state2 + align_up(sizeof(SysState));
+    w.off_part_it[1] = w.off_part_it[0] + pb;
+    w.total = w.off_part_it[1] + pb;
+  }
   return w;
+}
+
+// The workspace pointers of a system's descriptor.
+void set_work(SysDesc& d, const WorkLayout& w, char* wk) {
+  d.vec[VS_R] = wk + w.off_r;
+  d.vec[VS_P] = wk + w.off_p;
+  d.vec[VS_Q] = wk + w.off_q;
+  d.vec[VS_XLO] = wk + w.off_xlo;
+  d.vec[VS_XBEST] = wk + w.off_xbest;
+  d.st = reinterpret_cast<SysState*>(wk + w.off_state);
+  d.partial = reinterpret_cast<double*>(wk + w.off_partial);
+  d.partial_vec = reinterpret_cast<double*>(wk + w.off_partial_vec);
+  d.nblk_iter = w.nblk_iter;
+  if (w.nblk_iter > 0) {
+    d.vec[VS_R2] = wk + w.off_r2;
+    d.vec[VS_P2] = wk + w.off_p2;
+    d.vec[VS_Q2] = wk + w.off_q2;
+    d.st2 = reinterpret_cast<SysState*>(wk + w.off_state2);
+    for (int i = 0; i < 2; ++i) d.part_it[i] = reinterpret_cast<double*>(wk + w.off_part_it[i]);
+  }
 }
 
 // Order the blocks of a grid so that each XCD (blocks are dispatched round-robin over
@@ -235,7 +297,9 @@ std::vector<BlockMap> xcd_order(const std::vector<BlockMap>& natural) {
 // many small systems also fills the GPU that one of them would leave idle.  A system's
 // block partition does not depend on its group, so results do not either.
 // reps: times a chunk repeats this group's iterations (sessions: equal time per group)
-struct Group { int a_off, na, v_off, nv, s_off, ns, ty, kind, reps = 1; };
+// ni: blocks of the one-launch iteration (0: a group of three-launch systems)
+// sys0: its first system (batch or slot index)
+struct Group { int a_off, na, v_off, nv, s_off, ns, ty, kind, i_off = 0, ni = 0, sys0 = 0, reps = 1; };
 
 // MALL bytes a launch group may fill (MEANAS_AMD_CACHE_MB overrides; 0: one group)
 size_t cache_budget() {
@@ -247,8 +311,11 @@ size_t cache_budget() {
   return b;
 }
 
-// bytes of one system's p and q, and of its operator's materials, in the inner precision
-size_t vec_hot_bytes(const mx_operator& op, int mode) { return 2 * (size_t)(3 * ncell_of(op)) * elem_bytes(mode); }
+// bytes of one system's p and q (of both copies of r, p and q and of x_lo in the one-launch
+// iteration), and of its operator's materials, in the inner precision
+size_t vec_hot_bytes(const mx_operator& op, int mode, bool one) {
+  return (one ? 7 : 2) * (size_t)(3 * ncell_of(op)) * elem_bytes(mode);
+}
 size_t mat_hot_bytes(const mx_operator& op, int mode) {
   const size_t n = (size_t)ncell_of(op), real = mode == MX_MIXED ? 4 : 8;
   auto mat = [&](bool cplx, bool aniso) { return (aniso ? 3 : 1) * n * real * (cplx ? 2 : 1); };
@@ -269,11 +336,18 @@ struct Batch {
   SysDesc* d_sys = nullptr;
   BlockMap* d_bmap_apply = nullptr;
   BlockMap* d_bmap_vec = nullptr;
+  BlockMap* d_bmap_iter = nullptr;   // of the group being enqueued, if it is of one-launch systems
+  int nb_iter = 0;
+  int sys0 = 0;                      // that group's first system
+  const SysDesc* host_sys = nullptr;       // host copies of the tables (one-system launches take theirs by value)
+  const mx_operator* host_ops = nullptr;
+  bool fused_form = false;           // the options' iteration form is the fused one
   int* d_syslist = nullptr;   // systems the finishing kernels visit (one block each)
   int nsl = 0;
   // the whole (all groups) maps; d_bmap_apply etc. point at one group while it is enqueued
   BlockMap* bm_apply0 = nullptr;
   BlockMap* bm_vec0 = nullptr;
+  BlockMap* bm_iter0 = nullptr;
   int* syslist0 = nullptr;
   int nb_apply0 = 0, nb_vec0 = 0, nsl0 = 0;
   std::vector<Group> groups;
@@ -295,11 +369,13 @@ struct Batch {
     ty = g.ty; kind = g.kind;
     d_bmap_apply = bm_apply0 + g.a_off; nb_apply = g.na;
     d_bmap_vec = bm_vec0 + g.v_off; nb_vec = g.nv;
+    d_bmap_iter = bm_iter0 ? bm_iter0 + g.i_off : nullptr; nb_iter = g.ni; sys0 = g.sys0;
     d_syslist = syslist0 + g.s_off; nsl = g.ns;
   }
   void use_all() {
     d_bmap_apply = bm_apply0; nb_apply = nb_apply0;
     d_bmap_vec = bm_vec0; nb_vec = nb_vec0;
+    d_bmap_iter = nullptr; nb_iter = 0;
     d_syslist = syslist0; nsl = nsl0;
   }
 
@@ -320,20 +396,24 @@ struct Member {
   int op_id;                // systems with the same op_id share materials
   int ty;                   // apply tile height
   int kind;                 // material kind (op_kind)
-  int na, nv;               // apply and vector blocks
+  int na, nv, ni;           // apply and vector blocks; one-launch iteration blocks (0: three launches)
 };
 
-// Lay `members` out as consecutive launch groups (see Group): one tile height and one
-// material kind per group, and within those, consecutive members
+// Lay `members` out as consecutive launch groups (see Group): one tile height, one
+// material kind and one launch form per group, and within those, consecutive members
 // while their hot bytes fit the cache budget.  Each group's maps are XCD-ordered on their
-// own; apply, vec and sl receive the concatenated maps and system lists.
+// own; apply, vec, iter and sl receive the concatenated maps and system lists.
 void make_groups(const std::vector<Member>& members, int mode, std::vector<BlockMap>& apply,
-                 std::vector<BlockMap>& vec, std::vector<int>& sl, std::vector<Group>& groups) {
+                 std::vector<BlockMap>& vec, std::vector<BlockMap>& iter, std::vector<int>& sl,
+                 std::vector<Group>& groups) {
   const size_t budget = cache_budget();
-  apply.clear(); vec.clear(); sl.clear(); groups.clear();
+  apply.clear(); vec.clear(); iter.clear(); sl.clear(); groups.clear();
   for (int ty : {2, 4, 8})
-    for (int kind : {MK_SIMPLE, MK_ANISO, MK_MASK, MK_GENERAL}) {
-      std::vector<BlockMap> ga, gv;
+    for (int kind_form = 0; kind_form < 8; ++kind_form) {
+      constexpr int kKinds[4] = {MK_SIMPLE, MK_ANISO, MK_MASK, MK_GENERAL};
+      const int kind = kKinds[kind_form / 2];
+      const bool one = kind_form % 2 != 0;
+      std::vector<BlockMap> ga, gv, gi;
       std::vector<int> gs, gops;
       size_t bytes = 0;
       auto close = [&]() {
@@ -344,22 +424,26 @@ void make_groups(const std::vector<Member>& members, int mode, std::vector<Block
         apply.insert(apply.end(), oa.begin(), oa.end());
         vec.insert(vec.end(), ov.begin(), ov.end());
         sl.insert(sl.end(), gs.begin(), gs.end());
-        g.na = (int)oa.size(); g.nv = (int)ov.size(); g.ns = (int)gs.size();
-        g.ty = ty; g.kind = kind;
+        const std::vector<BlockMap> oi = xcd_order(gi);
+        g.i_off = (int)iter.size();
+        iter.insert(iter.end(), oi.begin(), oi.end());
+        g.na = (int)oa.size(); g.nv = (int)ov.size(); g.ns = (int)gs.size(); g.ni = (int)oi.size();
+        g.ty = ty; g.kind = kind; g.sys0 = gs[0];
         groups.push_back(g);
-        ga.clear(); gv.clear(); gs.clear(); gops.clear();
+        ga.clear(); gv.clear(); gi.clear(); gs.clear(); gops.clear();
         bytes = 0;
       };
       for (const Member& m : members) {
-        if (m.ty != ty || m.kind != kind) continue;
+        if (m.ty != ty || m.kind != kind || (m.ni > 0) != one) continue;
         const bool new_op = std::find(gops.begin(), gops.end(), m.op_id) == gops.end();
-        const size_t add = vec_hot_bytes(*m.op, mode) + (new_op ? mat_hot_bytes(*m.op, mode) : 0);
+        const size_t add = vec_hot_bytes(*m.op, mode, one) + (new_op ? mat_hot_bytes(*m.op, mode) : 0);
         if (budget > 0 && !gs.empty() && bytes + add > budget) close();
         if (std::find(gops.begin(), gops.end(), m.op_id) == gops.end()) gops.push_back(m.op_id);
         bytes += add;
         gs.push_back(m.sys);
         for (int b = 0; b < m.na; ++b) ga.push_back({m.sys, b});
         for (int b = 0; b < m.nv; ++b) gv.push_back({m.sys, b});
+        for (int b = 0; b < m.ni; ++b) gi.push_back({m.sys, b});
       }
       close();
     }
@@ -372,15 +456,16 @@ int layout_groups(Batch& B, const std::vector<char>& active) {
   for (int s = 0; s < B.nsys; ++s)
     if (active[s])
       members.push_back({s, &B.ops[B.h_op[s]], B.h_op[s], B.h_ty[s], op_kind(B.ops[B.h_op[s]]),
-                         B.h_sys[s].nblk_apply, B.h_sys[s].nblk_vec});
-  std::vector<BlockMap> apply, vec;
+                         B.h_sys[s].nblk_apply, B.h_sys[s].nblk_vec, B.fused_form ? B.h_sys[s].nblk_iter : 0});
+  std::vector<BlockMap> apply, vec, iter;
   std::vector<int> sl;
-  make_groups(members, B.mode, apply, vec, sl, B.groups);
+  make_groups(members, B.mode, apply, vec, iter, sl, B.groups);
   B.nb_apply0 = (int)apply.size();
   B.nb_vec0 = (int)vec.size();
   B.nsl0 = (int)sl.size();
   if (!apply.empty()) MX_TRY(copy_now(B.bm_apply0, apply.data(), sizeof(BlockMap) * apply.size(), hipMemcpyHostToDevice));
   if (!vec.empty()) MX_TRY(copy_now(B.bm_vec0, vec.data(), sizeof(BlockMap) * vec.size(), hipMemcpyHostToDevice));
+  if (!iter.empty()) MX_TRY(copy_now(B.bm_iter0, iter.data(), sizeof(BlockMap) * iter.size(), hipMemcpyHostToDevice));
   if (!sl.empty()) MX_TRY(copy_now(B.syslist0, sl.data(), sizeof(int) * sl.size(), hipMemcpyHostToDevice));
   B.use_all();
   return 0;
@@ -389,6 +474,7 @@ int layout_groups(Batch& B, const std::vector<char>& active) {
 int build_batch(Batch& B, const mx_operator* ops, int nops, const mx_system* sys, int nsys, const mx_options& o) {
   std::string why;
   B.mode = o.mode;
+  B.fused_form = o.form == MX_FORM_FUSED;
   B.nops = nops;
   B.nsys = nsys;
   B.ops = ops;
@@ -398,7 +484,7 @@ int build_batch(Batch& B, const mx_operator* ops, int nops, const mx_system* sys
   for (int i = 0; i < nops; ++i)
     if (!valid_op(ops[i], o.mode, &why)) return fail("operator " + std::to_string(i) + ": " + why);
 
-  size_t total_apply = 0, total_vec = 0;
+  size_t total_apply = 0, total_vec = 0, total_iter = 0;
   B.h_sys.resize(nsys);
   B.h_op.resize(nsys);
   B.h_ty.resize(nsys);
@@ -424,19 +510,13 @@ int build_batch(Batch& B, const mx_operator* ops, int nops, const mx_system* sys
                   " apply blocks exceed the reduction limit; use a deeper slab");
     d.vec[VS_X] = y.x;
     d.vec[VS_B] = const_cast<void*>(y.b);
-    d.vec[VS_R] = wk + w.off_r;
-    d.vec[VS_P] = wk + w.off_p;
-    d.vec[VS_Q] = wk + w.off_q;
-    d.vec[VS_XLO] = wk + w.off_xlo;
-    d.vec[VS_XBEST] = wk + w.off_xbest;
-    d.st = reinterpret_cast<SysState*>(wk + w.off_state);
-    d.partial = reinterpret_cast<double*>(wk + w.off_partial);
-    d.partial_vec = reinterpret_cast<double*>(wk + w.off_partial_vec);
+    set_work(d, w, wk);
     B.h_sys[s] = d;
     B.h_op[s] = y.op;
     B.h_ty[s] = ty;
     total_apply += d.nblk_apply;
     total_vec += d.nblk_vec;
+    total_iter += d.nblk_iter;
   }
 
   const size_t s_ops32 = align_up(sizeof(OpView<float>) * nops);
@@ -444,14 +524,16 @@ int build_batch(Batch& B, const mx_operator* ops, int nops, const mx_system* sys
   const size_t s_sys = align_up(sizeof(SysDesc) * nsys);
   const size_t s_ba = align_up(sizeof(BlockMap) * total_apply);
   const size_t s_bv = align_up(sizeof(BlockMap) * total_vec);
+  const size_t s_bi = align_up(sizeof(BlockMap) * total_iter);
   const size_t s_sl = align_up(sizeof(int) * nsys);
-  MX_TRY(hipMalloc(&B.d_mem, s_ops32 + s_ops64 + s_sys + s_ba + s_bv + s_sl));
+  MX_TRY(hipMalloc(&B.d_mem, s_ops32 + s_ops64 + s_sys + s_ba + s_bv + s_bi + s_sl));
   char* p = B.d_mem;
   B.d_ops32 = reinterpret_cast<OpView<float>*>(p); p += s_ops32;
   B.d_ops64 = reinterpret_cast<OpView<double>*>(p); p += s_ops64;
   B.d_sys = reinterpret_cast<SysDesc*>(p); p += s_sys;
   B.bm_apply0 = reinterpret_cast<BlockMap*>(p); p += s_ba;
   B.bm_vec0 = reinterpret_cast<BlockMap*>(p); p += s_bv;
+  B.bm_iter0 = reinterpret_cast<BlockMap*>(p); p += s_bi;
   B.syslist0 = reinterpret_cast<int*>(p);
 
   std::vector<OpView<float>> v32(nops);
@@ -515,6 +597,17 @@ int enqueue_replacement(Batch& B, hipStream_t s) {
 }
 
 int enqueue_group_chunk(Batch& B, hipStream_t s, int iters, int check_every) {
+  if (B.nb_iter > 0) {   // one-launch systems: runs of launches between the replacement points
+    const SysDesc* one = B.nsl == 1 ? &B.host_sys[B.sys0] : nullptr;
+    OpView<double> op;
+    if (one) op = view_of<double>(B.host_ops[one->op]);
+    for (int it = 0; it < iters; it += check_every) {
+      MX_TRY(launch_iterations(B.kind, one, one ? &op : nullptr, B.d_ops64, B.d_sys, B.d_bmap_iter, B.nb_iter,
+                               B.d_syslist, B.nsl, std::min(check_every, iters - it), s));
+      if (enqueue_replacement(B, s)) return -1;
+    }
+    return 0;
+  }
   for (int it = 0; it < iters; ++it) {
     if (enqueue_iteration(B, s)) return -1;
     if ((it + 1) % check_every == 0 || it + 1 == iters) {
@@ -545,6 +638,12 @@ int enqueue_replacement_groups(Batch& B, hipStream_t s) {
 // is the same chunk with the same check points, so a system's iterates do not depend on
 // how often its group repeats.
 int enqueue_chunk(Batch& B, hipStream_t s, int iters, int check_every) {
+  // a batch's own tables, this call's (a kept batch outlives the caller's array of the call
+  // before); a session's view has none and is given the session's
+  if (!B.h_sys.empty()) {
+    B.host_sys = B.h_sys.data();
+    B.host_ops = B.ops;
+  }
   if (B.groups.empty()) return enqueue_group_chunk(B, s, iters, check_every);
   int rc = 0;
   for (const Group& g : B.groups) {
@@ -1045,7 +1144,14 @@ int mx_solve_plan_release(void) {
 int mx_solve(const mx_operator* ops, int32_t nops, const mx_system* systems, int32_t nsys, const mx_options* opt,
              mx_stats* stats, void* stream) {
   if (!ops || nops < 1 || !systems || nsys < 1) return fail("mx_solve: empty batch");
-  const mx_options o = defaults(opt);
+  mx_options o = defaults(opt);
+  // a batch of one-launch systems takes longer chunks by default: the seven launches that
+  // close a chunk cost as much as two of its iterations
+  if ((!opt || opt->chunk <= 0) && o.form == MX_FORM_FUSED &&
+      std::all_of(ops, ops + nops, [&](const mx_operator& op) { return one_launch(op, o.mode); })) {
+    if (o.check_every == o.chunk) o.check_every = kOneLaunchChunk;
+    o.chunk = kOneLaunchChunk;
+  }
   std::string why;
   if (!valid_options(o, &why)) return fail(why);
   PlanUse plan;
@@ -1219,7 +1325,7 @@ struct mx_session {
   OpView<float>* d_ops32 = nullptr;
   OpView<double>* d_ops64 = nullptr;
   SysDesc* d_sys = nullptr;
-  BlockMap* d_bm = nullptr;              // combined maps: apply blocks, then vector blocks
+  BlockMap* d_bm = nullptr;              // combined maps: apply, vector and one-launch iteration blocks
   size_t bm_cap = 0;
   BlockMap* d_adm = nullptr;             // maps of the slot being admitted
   size_t adm_cap = 0;
@@ -1284,7 +1390,8 @@ int ensure_staging(mx_session* S, size_t need) {
 // maps of the admitted slot (one group of tile height ty), or with `groups` the launch
 // groups of every active slot.
 Batch session_batch(mx_session* S, const BlockMap* bm_apply, int nb_apply, const BlockMap* bm_vec, int nb_vec,
-                    const int* syslist, int nsl, int ty, int kind, const std::vector<Group>* groups = nullptr) {
+                    const int* syslist, int nsl, int ty, int kind, const std::vector<Group>* groups = nullptr,
+                    const BlockMap* bm_iter = nullptr) {
   Batch B;
   B.mode = S->o.mode;
   B.d_ops32 = S->d_ops32;
@@ -1292,6 +1399,7 @@ Batch session_batch(mx_session* S, const BlockMap* bm_apply, int nb_apply, const
   B.d_sys = S->d_sys;
   B.bm_apply0 = const_cast<BlockMap*>(bm_apply);
   B.bm_vec0 = const_cast<BlockMap*>(bm_vec);
+  B.bm_iter0 = const_cast<BlockMap*>(bm_iter);
   B.syslist0 = const_cast<int*>(syslist);
   B.nb_apply0 = nb_apply;
   B.nb_vec0 = nb_vec;
@@ -1338,20 +1446,21 @@ int session_rebuild(mx_session* S) {
   for (int i = 0; i < S->capacity; ++i)
     if (S->active[i])
       members.push_back({i, &S->h_ops[i], i, S->h_ty[i], op_kind(S->h_ops[i]), S->h_sys[i].nblk_apply,
-                         S->h_sys[i].nblk_vec});
-  std::vector<BlockMap> a, v;
+                         S->h_sys[i].nblk_vec, S->o.form == MX_FORM_FUSED ? S->h_sys[i].nblk_iter : 0});
+  std::vector<BlockMap> a, v, it;
   std::vector<int> sl;
-  make_groups(members, S->o.mode, a, v, sl, S->groups);
+  make_groups(members, S->o.mode, a, v, it, sl, S->groups);
   session_group_reps(S, sl);
   S->nsl = (int)sl.size();
   S->nb_apply = (int)a.size();
   S->nb_vec = (int)v.size();
-  const size_t need = a.size() + v.size();
+  const size_t need = a.size() + v.size() + it.size();
   if (ensure_device(&S->d_bm, &S->bm_cap, std::max<size_t>(need, 1), S->stream)) return -1;
   if (ensure_staging(S, std::max<size_t>(need, 1))) return -1;
   MX_TRY(hipStreamSynchronize(S->stream));   // staging buffer reuse
   std::copy(a.begin(), a.end(), S->h_bm);
   std::copy(v.begin(), v.end(), S->h_bm + a.size());
+  std::copy(it.begin(), it.end(), S->h_bm + a.size() + v.size());
   if (need) MX_TRY(hipMemcpyAsync(S->d_bm, S->h_bm, need * sizeof(BlockMap), hipMemcpyHostToDevice, S->stream));
   if (!sl.empty()) MX_TRY(copy_now(S->d_syslist, sl.data(), sizeof(int) * sl.size(), hipMemcpyHostToDevice));
   if (S->gexec) { MX_TRY(hipGraphExecDestroy(S->gexec)); S->gexec = nullptr; }
@@ -1424,14 +1533,7 @@ int mx_session_admit(mx_session* S, const mx_operator* op, const mx_system* y, v
   if (d.nblk_apply > kMaxPartials) return fail("too many apply blocks for one system; use a deeper slab");
   d.vec[VS_X] = y->x;
   d.vec[VS_B] = const_cast<void*>(y->b);
-  d.vec[VS_R] = wk + w.off_r;
-  d.vec[VS_P] = wk + w.off_p;
-  d.vec[VS_Q] = wk + w.off_q;
-  d.vec[VS_XLO] = wk + w.off_xlo;
-  d.vec[VS_XBEST] = wk + w.off_xbest;
-  d.st = reinterpret_cast<SysState*>(wk + w.off_state);
-  d.partial = reinterpret_cast<double*>(wk + w.off_partial);
-  d.partial_vec = reinterpret_cast<double*>(wk + w.off_partial_vec);
+  set_work(d, w, wk);
   S->h_sys[slot] = d;
   S->h_ops[slot] = *op;
   S->h_ty[slot] = ty;
@@ -1493,7 +1595,10 @@ int mx_session_step(mx_session* S, int32_t iterations, void* stream) {
   if (S->dirty && session_rebuild(S)) return -1;
   if (S->nb_apply == 0 || iterations <= 0) return 0;
   Batch B = session_batch(S, S->d_bm, S->nb_apply, S->d_bm + S->nb_apply, S->nb_vec, S->d_syslist, S->nsl, S->ty,
-                          MK_GENERAL, &S->groups);   // each launch group carries its own kind
+                          MK_GENERAL, &S->groups,   // each launch group carries its own kind
+                          S->d_bm + S->nb_apply + S->nb_vec);
+  B.host_sys = S->h_sys.data();
+  B.host_ops = S->h_ops.data();
   B.classic_launch = S->o.form != MX_FORM_FUSED;
   B.merged_fin = !B.classic_launch && merged_fin_enabled();
   const int check = std::min<int>(S->o.check_every, iterations);

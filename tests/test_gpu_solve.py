@@ -171,6 +171,50 @@ def test_batch_equals_alone_bitwise():
         assert numpy.array_equal(mixed[k], alone[i])
 
 
+# (42x41x17 with mu, PEC and PMC does not converge in 20000 iterations, in either form)
+@pytest.mark.parametrize('shape, variant',
+                         [(shape, variant) for shape in [(8, 8, 8), (9, 7, 10), (17, 2, 9), (1, 16, 11), (16, 24, 8),
+                                                         (42, 41, 9), (42, 41, 17)]
+                          for variant in ['iso', 'aniso', 'iso_pec', 'mu_pec_pmc']
+                          if not (shape == (42, 41, 17) and variant == 'mu_pec_pmc')])
+def test_small_fp64_systems_at_tile_edges(shape, variant):
+    """Small complex128 systems iterate in one launch over 8x8x8 tiles, larger or poorly
+    filling ones (42x41x17) in three: grids of whole tiles, one cell more or less, and thinner
+    than a tile, for each kind of material.  The scaled residual is at most rtol 1e-10 and the
+    field scaling of these grids (2 cells of PML) is below 100, so the physical residual is
+    below 1e-8 -- with even and odd run lengths between the checks, and with the same bits
+    beside another system as alone."""
+    import torch
+    from meanas_amd import _lib
+    from meanas_amd.fdfd.device import DeviceOperator, solve_batch
+    pec_pmc = dict(iso={}, aniso={}, iso_pec=dict(pec_frac=0.05),
+                   mu_pec_pmc=dict(pec_frac=0.05, pmc_frac=0.05, with_mu=True))[variant]
+    omega, dxes, J, eps, mu, pec, pmc = small_problem(shape, 77, **pec_pmc)
+    n = eps.size // 3
+    if variant != 'mu_pec_pmc':
+        eps = eps.real if variant == 'aniso' else numpy.tile(eps.real[:n], 3)
+    op = DeviceOperator(omega, dxes, eps, mu=mu, pec=pec, pmc=pmc)
+    b = op.map(_lib.MX_MAP_RHS, torch.from_numpy(J).cuda(), coef=-1j * omega)
+    other = small_problem((11, 9, 12), 78)
+    op2 = DeviceOperator(other[0], other[1], other[3])
+    b2 = op2.map(_lib.MX_MAP_RHS, torch.from_numpy(other[2]).cuda(), coef=-1j * other[0])
+
+    def run(batch, options=None):
+        xs = [torch.zeros_like(v) for v in (b, b2)[:batch]]
+        st = solve_batch([op, op2][:batch],
+                         [dict(op=i, b=(b, b2)[i], x=x, rtol=1e-10, maxiter=20000) for i, x in enumerate(xs)],
+                         mode=_lib.MX_FP64, options=options)
+        assert st[0]['status'] == 'converged', st
+        return xs[0]
+    A0 = ref.e_full(omega, dxes, eps, mu, pec=pec, pmc=pmc)
+    b0 = -1j * omega * J
+    for options in (None, dict(chunk=7, check_every=7), dict(chunk=5, check_every=1)):
+        x = run(1, options)
+        E = op.map(_lib.MX_MAP_E, x).cpu().numpy()
+        assert rel(A0 @ E, b0) < 1e-8
+        assert torch.equal(run(2, options), x)
+
+
 @pytest.mark.parametrize('maxiter', [3, 40])
 def test_maxiter_returns_best_iterate_with_status(maxiter):
     """An unconverged solve returns its best FP64 iterate (lowest true residual seen at a
