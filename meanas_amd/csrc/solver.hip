@@ -147,21 +147,25 @@ int op_kind(const mx_operator& op) { return mat_kind(view_of<double>(op).flags);
 
 // Which systems run the one-launch iteration (iter.hip) in the fused form: complex128 grids of
 // few tiles that fill those tiles well.  A system's own grid decides, never the batch, so that
-// its bits do not depend on the batch.  Alone, one launch wins far beyond this line
+// its bits do not depend on the batch.  Alone, one launch wins beyond this line
 // (microseconds per iteration, three launches / one: 16^3 22.7 / 10.7, 48^3 29.8 / 14.4,
-// 64^3 38.5 / 22.4), but in a batch that fills the GPU its per-tile work decides: it costs
-// about the same per tile at every size while the three launches get cheaper per cell.
-// Batches of about 1.2 million cells, three launches / one:
-//   tiles used well: 20^3 183 / 148, 40x44x36 123 / 113, 48^3 118.3 / 118.6, 48^3 with mu
-//   faster, 56^3 120 / 129, 64^3 162 / 181: the line is at 216 tiles (48^3);
+// 64^3 38.5 / 22.4, 72^3 50 / 32), but in a batch that fills the GPU its per-tile work decides:
+// it costs about the same per tile at every size, full or not, while the three launches get
+// cheaper per cell.  Batches of 1 to 2 million cells, three launches / one, each in the
+// lanes that its group gets:
+//   tiles used well: 20^3 183 / 148, 40^3 x16 105 / 83, 48^3 x12 119 / 101, 56^3 x8 118 / 117,
+//   64^3 x4 89 / 77, x8 158 / 151, 72^3 x4 122 / 134: the line is at 512 tiles (64^3);
 //   partly empty tiles (padded / cells): 12^3 (2.4) 168 / 115, 25^3 (2.1) 157 / 154,
-//   33^3 (1.8) 133 / 137, 41^3 (1.6) 116 / 126, 43^3 (1.4) 115 / 117, 37^3 (1.3) 127 / 121:
-//   above 72 tiles at most 1.4.
-constexpr int kIterTiles = 216, kIterAnyFill = 72;
+//   33^3 (1.8) 133 / 137, 41^3 (1.6) 116 / 126, 43^3 (1.4) 115 / 117, 37^3 (1.3) 127 / 121,
+//   52^3 (1.2) 121 / 125, 64x56x60 (1.07) 120 / 125: any up to 72 tiles, at most 1.4 up to
+//   216, at most 1.05 above.
+constexpr int kIterTiles = 512, kIterFillTiles = 216, kIterAnyFill = 72;
 bool one_launch(const mx_operator& op, int mode) {
   if (mode != MX_FP64) return false;
   const long long tiles = iter_blocks(op.nx, op.ny, op.nz);
-  return tiles <= kIterAnyFill || (tiles <= kIterTiles && tiles * kIterTileCells * 10 <= ncell_of(op) * 14);
+  const long long padded = tiles * kIterTileCells * 100, cells = ncell_of(op);
+  return tiles <= kIterAnyFill || (tiles <= kIterFillTiles && padded <= 140 * cells) ||
+         (tiles <= kIterTiles && padded <= 105 * cells);
 }
 // Iterations per chunk of a batch of such systems
 constexpr int kOneLaunchChunk = 32;
@@ -299,7 +303,8 @@ std::vector<BlockMap> xcd_order(const std::vector<BlockMap>& natural) {
 // reps: times a chunk repeats this group's iterations (sessions: equal time per group)
 // ni: blocks of the one-launch iteration (0: a group of three-launch systems)
 // sys0: its first system (batch or slot index)
-struct Group { int a_off, na, v_off, nv, s_off, ns, ty, kind, i_off = 0, ni = 0, sys0 = 0, reps = 1; };
+// lane, lanes: consecutive groups 0 .. lanes - 1 run side by side (split_lanes)
+struct Group { int a_off, na, v_off, nv, s_off, ns, ty, kind, i_off = 0, ni = 0, sys0 = 0, reps = 1, lane = 0, lanes = 1; };
 
 // MALL bytes a launch group may fill (MEANAS_AMD_CACHE_MB overrides; 0: one group)
 size_t cache_budget() {
@@ -324,6 +329,23 @@ size_t mat_hot_bytes(const mx_operator& op, int mode) {
   if (op.flags & MX_MASK) b += n;
   return b;
 }
+
+// The second launch lane (Group::lane) beside a batch's or session's stream; its fork and join.
+struct Lane {
+  hipStream_t stream = nullptr;
+  hipEvent_t fork = nullptr, join = nullptr;
+  hipError_t create() {
+    hipError_t e = hipStreamCreateWithFlags(&stream, hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&fork, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&join, hipEventDisableTiming);
+    return e;
+  }
+  ~Lane() {
+    if (join) (void)hipEventDestroy(join);
+    if (fork) (void)hipEventDestroy(fork);
+    if (stream) (void)hipStreamDestroy(stream);
+  }
+};
 
 struct Batch {
   int mode = MX_MIXED;
@@ -358,6 +380,8 @@ struct Batch {
   SysState* h_state[2] = {nullptr, nullptr};   // pinned, double-buffered polls
   hipStream_t stream = nullptr;                  // library-owned capture stream
   hipEvent_t ev[2] = {nullptr, nullptr};
+  Lane* own_lane = nullptr;
+  const Lane* lane = nullptr;   // null: one lane only (a session's view is given the session's)
   hipGraphExec_t gexec = nullptr;
   hipGraph_t graph = nullptr;
   int graph_chunk = 0;
@@ -383,6 +407,7 @@ struct Batch {
     if (gexec) (void)hipGraphExecDestroy(gexec);
     if (graph) (void)hipGraphDestroy(graph);
     for (auto& e : ev) if (e) (void)hipEventDestroy(e);
+    delete own_lane;
     if (stream) (void)hipStreamDestroy(stream);
     for (auto& h : h_state) if (h) (void)hipHostFree(h);
     if (d_mem) (void)hipFree(d_mem);
@@ -399,13 +424,44 @@ struct Member {
   int na, nv, ni;           // apply and vector blocks; one-launch iteration blocks (0: three launches)
 };
 
+// Two lanes of launches for a group that fills the GPU: half of its systems in each, the two
+// side by side in the chunk's graph, so that one's launches start and drain (4 to 9 us:
+// dispatch, cold lines, write-back) while the other's run.  Results do not change; the split
+// must be even, or one lane is left alone, and a lane's launches must fill the chip half by
+// themselves, since a launch of a forked graph costs more than one of a single chain.
+// Microseconds per iteration, one lane / two:
+//   one-launch systems, from 512 tiles (two per CU): 28^3 x8 27.6 / 23.7, x32 80.0 / 74.8,
+//   48^3 x12 119 / 103, 64^3 x2 44.0 / 39.5, x8 175 / 152; below: 16^3 x16 14.1 / 17.4,
+//   28^3 x2 12.7 / 16.3; uneven (1 : 2): 64x48x56 x3 42.5 / 44.1;
+//   three launches, from 32 MB of p and q: complex64 48^3 x8 89.8 / 85.6, 80^3 x2 89.7 / 86.6,
+//   128^3 x2 225 / 203, complex128 96^3 x2 132 / 126; below: complex64 48^3 x3 53 / 63,
+//   64^3 x2 59.7 / 64.3, 28^3 x2 37 / 62.
+constexpr int kLaneTiles = 512;
+constexpr size_t kLaneBytes = 32u << 20;
+bool split_lanes(const std::vector<const Member*>& held, bool one, int mode, std::vector<int>& lane_of) {
+  long long load[2] = {0, 0};
+  size_t tiles = 0, bytes = 0;
+  std::vector<int> to;
+  for (const Member* m : held) {   // each to the lane with fewer cells so far
+    const int l = load[1] < load[0];
+    load[l] += ncell_of(*m->op);
+    to.push_back(l);
+    tiles += m->ni;
+    bytes += vec_hot_bytes(*m->op, mode, false);
+  }
+  if (one ? tiles < (size_t)kLaneTiles : bytes < kLaneBytes) return false;
+  if (10 * std::max(load[0], load[1]) > 6 * (load[0] + load[1])) return false;
+  lane_of = to;
+  return true;
+}
+
 // Lay `members` out as consecutive launch groups (see Group): one tile height, one
 // material kind and one launch form per group, and within those, consecutive members
 // while their hot bytes fit the cache budget.  Each group's maps are XCD-ordered on their
 // own; apply, vec, iter and sl receive the concatenated maps and system lists.
 void make_groups(const std::vector<Member>& members, int mode, std::vector<BlockMap>& apply,
                  std::vector<BlockMap>& vec, std::vector<BlockMap>& iter, std::vector<int>& sl,
-                 std::vector<Group>& groups) {
+                 std::vector<Group>& groups, bool two_lanes) {
   const size_t budget = cache_budget();
   apply.clear(); vec.clear(); iter.clear(); sl.clear(); groups.clear();
   for (int ty : {2, 4, 8})
@@ -413,37 +469,61 @@ void make_groups(const std::vector<Member>& members, int mode, std::vector<Block
       constexpr int kKinds[4] = {MK_SIMPLE, MK_ANISO, MK_MASK, MK_GENERAL};
       const int kind = kKinds[kind_form / 2];
       const bool one = kind_form % 2 != 0;
-      std::vector<BlockMap> ga, gv, gi;
-      std::vector<int> gs, gops;
+      std::vector<const Member*> held;   // the members of the group being filled
+      std::vector<int> gops;
       size_t bytes = 0;
       auto close = [&]() {
-        if (gs.empty()) return;
-        Group g;
-        g.a_off = (int)apply.size(); g.v_off = (int)vec.size(); g.s_off = (int)sl.size();
-        const std::vector<BlockMap> oa = xcd_order(ga), ov = xcd_order(gv);
-        apply.insert(apply.end(), oa.begin(), oa.end());
-        vec.insert(vec.end(), ov.begin(), ov.end());
-        sl.insert(sl.end(), gs.begin(), gs.end());
-        const std::vector<BlockMap> oi = xcd_order(gi);
-        g.i_off = (int)iter.size();
-        iter.insert(iter.end(), oi.begin(), oi.end());
-        g.na = (int)oa.size(); g.nv = (int)ov.size(); g.ns = (int)gs.size(); g.ni = (int)oi.size();
-        g.ty = ty; g.kind = kind; g.sys0 = gs[0];
-        groups.push_back(g);
-        ga.clear(); gv.clear(); gi.clear(); gs.clear(); gops.clear();
+        if (held.empty()) return;
+        std::vector<int> lane_of(held.size(), 0);
+        const int lanes = two_lanes && split_lanes(held, one, mode, lane_of) ? 2 : 1;
+        for (int l = 0; l < lanes; ++l) {
+          std::vector<BlockMap> ga, gv, gi;
+          Group g{(int)apply.size(), 0, (int)vec.size(), 0, (int)sl.size(), 0, ty, kind};
+          for (size_t i = 0; i < held.size(); ++i) {
+            if (lane_of[i] != l) continue;
+            const Member& m = *held[i];
+            if (g.ns++ == 0) g.sys0 = m.sys;
+            sl.push_back(m.sys);
+            for (int b = 0; b < m.na; ++b) ga.push_back({m.sys, b});
+            for (int b = 0; b < m.nv; ++b) gv.push_back({m.sys, b});
+            for (int b = 0; b < m.ni; ++b) gi.push_back({m.sys, b});
+          }
+          g.lane = l; g.lanes = lanes;
+          g.na = (int)ga.size(); g.nv = (int)gv.size(); g.ni = (int)gi.size();
+          g.i_off = (int)iter.size();
+          auto append = [](std::vector<BlockMap>& to, const std::vector<BlockMap>& natural) {
+            const std::vector<BlockMap> o = xcd_order(natural);
+            to.insert(to.end(), o.begin(), o.end());
+          };
+          append(apply, ga);
+          append(vec, gv);
+          append(iter, gi);
+          groups.push_back(g);
+        }
+        held.clear(); gops.clear();
         bytes = 0;
+      };
+      auto added = [&](const Member& m) {   // hot bytes a member adds to the group
+        const bool new_op = std::find(gops.begin(), gops.end(), m.op_id) == gops.end();
+        return vec_hot_bytes(*m.op, mode, one) + (new_op ? mat_hot_bytes(*m.op, mode) : 0);
+      };
+      auto hold = [&](const Member& m) {
+        bytes += added(m);
+        if (std::find(gops.begin(), gops.end(), m.op_id) == gops.end()) gops.push_back(m.op_id);
+        held.push_back(&m);
       };
       for (const Member& m : members) {
         if (m.ty != ty || m.kind != kind || (m.ni > 0) != one) continue;
-        const bool new_op = std::find(gops.begin(), gops.end(), m.op_id) == gops.end();
-        const size_t add = vec_hot_bytes(*m.op, mode, one) + (new_op ? mat_hot_bytes(*m.op, mode) : 0);
-        if (budget > 0 && !gs.empty() && bytes + add > budget) close();
-        if (std::find(gops.begin(), gops.end(), m.op_id) == gops.end()) gops.push_back(m.op_id);
-        bytes += add;
-        gs.push_back(m.sys);
-        for (int b = 0; b < m.na; ++b) ga.push_back({m.sys, b});
-        for (int b = 0; b < m.nv; ++b) gv.push_back({m.sys, b});
-        for (int b = 0; b < m.ni; ++b) gi.push_back({m.sys, b});
+        if (budget > 0 && !held.empty() && bytes + added(m) > budget) {
+          // one-launch systems: a full group of an odd number leaves its last system to the
+          // next, so that it divides into two lanes (56^3 x8: 3+3+2 128 us, 2+2+2+2 117)
+          const Member* back = two_lanes && one && held.size() > 1 && held.size() % 2 ? held.back() : nullptr;
+          if (back) held.pop_back();
+          close();
+          if (back) hold(*back);
+          if (back && bytes + added(m) > budget) close();
+        }
+        hold(m);
       }
       close();
     }
@@ -459,7 +539,7 @@ int layout_groups(Batch& B, const std::vector<char>& active) {
                          B.h_sys[s].nblk_apply, B.h_sys[s].nblk_vec, B.fused_form ? B.h_sys[s].nblk_iter : 0});
   std::vector<BlockMap> apply, vec, iter;
   std::vector<int> sl;
-  make_groups(members, B.mode, apply, vec, iter, sl, B.groups);
+  make_groups(members, B.mode, apply, vec, iter, sl, B.groups, B.lane != nullptr);
   B.nb_apply0 = (int)apply.size();
   B.nb_vec0 = (int)vec.size();
   B.nsl0 = (int)sl.size();
@@ -548,6 +628,11 @@ int build_batch(Batch& B, const mx_operator* ops, int nops, const mx_system* sys
   MX_TRY(copy_now(B.d_ops32, v32.data(), sizeof(OpView<float>) * nops, hipMemcpyHostToDevice));
   MX_TRY(copy_now(B.d_ops64, v64.data(), sizeof(OpView<double>) * nops, hipMemcpyHostToDevice));
   MX_TRY(copy_now(B.d_sys, B.h_sys.data(), sizeof(SysDesc) * nsys, hipMemcpyHostToDevice));
+  if (o.use_graph && nsys > 1) {   // (launched one by one, a second lane's launches only queue up)
+    B.own_lane = new Lane;
+    MX_TRY(B.own_lane->create());
+    B.lane = B.own_lane;
+  }
   if (layout_groups(B, std::vector<char>(nsys, 1))) return -1;
 
   for (auto& h : B.h_state) MX_TRY(hipHostMalloc(reinterpret_cast<void**>(&h), sizeof(SysState) * nsys, hipHostMallocDefault));
@@ -648,8 +733,18 @@ int enqueue_chunk(Batch& B, hipStream_t s, int iters, int check_every) {
   int rc = 0;
   for (const Group& g : B.groups) {
     B.use_group(g);
-    for (int r = 0; r < g.reps && !rc; ++r) rc = enqueue_group_chunk(B, s, iters, check_every);
+    hipStream_t on = s;
+    if (g.lane == 0 && g.lanes > 1) MX_TRY(hipEventRecord(B.lane->fork, s));
+    if (g.lane > 0) {
+      on = B.lane->stream;
+      MX_TRY(hipStreamWaitEvent(on, B.lane->fork, 0));
+    }
+    for (int r = 0; r < g.reps && !rc; ++r) rc = enqueue_group_chunk(B, on, iters, check_every);
     if (rc) break;
+    if (g.lane > 0) {
+      MX_TRY(hipEventRecord(B.lane->join, on));
+      MX_TRY(hipStreamWaitEvent(s, B.lane->join, 0));
+    }
   }
   B.use_all();
   return rc;
@@ -1348,10 +1443,12 @@ struct mx_session {
   hipGraphExec_t gexec = nullptr;
   hipGraph_t graph = nullptr;
   int graph_iters = 0;
+  Lane* lane = nullptr;                  // the second launch lane (with graphs and more than one slot)
 
   ~mx_session() {
     if (gexec) (void)hipGraphExecDestroy(gexec);
     if (graph) (void)hipGraphDestroy(graph);
+    delete lane;
     if (ev) (void)hipEventDestroy(ev);
     if (stream) (void)hipStreamDestroy(stream);
     if (h_state) (void)hipHostFree(h_state);
@@ -1434,11 +1531,12 @@ void session_group_reps(mx_session* S, const std::vector<int>& sl) {
   double cmax = 0.0;
   for (size_t g = 0; g < S->groups.size(); ++g) {
     const Group& G = S->groups[g];
-    for (int i = 0; i < G.ns; ++i) cost[g] += (double)(S->h_sys[sl[G.s_off + i]].n3 / 3);
-    cmax = std::max(cmax, cost[g]);
+    const size_t first = g - G.lane;   // lanes run side by side: their group's cost, and its repetitions
+    for (int i = 0; i < G.ns; ++i) cost[first] += (double)(S->h_sys[sl[G.s_off + i]].n3 / 3);
+    cmax = std::max(cmax, cost[first]);
   }
   for (size_t g = 0; g < S->groups.size(); ++g)
-    S->groups[g].reps = std::max(1, std::min(kMaxGroupReps, (int)(cmax / cost[g])));
+    S->groups[g].reps = std::max(1, std::min(kMaxGroupReps, (int)(cmax / cost[g - S->groups[g].lane])));
 }
 
 int session_rebuild(mx_session* S) {
@@ -1449,7 +1547,7 @@ int session_rebuild(mx_session* S) {
                          S->h_sys[i].nblk_vec, S->o.form == MX_FORM_FUSED ? S->h_sys[i].nblk_iter : 0});
   std::vector<BlockMap> a, v, it;
   std::vector<int> sl;
-  make_groups(members, S->o.mode, a, v, it, sl, S->groups);
+  make_groups(members, S->o.mode, a, v, it, sl, S->groups, S->lane != nullptr);
   session_group_reps(S, sl);
   S->nsl = (int)sl.size();
   S->nb_apply = (int)a.size();
@@ -1494,6 +1592,10 @@ mx_session* mx_session_create(int32_t capacity, const mx_options* opt) {
   hipError_t e = hipMalloc(&S->d_tab, s32 + s64 + ss + ssl);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&S->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&S->ev, hipEventDisableTiming);
+  if (e == hipSuccess && S->o.use_graph && capacity > 1) {
+    S->lane = new Lane;
+    e = S->lane->create();
+  }
   if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&S->h_state), sizeof(SysState) * capacity, hipHostMallocDefault);
   if (e != hipSuccess) { fail(std::string("mx_session_create: ") + hipGetErrorString(e)); delete S; return nullptr; }
   S->d_ops32 = reinterpret_cast<OpView<float>*>(S->d_tab);
@@ -1599,6 +1701,7 @@ int mx_session_step(mx_session* S, int32_t iterations, void* stream) {
                           S->d_bm + S->nb_apply + S->nb_vec);
   B.host_sys = S->h_sys.data();
   B.host_ops = S->h_ops.data();
+  B.lane = S->lane;
   B.classic_launch = S->o.form != MX_FORM_FUSED;
   B.merged_fin = !B.classic_launch && merged_fin_enabled();
   const int check = std::min<int>(S->o.check_every, iterations);

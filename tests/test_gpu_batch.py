@@ -221,6 +221,39 @@ def test_kept_plans_are_per_thread(rnd):
         assert par[key][1] == seq[key][1], key
 
 
+@pytest.mark.parametrize('method, shape, nrhs', [('fp64', (28, 26, 30), 8),     # one launch, even halves
+                                                 ('fp64', (56, 40, 64), 3),     # full tiles; 1 : 2, not split
+                                                 ('fp64', (56, 40, 64), 5),
+                                                 ('fp64', (33, 33, 33), 11),    # three launches
+                                                 ('mixed', (48, 48, 48), 9)])
+def test_two_launch_lanes_equal_one(method, shape, nrhs):
+    """A batch that fills the GPU runs in two lanes side by side in its captured chunk, and in
+    one where launches are not captured: the same bits, and those of a system alone.  The
+    fields converge to the oracle operator's solution."""
+    import torch
+    from meanas_amd import _lib
+    from meanas_amd.fdfd.device import DeviceOperator, solve_batch
+    mode = _lib.MX_FP64 if method == 'fp64' else _lib.MX_MIXED
+    omega, dxes, eps, Js = small_aniso(shape, nrhs, seed=9)
+    op = DeviceOperator(omega, dxes, eps)
+    bs = [op.map(_lib.MX_MAP_RHS, torch.from_numpy(J).cuda(), coef=-1j * omega) for J in Js]
+
+    def run(some, maxiter, options=None):
+        xs = [torch.zeros_like(bs[k]) for k in some]
+        st = solve_batch([op], [dict(op=0, b=bs[k], x=x, rtol=1e-9, maxiter=maxiter) for k, x in zip(some, xs)],
+                         mode=mode, options=options)
+        return xs, st
+    every = list(range(nrhs))
+    two, st = run(every, 20000)
+    assert all(s['status'] == 'converged' for s in st), st
+    E = op.map(_lib.MX_MAP_E, two[-1]).cpu().numpy()
+    assert physical_residual(omega, dxes, eps, Js[-1], E) < 1e-8
+    one, _ = run(every, 20000, dict(use_graph=0))
+    alone, _ = run([nrhs - 1], 20000)
+    assert all(torch.equal(a, b) for a, b in zip(two, one))
+    assert torch.equal(alone[0], two[-1])
+
+
 def test_uneven_structures_with_pec():
     import torch
     from meanas_amd import _lib, workloads
