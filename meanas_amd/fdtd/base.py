@@ -52,35 +52,49 @@ def _prec(dtype) -> int:
     raise TypeError(f'FDTD fields must be float32 or float64, got {dtype}')
 
 
+def _on_device(f, device) -> torch.Tensor:
+    """The field itself if it is a torch tensor (updated in place), else a device copy."""
+    if isinstance(f, torch.Tensor):
+        if not f.is_cuda or not f.is_contiguous():
+            raise ValueError('torch fields must be contiguous CUDA tensors (updated in place)')
+        t = f
+    else:
+        t = torch.from_numpy(numpy.ascontiguousarray(numpy.asarray(f))).to(device)
+    if t.dim() != 4 or t.shape[0] != 3:
+        raise ValueError('fields must have shape (3, nx, ny, nz)')
+    return t
+
+
+def _written(f, t: torch.Tensor):
+    """The caller's field after an update of its tensor: numpy inputs are written back."""
+    if t is not f:
+        f[...] = t.cpu().numpy()
+    return f
+
+
 class _Field:
     """A field on the device; numpy inputs are written back by `done()`."""
 
     def __init__(self, f, device, dtype=None):
         self.src = f
-        if isinstance(f, torch.Tensor):
-            if not f.is_cuda or not f.is_contiguous():
-                raise ValueError('torch fields must be contiguous CUDA tensors (updated in place)')
-            self.t = f
-        else:
-            a = numpy.asarray(f)
-            self.t = torch.from_numpy(numpy.ascontiguousarray(a)).to(device)
-        if self.t.dim() != 4 or self.t.shape[0] != 3:
-            raise ValueError('fields must have shape (3, nx, ny, nz)')
+        self.t = _on_device(f, device)
 
     def done(self):
-        if not isinstance(self.src, torch.Tensor):
-            self.src[...] = self.t.cpu().numpy()
-        return self.src
+        return _written(self.src, self.t)
 
 
 def _material(m, like: torch.Tensor):
     """(device tensor or None, scalar) for a material that may be a scalar or a field."""
     if m is None:
         return None, 1.0
-    if numpy.isscalar(m) or (isinstance(m, numpy.ndarray) and m.ndim == 0):
+    if isinstance(m, torch.Tensor):
+        t = m
+    elif numpy.isscalar(m) or (isinstance(m, numpy.ndarray) and m.ndim == 0):
         return None, float(m)
-    t = m if isinstance(m, torch.Tensor) else torch.from_numpy(numpy.ascontiguousarray(m))
-    t = t.to(device=like.device, dtype=like.dtype).contiguous()
+    else:
+        t = torch.from_numpy(numpy.ascontiguousarray(m))
+    if t.dtype != like.dtype or t.device != like.device or not t.is_contiguous():
+        t = t.to(device=like.device, dtype=like.dtype).contiguous()
     if t.shape != like.shape:
         raise ValueError('material shape must match the field shape')
     return t, 1.0
@@ -91,17 +105,18 @@ def maxwell_e(dt: float, dxes=None, device: str | torch.device = 'cuda') -> Call
     grids = {}
 
     def me(e, h, epsilon):
-        fe, fh = _Field(e, device), _Field(h, device)
-        shape = tuple(fe.t.shape[1:])
-        if shape not in grids:
-            grids[shape] = _Grid(dxes, shape, device)
-        m, ms = _material(epsilon, fe.t)
-        if fe.t.dtype != fh.t.dtype:
+        te, th = _on_device(e, device), _on_device(h, device)
+        shape = te.shape[1:]
+        grid = grids.get(shape)
+        if grid is None:
+            grid = grids[shape] = _Grid(dxes, tuple(shape), device)
+        m, ms = _material(epsilon, te)
+        if te.dtype != th.dtype:
             raise TypeError('e and h must have the same dtype')
-        _lib.check(_lib.lib().mx_fdtd_e(ctypes.byref(grids[shape].desc), _prec(fe.t.dtype), float(dt), fe.t.data_ptr(),
-                                        fh.t.data_ptr(), m.data_ptr() if m is not None else None, ms,
-                                        torch_stream_handle()), 'mx_fdtd_e')
-        return fe.done()
+        _lib.check(_lib.lib().mx_fdtd_e(ctypes.byref(grid.desc), _prec(te.dtype), float(dt), te.data_ptr(),
+                                     th.data_ptr(), m.data_ptr() if m is not None else None, ms, torch_stream_handle()),
+                   'mx_fdtd_e')
+        return _written(e, te)
     return me
 
 
@@ -110,17 +125,18 @@ def maxwell_h(dt: float, dxes=None, device: str | torch.device = 'cuda') -> Call
     grids = {}
 
     def mh(e, h, mu=None):
-        fe, fh = _Field(e, device), _Field(h, device)
-        shape = tuple(fh.t.shape[1:])
-        if shape not in grids:
-            grids[shape] = _Grid(dxes, shape, device)
-        m, ms = _material(mu, fh.t)
-        if fe.t.dtype != fh.t.dtype:
+        te, th = _on_device(e, device), _on_device(h, device)
+        shape = th.shape[1:]
+        grid = grids.get(shape)
+        if grid is None:
+            grid = grids[shape] = _Grid(dxes, tuple(shape), device)
+        m, ms = _material(mu, th)
+        if te.dtype != th.dtype:
             raise TypeError('e and h must have the same dtype')
-        _lib.check(_lib.lib().mx_fdtd_h(ctypes.byref(grids[shape].desc), _prec(fh.t.dtype), float(dt), fe.t.data_ptr(),
-                                        fh.t.data_ptr(), m.data_ptr() if m is not None else None, ms,
-                                        torch_stream_handle()), 'mx_fdtd_h')
-        return fh.done()
+        _lib.check(_lib.lib().mx_fdtd_h(ctypes.byref(grid.desc), _prec(th.dtype), float(dt), te.data_ptr(),
+                                     th.data_ptr(), m.data_ptr() if m is not None else None, ms, torch_stream_handle()),
+                   'mx_fdtd_h')
+        return _written(h, th)
     return mh
 
 

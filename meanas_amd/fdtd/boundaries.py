@@ -28,7 +28,7 @@ import torch
 
 from .. import _lib
 from ..fdfd.device import torch_stream_handle
-from .base import _Field, _prec
+from .base import _on_device, _prec, _written
 
 
 def conducting_boundary(direction: int, polarity: int, *,
@@ -43,16 +43,21 @@ def conducting_boundary(direction: int, polarity: int, *,
     dev = torch.device(device)
 
     def make(kind: int) -> Callable:
+        grids = {}
+
         def update(f):
-            ff = _Field(f, dev)
-            n = ff.t.shape[1 + direction]
+            t = _on_device(f, dev)
+            shape = t.shape[1:]
+            n = shape[direction]
             if n < (2 if pol < 0 else 3):
                 raise IndexError(f'axis {direction} has {n} cells; the face needs {2 if pol < 0 else 3}')
-            grid = _lib.MxFdtdGrid(*ff.t.shape[1:], 0, (ctypes.c_void_p * 3)(), (ctypes.c_void_p * 3)())
-            _lib.check(_lib.lib().mx_fdtd_conducting_boundary(ctypes.byref(grid), _prec(ff.t.dtype), direction, pol,
-                                                              kind, ff.t.data_ptr(), torch_stream_handle()),
+            grid = grids.get(shape)
+            if grid is None:
+                grid = grids[shape] = _lib.MxFdtdGrid(*shape, 0, (ctypes.c_void_p * 3)(), (ctypes.c_void_p * 3)())
+            _lib.check(_lib.lib().mx_fdtd_conducting_boundary(ctypes.byref(grid), _prec(t.dtype), direction, pol, kind,
+                                                              t.data_ptr(), torch_stream_handle()),
                        'mx_fdtd_conducting_boundary')
-            return ff.done()
+            return _written(f, t)
         return update
 
     return make(_lib.MX_FIELD_E), make(_lib.MX_FIELD_H)

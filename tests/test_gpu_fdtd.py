@@ -470,3 +470,21 @@ def test_planes_beyond_32_bit_offsets(name):
         z = torch.roll(x, 1, 1)
         want = torch.stack([(x[2] - y[2]) - (x[1] - z[1]), x[0] - z[0], -(x[0] - y[0])]) * 0.125
         torch.testing.assert_close(out[:, 0, j], want, rtol=1e-13, atol=1e-13)
+
+
+def test_calls_go_to_the_current_stream():
+    """The stream handle of a call is the current stream's: the default one, a side stream, and
+    the default one again; an explicit stream is taken as it is."""
+    import torch
+    from meanas_amd.fdfd.device import torch_stream_handle
+    side = torch.cuda.Stream()
+    default = torch.cuda.current_stream().cuda_stream
+
+    def handle(*args):
+        return torch_stream_handle(*args).value or 0
+    assert handle() == default
+    with torch.cuda.stream(side):
+        assert handle() == side.cuda_stream
+        assert handle(torch.cuda.default_stream()) == torch.cuda.default_stream().cuda_stream
+    assert handle() == default
+    assert handle(side) == side.cuda_stream
