@@ -11,6 +11,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <string>
+#include <type_traits>
 
 #include "common.hpp"
 #include "../../include/meanas_fdfd.h"
@@ -216,24 +217,27 @@ __device__ __forceinline__ int wrap(int v, int n) {
 // so a run equals the step-by-step updates bit for bit.
 //
 // Bound by the divisions' issue (58% of the time at 256^3 in float64) together with the
-// reads, 1.36 times the algorithmic ones with the halos.  Per step of a run (in brackets
-// with passes of one step and compiler divides): 256^3 float64 281 us (435), 256^3 float32
-// 148 us (266), 190 x 160 x 201 float32 57 us (129).  12 rows: 8 rows recompute half of
-// theirs (330 / 170 us at 256^3), 16 rows leave float64 128 VGPRs of the 142 it needs
-// (396 / 155 us).  Three steps a pass spill in float64 and gain nothing in float32 (159
-// us), since the halo grows with each.  Two rows per thread measured 285 / 161 us.
-constexpr int kStepRows = 12;
-constexpr int kStepMaxSlab = 128;
+// reads, 1.36 times the algorithmic ones with the halos.  In float32 the rows that a stage
+// does not need are left out (a row is a wave: 38 of 48 row stages remain, 2 to 4 %; float64
+// spills with it).  Per step of a run (in brackets with passes of one step and compiler
+// divides): 256^3 float64 275 us (435), 256^3 float32 148 us (266), 190 x 160 x 201 float32
+// 56 us (129).  12 or 14 rows (step_shape): 8 rows recompute half of theirs (330 / 170 us at
+// 256^3), 16 rows leave float64 128 VGPRs of the 142 it needs (396 / 155 us).  Three steps a
+// pass spill in float64 and gain nothing in float32 (159 us), since the halo grows with each.
+// Two rows per thread measured 285 / 161 us.
+constexpr int kStepRows = 12, kStepRowsMore = 14;   // (14 in float32 only)
+constexpr int kStepMaxSlab = 128, kStepMinSlab = 4;
 constexpr int kStepTab = 136;    // planes of the x table: the slab and the pipeline's run-in
 enum : int { MU_ONE = 0, MU_SCALAR = 1, MU_FIELD = 2 };
 
-template <typename T, int S, bool EPS, int MU>
-__global__ __launch_bounds__(64 * kStepRows) void k_fdtd_steps(RGrid g, T dt, const T* __restrict__ e0,
+template <typename T, int W, int S, bool EPS, int MU>
+__global__ __launch_bounds__(64 * W) void k_fdtd_steps(RGrid g, T dt, const T* __restrict__ e0,
                                                                const T* __restrict__ h0, T* __restrict__ e1,
                                                                T* __restrict__ h1, const T* __restrict__ eps,
                                                                T eps_s, const T* __restrict__ mu, T mu_s, int slab) {
 #pragma clang fp contract(off)
-  constexpr int W = kStepRows, OY = W - 2 * S, OZ = 64 - 2 * S;
+  constexpr int OY = W - 2 * S, OZ = 64 - 2 * S;
+  constexpr bool kSkip = sizeof(T) == 4;
   __shared__ T sE[S][2][W + 1][64];   // E_{s-1} x, z by row
   __shared__ T sH[S][2][W + 1][64];   // H_s x, z by row + 1
   __shared__ T sX[kStepTab][4];       // dx_e, 1 / dx_e, dx_h, 1 / dx_h by plane
@@ -329,7 +333,7 @@ __global__ __launch_bounds__(64 * kStepRows) void k_fdtd_steps(RGrid g, T dt, co
   auto step = [&](const int t, In& cur, In& nxt) {
     fetch(nxt);
     // phase 1
-    T hs[S][3];
+    T hs[S][3] = {};
     if constexpr (MU == MU_FIELD) {
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
@@ -339,6 +343,7 @@ __global__ __launch_bounds__(64 * kStepRows) void k_fdtd_steps(RGrid g, T dt, co
     }
 #pragma unroll
     for (int s = 0; s < S; ++s) {
+      if (kSkip && (ty < s || ty > W - 2 - s)) continue;   // (uniform in a wave)
       const T* xt = sX[t + kLag - 2 * s];
       const T dx = xt[0], rx = xt[1];
       const T (&ec)[3] = Ec[s];
@@ -361,7 +366,7 @@ __global__ __launch_bounds__(64 * kStepRows) void k_fdtd_steps(RGrid g, T dt, co
     }
     __syncthreads();
     // phase 2
-    T es[S][3];
+    T es[S][3] = {};
     if constexpr (EPS) {
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
@@ -371,6 +376,7 @@ __global__ __launch_bounds__(64 * kStepRows) void k_fdtd_steps(RGrid g, T dt, co
     }
 #pragma unroll
     for (int s = 0; s < S; ++s) {
+      if (kSkip && (ty < s + 1 || ty > W - 2 - s)) continue;
       const T* xt = sX[t + kLag - 2 * s];
       const T dx = xt[2], rx = xt[3];
       const T hx = hs[s][0], hy = hs[s][1], hz = hs[s][2];
@@ -917,29 +923,45 @@ hipError_t launch_cpml(const RGrid& v, int prec, int psi_prec, double dt, const 
   return hipGetLastError();
 }
 
-// Slab depth of a pass: the one with the least modelled time.  A block takes slab + 3 S - 2
-// iterations; per iteration the n blocks that a CU gets (256 CUs) cost n, plus a fifth of
-// one where two blocks share it (float32) that a lone block cannot hide.  Measured at
-// 256^3 float64, two steps: slabs 16/24/32/48/64/128 model 200/196/180/208/204/264, time
-// 611/576/542/595/572/696 us.
-int step_slab(const RGrid& v, int steps, size_t elem) {
+struct StepShape { int rows, slab; };
+long long step_tiles(const RGrid& v, int rows, int steps) {
+  const int oy = rows - 2 * steps, oz = 64 - 2 * steps;
+  return (long long)((v.ny + oy - 1) / oy) * ((v.nz + oz - 1) / oz);
+}
+
+// Rows and slab depth of a pass: those with the least modelled time, over all equal divisions
+// of x.  A block takes slab + 3 S - 2 iterations, each as long as its rows are many; the n
+// blocks that a CU gets (256 CUs) cost n, plus a fifth of one in float32, where two blocks
+// share a CU.  Measured at 256^3 float64, two steps: slabs 16/24/32/48/64/128 model
+// 200/196/180/208/204/264, time 611/576/542/595/572/696 us.  Float32 with 14 rows instead of
+// 12, model / time: 100^3 1.17 / 1.13, 150x141x130 0.82 / 0.85, 320^3 0.94 / 0.88, 256^3 1.15 /
+// 1.02 (float64 has no registers for 14).  Against 12 rows and slabs of powers of two and
+// three halves of them, us per step: float32 150x141x130 with mu 45 / 39, 320^3 309 / 256,
+// 64x150x250 with mu 38 / 31, float64 150x141x130 with mu 114 / 89, 190x160x201 123 / 111;
+// 256^3, 60^3 and 100^3 alike.
+StepShape step_shape(const RGrid& v, int steps, size_t elem) {
   static const int forced = [] {   // MEANAS_AMD_FDTD_SLAB overrides the slab depth (tuning runs)
     const char* env = getenv("MEANAS_AMD_FDTD_SLAB");
     return env ? atoi(env) : 0;
   }();
-  if (forced > 0) return std::min(std::min(forced, kStepMaxSlab), v.nx);
-  const long long tiles = (long long)((v.ny + kStepRows - 2 * steps - 1) / (kStepRows - 2 * steps)) *
-                          ((v.nz + 63 - 2 * steps) / (64 - 2 * steps));
-  int best = 1;
+  StepShape best{0, 0};
   double best_cost = 0.0;
-  for (int want : {4, 6, 8, 12, 16, 24, 32, 48, 64, 96, kStepMaxSlab}) {
-    const int slab = std::min(want, v.nx);
-    const long long blocks = tiles * ((v.nx + slab - 1) / slab);
-    const double n = (double)((blocks + 255) / 256) + (elem == 4 ? 0.2 : 0.0);
-    const double cost = n * (slab + 3 * steps - 2);
-    if (best_cost == 0.0 || cost < best_cost) {
-      best_cost = cost;
-      best = slab;
+  for (int rows : {kStepRows, kStepRowsMore}) {
+    if (rows > kStepRows && elem != 4) continue;
+    const long long tiles = step_tiles(v, rows, steps);
+    int last = 0;
+    for (int count = (v.nx + kStepMaxSlab - 1) / kStepMaxSlab; count <= v.nx; ++count) {
+      const int slab = forced > 0 ? std::min(std::min(forced, kStepMaxSlab), v.nx) : (v.nx + count - 1) / count;
+      if (slab == last) continue;
+      if (slab < kStepMinSlab && last > 0) break;
+      last = slab;
+      const long long blocks = tiles * ((v.nx + slab - 1) / slab);
+      const double n = (double)((blocks + 255) / 256) + (elem == 4 ? 0.2 : 0.0);
+      const double cost = n * (slab + 3 * steps - 2) * rows;
+      if (best.slab == 0 || cost < best_cost) {
+        best_cost = cost;
+        best = {rows, slab};
+      }
     }
   }
   return best;
@@ -949,17 +971,25 @@ template <typename T, int S>
 hipError_t launch_pass(const RGrid& v, T dt, const void* ei, const void* hi, void* eo, void* ho, const void* eps,
                        double eps_s, const void* mu, double mu_s, hipStream_t s) {
   static_assert(kStepMaxSlab + 5 * S - 4 <= kStepTab, "x table");
-  const int slab = step_slab(v, S, sizeof(T));
-  const long long tiles =
-      (long long)((v.ny + kStepRows - 2 * S - 1) / (kStepRows - 2 * S)) * ((v.nz + 63 - 2 * S) / (64 - 2 * S));
-  const long long nwork = tiles * ((v.nx + slab - 1) / slab);
+  const StepShape shape = step_shape(v, S, sizeof(T));
+  const int slab = shape.slab;
+  const long long nwork = step_tiles(v, shape.rows, S) * ((v.nx + slab - 1) / slab);
   const unsigned nb = (unsigned)(((nwork + 7) / 8) * 8);
 #define MX_STEP_CASE(EPS, MU)                                                                                   \
-  hipLaunchKernelGGL((k_fdtd_steps<T, S, EPS, MU>), dim3(nb), dim3(64, kStepRows), 0, s, v, dt, (const T*)ei,   \
+  hipLaunchKernelGGL((k_fdtd_steps<T, W, S, EPS, MU>), dim3(nb), dim3(64, W), 0, s, v, dt, (const T*)ei,        \
                      (const T*)hi, (T*)eo, (T*)ho, (const T*)eps, (T)eps_s, (const T*)mu, (T)mu_s, slab)
-  if (mu) { if (eps) MX_STEP_CASE(true, MU_FIELD); else MX_STEP_CASE(false, MU_FIELD); }
-  else if (mu_s == 1.0) { if (eps) MX_STEP_CASE(true, MU_ONE); else MX_STEP_CASE(false, MU_ONE); }
-  else { if (eps) MX_STEP_CASE(true, MU_SCALAR); else MX_STEP_CASE(false, MU_SCALAR); }
+  auto go = [&](auto rows) {
+    constexpr int W = decltype(rows)::value;
+    if (mu) { if (eps) MX_STEP_CASE(true, MU_FIELD); else MX_STEP_CASE(false, MU_FIELD); }
+    else if (mu_s == 1.0) { if (eps) MX_STEP_CASE(true, MU_ONE); else MX_STEP_CASE(false, MU_ONE); }
+    else { if (eps) MX_STEP_CASE(true, MU_SCALAR); else MX_STEP_CASE(false, MU_SCALAR); }
+  };
+  if constexpr (sizeof(T) == 4) {
+    if (shape.rows == kStepRowsMore) go(std::integral_constant<int, kStepRowsMore>());
+    else go(std::integral_constant<int, kStepRows>());
+  } else {
+    go(std::integral_constant<int, kStepRows>());
+  }
 #undef MX_STEP_CASE
   return hipGetLastError();
 }

@@ -90,6 +90,27 @@ def test_run_passes_at_tile_edges(shape, eps_kind, mu_kind, dtype, steps):
     assert torch.equal(et, e2) and torch.equal(ht, h2)
 
 
+@pytest.mark.parametrize('shape', [(326, 9, 61), (326, 10, 61), (214, 19, 61)])
+@pytest.mark.parametrize('mu_kind', [None, 'field'])
+@pytest.mark.parametrize('steps', [1, 4])
+def test_float32_runs_in_blocks_of_14_rows(shape, mu_kind, steps):
+    """Long thin float32 grids, where blocks of 14 rows (10 stored by a pass of two steps) fit
+    the chip better than those of 12: 9, 10 and 19 rows, a last slab shorter than the others,
+    against the separate updates bit for bit."""
+    from meanas_amd import fdtd
+    e, h, eps, mu, dxes = _fields(shape, 4, numpy.float32)
+    mu = mu if mu_kind == 'field' else None
+    dt = 0.2
+    et, ht = torch.from_numpy(e.copy()).cuda(), torch.from_numpy(h.copy()).cuda()
+    fdtd.run(et, ht, eps, dt, dxes, steps=steps, mu=mu)
+    me, mh = fdtd.maxwell_e(dt, dxes), fdtd.maxwell_h(dt, dxes)
+    e2, h2 = torch.from_numpy(e.copy()).cuda(), torch.from_numpy(h.copy()).cuda()
+    for _ in range(steps):
+        mh(e2, h2, mu)
+        me(e2, h2, eps)
+    assert torch.equal(et, e2) and torch.equal(ht, h2)
+
+
 @pytest.mark.parametrize('dtype', [numpy.float64, numpy.float32])
 def test_updates_keep_infinities_zeros_and_nan(dtype):
     """Infinite fields and materials, zero and NaN values divide as numpy divides them."""
