@@ -157,15 +157,18 @@ int op_kind(const mx_operator& op) { return mat_kind(view_of<double>(op).flags);
 //   64^3 x4 89 / 77, x8 158 / 151, 72^3 x4 122 / 134: the line is at 512 tiles (64^3);
 //   partly empty tiles (padded / cells): 12^3 (2.4) 168 / 115, 25^3 (2.1) 157 / 154,
 //   33^3 (1.8) 133 / 137, 41^3 (1.6) 116 / 126, 43^3 (1.4) 115 / 117, 37^3 (1.3) 127 / 121,
-//   52^3 (1.2) 121 / 125, 64x56x60 (1.07) 120 / 125: any up to 72 tiles, at most 1.4 up to
-//   216, at most 1.05 above.
+//   52^3 (1.2) 121 / 125, 61^3 (1.15) 144 / 150, 63^3 (1.05) 152 / 159: any up to 72 tiles, at
+//   most 1.4 up to 216, at most 1.04 above.
+// What that line gives away: alone 60^3 would take 22 us instead of 39, 52^3 21 instead of 33.
+// What it costs: an odd batch of 5 or more near the upper line ends with a group of one
+// system (48x48x95 x9 168 / 177, 64^3 x7 139 / 138, x5 107 / 101).
 constexpr int kIterTiles = 512, kIterFillTiles = 216, kIterAnyFill = 72;
 bool one_launch(const mx_operator& op, int mode) {
   if (mode != MX_FP64) return false;
   const long long tiles = iter_blocks(op.nx, op.ny, op.nz);
   const long long padded = tiles * kIterTileCells * 100, cells = ncell_of(op);
   return tiles <= kIterAnyFill || (tiles <= kIterFillTiles && padded <= 140 * cells) ||
-         (tiles <= kIterTiles && padded <= 105 * cells);
+         (tiles <= kIterTiles && padded <= 104 * cells);
 }
 // Iterations per chunk of a batch of such systems
 constexpr int kOneLaunchChunk = 32;
