@@ -510,23 +510,26 @@ void make_groups(const std::vector<Member>& members, int mode, std::vector<Block
         const bool new_op = std::find(gops.begin(), gops.end(), m.op_id) == gops.end();
         return vec_hot_bytes(*m.op, mode, one) + (new_op ? mat_hot_bytes(*m.op, mode) : 0);
       };
-      auto hold = [&](const Member& m) {
-        bytes += added(m);
+      auto hold = [&](const Member& m, size_t add) {
+        bytes += add;
         if (std::find(gops.begin(), gops.end(), m.op_id) == gops.end()) gops.push_back(m.op_id);
         held.push_back(&m);
       };
       for (const Member& m : members) {
         if (m.ty != ty || m.kind != kind || (m.ni > 0) != one) continue;
-        if (budget > 0 && !held.empty() && bytes + added(m) > budget) {
+        // three launches: a structure's materials count in the first of its groups only (two
+        // systems of 128x96x96 with materials fill 243 MB: 85 us each together, 94 alone)
+        const size_t add = added(m);
+        if (budget > 0 && !held.empty() && bytes + add > budget) {
           // one-launch systems: a full group of an odd number leaves its last system to the
           // next, so that it divides into two lanes (56^3 x8: 3+3+2 128 us, 2+2+2+2 117)
           const Member* back = two_lanes && one && held.size() > 1 && held.size() % 2 ? held.back() : nullptr;
           if (back) held.pop_back();
           close();
-          if (back) hold(*back);
+          if (back) hold(*back, added(*back));
           if (back && bytes + added(m) > budget) close();
         }
-        hold(m);
+        hold(m, one ? added(m) : add);
       }
       close();
     }
