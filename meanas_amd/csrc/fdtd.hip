@@ -213,7 +213,7 @@ __device__ __forceinline__ int wrap(int v, int n) {
 // loaded one iteration ahead into alternating register sets, so nothing waits for a load
 // in the iteration that issues it.  Only the last stage is stored, by the lanes and rows
 // that are not halo: each stage's fields are valid one cell further in than those of the
-// stage before.  The expressions are those of k_fdtd_h and k_fdtd_e without contraction,
+// stage before.  The expressions are those of k_fdtd_update without contraction,
 // so a run equals the step-by-step updates bit for bit.
 //
 // Bound by the divisions' issue (58% of the time at 256^3 in float64) together with the
