@@ -333,20 +333,24 @@ size_t mat_hot_bytes(const mx_operator& op, int mode) {
   return b;
 }
 
-// The second launch lane (Group::lane) beside a batch's or session's stream; its fork and join.
-struct Lane {
-  hipStream_t stream = nullptr;
-  hipEvent_t fork = nullptr, join = nullptr;
+// The further launch lanes (Group::lane) beside a batch's or session's stream; their fork and
+// joins.
+constexpr int kMaxLanes = 3;
+struct Lanes {
+  hipStream_t stream[kMaxLanes - 1] = {};
+  hipEvent_t fork = nullptr, join[kMaxLanes - 1] = {};
   hipError_t create() {
-    hipError_t e = hipStreamCreateWithFlags(&stream, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&fork, hipEventDisableTiming);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&join, hipEventDisableTiming);
+    hipError_t e = hipEventCreateWithFlags(&fork, hipEventDisableTiming);
+    for (int l = 0; l < kMaxLanes - 1 && e == hipSuccess; ++l) {
+      e = hipStreamCreateWithFlags(&stream[l], hipStreamNonBlocking);
+      if (e == hipSuccess) e = hipEventCreateWithFlags(&join[l], hipEventDisableTiming);
+    }
     return e;
   }
-  ~Lane() {
-    if (join) (void)hipEventDestroy(join);
+  ~Lanes() {
+    for (hipEvent_t e : join) if (e) (void)hipEventDestroy(e);
+    for (hipStream_t t : stream) if (t) (void)hipStreamDestroy(t);
     if (fork) (void)hipEventDestroy(fork);
-    if (stream) (void)hipStreamDestroy(stream);
   }
 };
 
@@ -383,8 +387,8 @@ struct Batch {
   SysState* h_state[2] = {nullptr, nullptr};   // pinned, double-buffered polls
   hipStream_t stream = nullptr;                  // library-owned capture stream
   hipEvent_t ev[2] = {nullptr, nullptr};
-  Lane* own_lane = nullptr;
-  const Lane* lane = nullptr;   // null: one lane only (a session's view is given the session's)
+  Lanes* own_lane = nullptr;
+  const Lanes* lane = nullptr;   // null: one lane only (a session's view is given the session's)
   hipGraphExec_t gexec = nullptr;
   hipGraph_t graph = nullptr;
   int graph_chunk = 0;
@@ -427,7 +431,7 @@ struct Member {
   int na, nv, ni;           // apply and vector blocks; one-launch iteration blocks (0: three launches)
 };
 
-// Two lanes of launches for a group that fills the GPU: half of its systems in each, the two
+// Lanes of launches for a group that fills the GPU: half of its systems in each of two, the two
 // side by side in the chunk's graph, so that one's launches start and drain (4 to 9 us:
 // dispatch, cold lines, write-back) while the other's run.  Results do not change; the split
 // must be even, or one lane is left alone, and a lane's launches must fill the chip half by
@@ -435,13 +439,14 @@ struct Member {
 // Microseconds per iteration, one lane / two:
 //   one-launch systems, from 512 tiles (two per CU): 28^3 x8 27.6 / 23.7, x32 80.0 / 74.8,
 //   48^3 x12 119 / 103, 64^3 x2 44.0 / 39.5, x8 175 / 152; below: 16^3 x16 14.1 / 17.4,
-//   28^3 x2 12.7 / 16.3; uneven (1 : 2): 64x48x56 x3 42.5 / 44.1;
+//   28^3 x2 12.7 / 16.3; uneven (1 : 2): 64x48x56 x3 42.5 / 44.1, in three lanes 39.9
+//   (48^3 x3 32.0 / 29.9, 56^3 x3 48.3 / 43.0, 64^3 x3 alike), so three of about one size take three;
 //   three launches, from 32 MB of p and q: complex64 48^3 x8 89.8 / 85.6, 80^3 x2 89.7 / 86.6,
 //   128^3 x2 225 / 203, complex128 96^3 x2 132 / 126; below: complex64 48^3 x3 53 / 63,
 //   64^3 x2 59.7 / 64.3, 28^3 x2 37 / 62.
 constexpr int kLaneTiles = 512;
 constexpr size_t kLaneBytes = 32u << 20;
-bool split_lanes(const std::vector<const Member*>& held, bool one, int mode, std::vector<int>& lane_of) {
+int split_lanes(const std::vector<const Member*>& held, bool one, int mode, std::vector<int>& lane_of) {
   long long load[2] = {0, 0};
   size_t tiles = 0, bytes = 0;
   std::vector<int> to;
@@ -452,10 +457,16 @@ bool split_lanes(const std::vector<const Member*>& held, bool one, int mode, std
     tiles += m->ni;
     bytes += vec_hot_bytes(*m->op, mode, false);
   }
-  if (one ? tiles < (size_t)kLaneTiles : bytes < kLaneBytes) return false;
-  if (10 * std::max(load[0], load[1]) > 6 * (load[0] + load[1])) return false;
+  if (one ? tiles < (size_t)kLaneTiles : bytes < kLaneBytes) return 1;
+  long long most = 0;
+  for (const Member* m : held) most = std::max<long long>(most, ncell_of(*m->op));
+  if (one && held.size() == 3 && 5 * most <= 2 * (load[0] + load[1])) {
+    lane_of = {0, 1, 2};
+    return 3;
+  }
+  if (10 * std::max(load[0], load[1]) > 6 * (load[0] + load[1])) return 1;
   lane_of = to;
-  return true;
+  return 2;
 }
 
 // Lay `members` out as consecutive launch groups (see Group): one tile height, one
@@ -464,7 +475,7 @@ bool split_lanes(const std::vector<const Member*>& held, bool one, int mode, std
 // own; apply, vec, iter and sl receive the concatenated maps and system lists.
 void make_groups(const std::vector<Member>& members, int mode, std::vector<BlockMap>& apply,
                  std::vector<BlockMap>& vec, std::vector<BlockMap>& iter, std::vector<int>& sl,
-                 std::vector<Group>& groups, bool two_lanes) {
+                 std::vector<Group>& groups, bool with_lanes) {
   const size_t budget = cache_budget();
   apply.clear(); vec.clear(); iter.clear(); sl.clear(); groups.clear();
   for (int ty : {2, 4, 8})
@@ -478,7 +489,7 @@ void make_groups(const std::vector<Member>& members, int mode, std::vector<Block
       auto close = [&]() {
         if (held.empty()) return;
         std::vector<int> lane_of(held.size(), 0);
-        const int lanes = two_lanes && split_lanes(held, one, mode, lane_of) ? 2 : 1;
+        const int lanes = with_lanes ? split_lanes(held, one, mode, lane_of) : 1;
         for (int l = 0; l < lanes; ++l) {
           std::vector<BlockMap> ga, gv, gi;
           Group g{(int)apply.size(), 0, (int)vec.size(), 0, (int)sl.size(), 0, ty, kind};
@@ -523,7 +534,7 @@ void make_groups(const std::vector<Member>& members, int mode, std::vector<Block
         if (budget > 0 && !held.empty() && bytes + add > budget) {
           // one-launch systems: a full group of an odd number leaves its last system to the
           // next, so that it divides into two lanes (56^3 x8: 3+3+2 128 us, 2+2+2+2 117)
-          const Member* back = two_lanes && one && held.size() > 1 && held.size() % 2 ? held.back() : nullptr;
+          const Member* back = with_lanes && one && held.size() > 1 && held.size() % 2 ? held.back() : nullptr;
           if (back) held.pop_back();
           close();
           if (back) hold(*back, added(*back));
@@ -635,7 +646,7 @@ int build_batch(Batch& B, const mx_operator* ops, int nops, const mx_system* sys
   MX_TRY(copy_now(B.d_ops64, v64.data(), sizeof(OpView<double>) * nops, hipMemcpyHostToDevice));
   MX_TRY(copy_now(B.d_sys, B.h_sys.data(), sizeof(SysDesc) * nsys, hipMemcpyHostToDevice));
   if (o.use_graph && nsys > 1) {   // (launched one by one, a second lane's launches only queue up)
-    B.own_lane = new Lane;
+    B.own_lane = new Lanes;
     MX_TRY(B.own_lane->create());
     B.lane = B.own_lane;
   }
@@ -742,15 +753,13 @@ int enqueue_chunk(Batch& B, hipStream_t s, int iters, int check_every) {
     hipStream_t on = s;
     if (g.lane == 0 && g.lanes > 1) MX_TRY(hipEventRecord(B.lane->fork, s));
     if (g.lane > 0) {
-      on = B.lane->stream;
+      on = B.lane->stream[g.lane - 1];
       MX_TRY(hipStreamWaitEvent(on, B.lane->fork, 0));
     }
     for (int r = 0; r < g.reps && !rc; ++r) rc = enqueue_group_chunk(B, on, iters, check_every);
     if (rc) break;
-    if (g.lane > 0) {
-      MX_TRY(hipEventRecord(B.lane->join, on));
-      MX_TRY(hipStreamWaitEvent(s, B.lane->join, 0));
-    }
+    if (g.lane > 0) MX_TRY(hipEventRecord(B.lane->join[g.lane - 1], on));
+    for (int l = 1; l < g.lanes && g.lane + 1 == g.lanes; ++l) MX_TRY(hipStreamWaitEvent(s, B.lane->join[l - 1], 0));
   }
   B.use_all();
   return rc;
@@ -1449,7 +1458,7 @@ struct mx_session {
   hipGraphExec_t gexec = nullptr;
   hipGraph_t graph = nullptr;
   int graph_iters = 0;
-  Lane* lane = nullptr;                  // the second launch lane (with graphs and more than one slot)
+  Lanes* lane = nullptr;                 // the further launch lanes (with graphs and more than one slot)
 
   ~mx_session() {
     if (gexec) (void)hipGraphExecDestroy(gexec);
@@ -1599,7 +1608,7 @@ mx_session* mx_session_create(int32_t capacity, const mx_options* opt) {
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&S->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipEventCreateWithFlags(&S->ev, hipEventDisableTiming);
   if (e == hipSuccess && S->o.use_graph && capacity > 1) {
-    S->lane = new Lane;
+    S->lane = new Lanes;
     e = S->lane->create();
   }
   if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&S->h_state), sizeof(SysState) * capacity, hipHostMallocDefault);

@@ -222,12 +222,12 @@ def test_kept_plans_are_per_thread(rnd):
 
 
 @pytest.mark.parametrize('method, shape, nrhs', [('fp64', (28, 26, 30), 8),     # one launch, even halves
-                                                 ('fp64', (56, 40, 64), 3),     # full tiles; 1 : 2, not split
+                                                 ('fp64', (56, 40, 64), 3),     # full tiles; a lane each
                                                  ('fp64', (56, 40, 64), 5),
                                                  ('fp64', (33, 33, 33), 11),    # three launches
                                                  ('mixed', (48, 48, 48), 9)])
-def test_two_launch_lanes_equal_one(method, shape, nrhs):
-    """A batch that fills the GPU runs in two lanes side by side in its captured chunk, and in
+def test_launch_lanes_equal_one(method, shape, nrhs):
+    """A batch that fills the GPU runs in two or three lanes side by side in its captured chunk, and in
     one where launches are not captured: the same bits, and those of a system alone.  The
     fields converge to the oracle operator's solution."""
     import torch
