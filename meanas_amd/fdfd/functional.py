@@ -71,10 +71,16 @@ class _Grid:
         self.n3 = 3 * nx * ny * nz
 
 
+def _flat(f: torch.Tensor, device) -> torch.Tensor:
+    """f as a flat complex128 tensor whose memory holds its values: kernels read it by
+    pointer, so a lazy conjugation or negation (`f.conj()`) is carried out here."""
+    return f.to(device=device, dtype=torch.complex128).reshape(-1).contiguous().resolve_conj().resolve_neg()
+
+
 def _to_device(f, grid: _Grid, name: str) -> tuple[torch.Tensor, object]:
     """(flat complex128 device tensor, how to shape the result like the input)."""
     if isinstance(f, torch.Tensor):
-        t = f.to(device=grid.device, dtype=torch.complex128).reshape(-1).contiguous()
+        t = _flat(f, grid.device)
         like = ('torch', tuple(f.shape))
     else:
         a = numpy.asarray(f)
@@ -259,7 +265,7 @@ class _A0:
 
 def _dev_field(f, op: DeviceOperator):
     if isinstance(f, torch.Tensor):
-        t = f.to(device=op.device, dtype=torch.complex128).reshape(-1).contiguous()
+        t = _flat(f, op.device)
         like = ('torch', tuple(f.shape))
     else:
         a = numpy.asarray(f)

@@ -26,7 +26,7 @@ import torch
 
 from .. import _lib
 from .device import DeviceOperator, grid_shape, torch_stream_handle
-from .functional import _Grid
+from .functional import _flat, _Grid
 
 
 def _field_mask(mask, n3: int, ncell: int) -> numpy.ndarray:
@@ -45,7 +45,7 @@ def _field_mask(mask, n3: int, ncell: int) -> numpy.ndarray:
 
 def _to_dev(e, op: DeviceOperator) -> tuple[torch.Tensor, object]:
     if isinstance(e, torch.Tensor):
-        t = e.to(device=op.device, dtype=torch.complex128).reshape(-1).contiguous().resolve_conj()
+        t = _flat(e, op.device)
         like = ('torch', tuple(e.shape))
     else:
         a = numpy.asarray(e)
