@@ -807,7 +807,8 @@ ColumnGrid column_grid(const RGrid& v) {
   const long long nwork = pieces * ((v.nx + slab - 1) / slab);
   return {slab, (unsigned)((nwork + 7) / 8 * 8)};
 }
-// whether the byte offsets of a plane fit 32 bits (beyond: kernels with 64-bit offsets)
+// whether the byte offsets of a plane fit 32 bits (beyond: kernels with 64-bit offsets);
+// `prec` is the widest type that the kernel holds a value per cell of
 bool small_plane(const RGrid& v, int prec) {
   return (unsigned long long)v.ny * v.nz * (prec == MX_REAL64 ? 8 : 4) < (1ull << 32);
 }
@@ -911,13 +912,15 @@ hipError_t launch_cpml(const RGrid& v, int prec, int psi_prec, double dt, const 
 #define MX_CPML_CASE(T, TP, OFF)                                                                              \
   hipLaunchKernelGGL((k_cpml<T, TP, EUPD, OFF>), dim3(cg.blocks), dim3(kFB), 0, s, v, (T)dt, (const T*)f, (T*)out, \
                      (const T*)mat, dt / mat_s, tab, cg.slab)
-  const bool small = small_plane(v, prec);
+  // a layer's plane has at most the grid plane's cells, in the psi precision
+  const bool small = small_plane(v, prec == MX_REAL64 ? prec : psi_prec);
   if (prec == MX_REAL64) {
     if (psi_prec == MX_REAL64) { if (small) MX_CPML_CASE(double, double, unsigned); else MX_CPML_CASE(double, double, size_t); }
     else { if (small) MX_CPML_CASE(double, float, unsigned); else MX_CPML_CASE(double, float, size_t); }
+  } else if (psi_prec == MX_REAL64) {
+    if (small) MX_CPML_CASE(float, double, unsigned); else MX_CPML_CASE(float, double, size_t);
   } else {   // a float32 plane is always below 4 GiB (3 N < 2^31)
-    if (psi_prec == MX_REAL64) MX_CPML_CASE(float, double, unsigned);
-    else MX_CPML_CASE(float, float, unsigned);
+    MX_CPML_CASE(float, float, unsigned);
   }
 #undef MX_CPML_CASE
   return hipGetLastError();

@@ -252,6 +252,43 @@ def test_cpml_plane_beyond_32_bit_offsets():
         torch.testing.assert_close(h[:, 0, j], want, rtol=1e-14, atol=1e-14)
 
 
+@pytest.mark.parametrize('axis', [1, 2])
+def test_cpml_psi_beyond_32_bit_offsets(axis):
+    """float32 fields of less than 4 GiB a plane with float64 psi of more (one x plane, a layer
+    of 8 cells over the short axis; about 40 GB in all): two H updates at cells at both ends,
+    in the middle and on both sides of the psi's 4 GiB line."""
+    from meanas_amd import fdtd
+    n, t, dt = 70_000_000, 8, 0.25
+    shape = (1, t, n) if axis == 1 else (1, n, t)
+    e = torch.empty((3, *shape), dtype=torch.float32, device='cuda').uniform_(-1, 1)
+    h = torch.zeros_like(e)
+    layer = fdtd.cpml_params(axis=axis, polarity=-1, dt=dt, thickness=t)
+    layers = [[None, None] for _ in range(3)]
+    layers[axis][0] = layer
+    _, uH = fdtd.updates_with_cpml(layers, dt, [[numpy.ones(k) for k in shape] for _ in range(2)], e, dtype=numpy.float64)
+    uH(e, h)
+    uH(e, h)
+    line = 2 ** 29 // t if axis == 2 else 2 ** 29 - (2 ** 29 // n) * n   # where 8-byte offsets pass 2^32
+    p0, p1, p2 = [torch.from_numpy(q.ravel()).cuda() for q in layer['param_h']]
+    for at in (0, line - 1, line, n // 2, n - 1):
+        here, nxt = [e[:, 0, :, k] if axis == 1 else e[:, 0, k] for k in (at, (at + 1) % n)]   # (3, t)
+        across = (torch.roll(here, -1, 1) - here).double() * p2   # along the layer's axis
+        along = (nxt - here).double()
+        dy, dz = (across, along) if axis == 1 else (along, across)
+        curl = torch.stack([dy[2] - dz[1], dz[0], -dy[0]])
+        psi = p1 * across                                  # after the first update
+        both = 2 * psi + p0 * psi                          # and summed over the two
+        aux = torch.zeros_like(curl)
+        if axis == 1:
+            aux[0], aux[2] = both[2], -both[0]
+        else:
+            aux[0], aux[1] = -both[1], both[0]
+        want = -dt * (2 * curl + aux)
+        got = h[:, 0, :, at] if axis == 1 else h[:, 0, at]
+        # |h| < 4, rounded to float32 once per update: at most 2 x 1.2e-7
+        assert float((got.double() - want).abs().max()) < 3e-7, (axis, at)
+
+
 @pytest.mark.parametrize('axis,comp', [(0, 1), (1, 2), (2, 0)])
 def test_cpml_absorbs_a_pulse_on_gpu(axis, comp):
     from meanas_amd import fdtd
