@@ -79,10 +79,17 @@ __device__ __forceinline__ void put(T* f, size_t base, OFF off, T v) {
 }
 
 // x / d given rd = 1 / d: one product, its exact residual and one correction, then the
-// divide fix-up instruction for zeros, infinities and NaN.  The value rounded at the end
-// is within 2^-20 ulp of the quotient (2^-50 in float64), so the result is the correctly
-// rounded quotient in all but about one of 10^6 (10^15) near-ties.  4 instructions at full
-// rate; the compiler's divide takes 9 (float32) or 13 (float64) of that issue time.
+// divide fix-up instruction for zeros, infinities and NaN; it also makes an infinity of a
+// quotient that overflows, where the correction is inf - inf.  4 instructions at full rate;
+// the compiler's divide takes 9 (float32) or 13 (float64) of that issue time.
+// Where the residual is exact (dividends above 2^-102 in float32, 2^-969 in float64) the
+// value rounded at the end is within 2^-20 ulp of the quotient (2^-50 in float64), so the
+// result is the correctly rounded quotient in all but about one of 10^6 (10^15) near-ties;
+// smaller dividends give a quotient within an ulp (float32, 1e-37: 2.3 % of them an ulp off).
+// Divisors that recip() takes: magnitudes from 2^-126 to 2^126 in float32, from 2^-1022 in
+// float64, zero and infinity.  A larger float32 one counts as infinite (the hardware flushes
+// its reciprocal), a subnormal one as zero.  Looking for them in each cell, to divide by the
+// compiler's code there, cost 3 to 7 % (registers: up to 1.6 times in float64 runs with mu).
 __device__ __forceinline__ double div_by(double x, double d, double rd) {
   const double q = x * rd;
   return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-q, d, x), rd, q), d, x);

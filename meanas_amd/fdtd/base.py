@@ -11,6 +11,10 @@ Fields are real `(3, nx, ny, nz)` arrays, float64 or float32.  torch CUDA tensor
 updated in place on the device; numpy arrays are copied to the device, updated and
 written back in place (so a caller holding the array sees the new values, as with the
 reference).  The kernels run through the C ABI (`mx_fdtd_h`, `mx_fdtd_e`, `mx_fdtd_run`).
+
+Widths and materials divide.  Their magnitudes may be zero, infinite, 2^-126 to 2^126 (about
+8e37) in float32 and at least 2^-1022 in float64: larger ones may be taken as infinite, smaller
+ones as zero.
 """
 from __future__ import annotations
 
