@@ -257,6 +257,7 @@ class _A0:
         self.reversed = 1 if reversed else 0
 
     def __call__(self, x: torch.Tensor) -> torch.Tensor:
+        self.op._check_vec(x, torch.complex128)
         y = torch.empty_like(x)
         _lib.check(_lib.lib().mx_wave(ctypes.byref(self.op.desc), ctypes.byref(self.grid.desc), self.reversed,
                                       x.data_ptr(), y.data_ptr(), torch_stream_handle()), 'mx_wave')

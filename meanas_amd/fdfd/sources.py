@@ -72,6 +72,7 @@ def _masked_source(omega, dxes, epsilon, mu, device, q, keep) -> Callable:
 
     def f(e):
         et, like = _to_dev(e, op)
+        op._check_vec(et, torch.complex128)
         j = torch.empty_like(et)
         _lib.check(_lib.lib().mx_wave_source(ctypes.byref(op.desc), ctypes.byref(grid.desc), q.data_ptr(),
                                              None if keep is None else keep.data_ptr(), c.real, c.imag,

@@ -307,3 +307,16 @@ def test_bench_refuses_several_gpus():
                              env=env2, timeout=120)
         assert res.returncode == 2, res.stderr
         assert 'one GPU only' in res.stdout
+
+
+def test_wave_operators_refuse_host_tensors():
+    """A wave operator or source made for the CPU raises instead of giving host memory to a kernel."""
+    from meanas_amd.fdfd import functional, sources
+    dxes = [[numpy.ones(n) for n in (4, 3, 5)] for _ in range(2)]
+    v = numpy.ones(180, dtype=complex)
+    eps = numpy.ones(180)
+    for f in (functional.e_full(0.3, dxes, eps, device='cpu'), functional.h_full(0.3, dxes, eps, device='cpu'),
+              sources.e_tfsf_source(eps, 0.3, dxes, eps, device='cpu'),
+              sources.e_boundary_source(eps, 0.3, dxes, eps, device='cpu')):
+        with pytest.raises(ValueError, match='CUDA tensor'):
+            f(v)
