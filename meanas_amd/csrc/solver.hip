@@ -1259,8 +1259,8 @@ int mx_solve(const mx_operator* ops, int32_t nops, const mx_system* systems, int
   // close a chunk cost as much as two of its iterations
   if ((!opt || opt->chunk <= 0) && o.form == MX_FORM_FUSED &&
       std::all_of(ops, ops + nops, [&](const mx_operator& op) { return one_launch(op, o.mode); })) {
-    if (o.check_every == o.chunk) o.check_every = kOneLaunchChunk;
     o.chunk = kOneLaunchChunk;
+    if (!opt || opt->check_every <= 0) o.check_every = o.chunk;
   }
   std::string why;
   if (!valid_options(o, &why)) return fail(why);

@@ -97,6 +97,29 @@ def test_merged_finishing_equals_separate(case, monkeypatch):
         assert all(s['status'] == 'converged' for s in sm), sm
 
 
+def test_given_check_interval_stands_beside_the_automatic_chunk():
+    """A batch of one-launch systems runs chunks of 32 iterations unless told otherwise; the
+    caller's check_every stands with them.  Options that resolve alike share a kept plan."""
+    import torch
+    from meanas_amd import _lib
+    from meanas_amd.fdfd.device import DeviceOperator, solve_batch
+    omega, dxes, eps, Js = small_aniso(nrhs=1)
+    op = DeviceOperator(omega, dxes, eps)
+    b = op.map(_lib.MX_MAP_RHS, torch.from_numpy(Js[0]).cuda(), coef=-1j * omega)
+    x = torch.zeros_like(b)
+    work = torch.empty(op.work_bytes(_lib.MX_FP64), dtype=torch.uint8, device=b.device)
+
+    def reused(**options):
+        before = _lib.lib().mx_solve_plan_reuses()
+        x.zero_()
+        solve_batch([op], [dict(op=0, b=b, x=x, work=work, rtol=1e-6)], mode=_lib.MX_FP64, options=options)
+        return _lib.lib().mx_solve_plan_reuses() - before
+    for check in (15, 16, 17, 32):
+        reused(chunk=32, check_every=check)
+        assert reused(chunk=0, check_every=check) == 1, check
+    assert reused(chunk=0, check_every=0) == 1   # as 32 and 32
+
+
 def test_kept_plans_equal_fresh_plans(monkeypatch):
     """mx_solve keeps the last call's tables, maps and captured graph per thread and reuses
     them when the next call has the same inputs.  Consecutive calls on the same buffers --
