@@ -37,28 +37,46 @@ __device__ __forceinline__ double width_u(const double* w, int n) {
   return w ? ((const MX_CONST double*)w)[n] : 1.0;
 }
 
-// A thread's column of a kernel that marches along x: cell t = j nz + k of the (y, z)
-// plane and the planes [ib, ie) of one slab.  Consecutive threads take consecutive cells
-// of the flattened plane (no lanes lost on short or odd rows), and the work items (plane
-// pieces of kFB cells, slab by slab) are dealt so that each XCD -- workgroups go round the
-// 8 of them -- has a contiguous run, whose neighbouring rows and planes meet in its L2.
+// A thread's part of a column kernel: cell t = j nz + k of the (y, z) plane and the planes
+// [ib, ie).  The work items (kFB threads each) are dealt so that each XCD -- workgroups go
+// round the 8 of them -- has a contiguous run, whose neighbouring rows and planes meet in
+// its L2.  Two forms, by the type of the byte offsets (column_grid chooses):
+//   32 bits: a column each, marching along x through one slab.  Consecutive threads take
+//     consecutive cells of the flattened plane (no lanes lost on short or odd rows), and a
+//     block stays in one slab, so the plane and what belongs to it are uniform;
+//   64 bits: a cell each, consecutive threads consecutive cells of the grid (`slab`: nonzero,
+//     or 0 to take the items in the order of the blocks).
+template <typename OFF> constexpr bool kMarches = sizeof(OFF) == 4;
 struct Column {
   int j, k, t, ib, ie;
   bool ok;
 };
-__device__ __forceinline__ Column column(const RGrid& g, int slab) {
-  const int plane = g.ny * g.nz, pieces = (plane + kFB - 1) / kFB;
-  const int nwork = pieces * ((g.nx + slab - 1) / slab), per = (nwork + 7) / 8;
-  const int w = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
-  const int s = w / pieces, piece = w - s * pieces;
+template <typename OFF> __device__ __forceinline__ Column column(const RGrid& g, int slab) {
+  const int plane = g.ny * g.nz, run = kMarches<OFF> ? plane : g.nx * plane;
+  const int pieces = (run + kFB - 1) / kFB;
+  const int nwork = kMarches<OFF> ? pieces * ((g.nx + slab - 1) / slab) : pieces, per = (nwork + 7) / 8;
+  const bool plain = !kMarches<OFF> && slab == 0;
+  const int w = plain ? (int)blockIdx.x : (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+  const int s = kMarches<OFF> ? w / pieces : 0, piece = w - s * pieces;
   Column c;
   c.t = piece * kFB + (int)threadIdx.x;
-  c.ok = (int)(blockIdx.x / 8) < per && w < nwork && c.t < plane;
+  c.ok = (plain || (int)(blockIdx.x / 8) < per) && w < nwork && c.t < run;
+  if constexpr (kMarches<OFF>) {
+    c.ib = s * slab;
+    c.ie = min(c.ib + slab, g.nx);
+  } else {
+    c.ib = c.t / plane;
+    c.ie = c.ib + 1;
+    c.t -= c.ib * plane;
+  }
   c.j = c.t / g.nz;
   c.k = c.t - c.j * g.nz;
-  c.ib = s * slab;
-  c.ie = min(c.ib + slab, g.nx);
   return c;
+}
+// width n of the x axis, n a plane of the thread's column
+template <typename OFF> __device__ __forceinline__ double width_x(const double* w, int n) {
+  if constexpr (kMarches<OFF>) return width_u(w, n);
+  else return width(w, n);
 }
 // element of `f` at a uniform element offset plus a thread's byte offset: with a 32-bit OFF
 // one load from an SGPR base and a VGPR offset
@@ -139,15 +157,15 @@ template <typename T> __device__ __forceinline__ T lane_prev(T v) { return lane_
 // One leapfrog half step, HBM-bound: 36 (H) and 48 (E) bytes a cell in float32.  Marching
 // with the x neighbour in registers, no index division per cell and each XCD on its own
 // run of the grid reads each value about once (a thread per cell read 1.3 times as much).
-// E / H update: 256^3 float32 158 / 121 us (180 / 171 before), that is 5.1 / 5.0 TB/s, a
-// large copy's rate; float64 314 / 239 us (313 / 249); 150 x 141 x 130, in cache, float32
-// 21 / 17 us (28 / 24), float64 39 / 31 us (44 / 37).
+// E / H update: 256^3 float32 152 / 119 us (177 / 167 before), 5.3 / 5.1 TB/s, a large copy's
+// rate; float64 303 / 240 us (313 / 249); 150 x 141 x 130, in cache, float32 21 / 17 us (28 / 24),
+// float64 39 / 31 us (47 / 37).  Where columns lose: column_grid, launch_update.
 // H' = H - dt curl_f(E) / mu (EUPD false) or E' = E + dt curl_b(H) / eps (EUPD true), in
 // place: f is the field differenced, out the one updated.
 template <typename T, bool EUPD, typename OFF>
 __global__ __launch_bounds__(kFB) void k_fdtd_update(RGrid g, T dt, const T* __restrict__ f, T* __restrict__ out,
                                                      const T* __restrict__ mat, T mat_s, int slab) {
-  const Column c = column(g, slab);
+  const Column c = column<OFF>(g, slab);
   if (!c.ok) return;
   const int nx = g.nx, ny = g.ny, nz = g.nz, plane = ny * nz;
   const size_t nc = (size_t)nx * plane;
@@ -181,7 +199,7 @@ __global__ __launch_bounds__(kFB) void k_fdtd_update(RGrid g, T dt, const T* __r
       o[q] = at((const T*)out, q * nc + pi, own);
       m[q] = mat ? at(mat, q * nc + pi, own) : mat_s;
     }
-    const T dx = (T)width_u(wd[0], i), rx = recip(dx);
+    const T dx = (T)width_x<OFF>(wd[0], i), rx = recip(dx);
     const T (&here)[3] = EUPD ? ld : car;
     const T (&xn)[3] = EUPD ? car : ld;
     auto dif = [](T a, T b, T w, T r) { return div_by(EUPD ? a - b : b - a, w, r); };
@@ -487,7 +505,7 @@ __device__ __forceinline__ void cpml_layer(const double (&p)[3], TP (&q)[2], dou
 template <typename T, typename TP, bool EUPD, typename OFF>
 __global__ __launch_bounds__(kFB) void k_cpml(RGrid g, T dt, const T* __restrict__ f, T* __restrict__ out,
                                               const T* __restrict__ mat, double const_scale, CpmlTable tab, int slab) {
-  const Column c = column(g, slab);
+  const Column c = column<OFF>(g, slab);
   if (!c.ok) return;
   const int nx = g.nx, ny = g.ny, nz = g.nz, plane = ny * nz;
   const size_t nc = (size_t)nx * plane;
@@ -559,7 +577,7 @@ __global__ __launch_bounds__(kFB) void k_cpml(RGrid g, T dt, const T* __restrict
         sz[q][1] = at((const TP*)Z.psi, (size_t)(nx + i) * ny * Z.thickness, fz[q]);
       }
     }
-    const double wx = width_u(g.dxh[0], i), rx = recip(wx);
+    const double wx = width_x<OFF>(g.dxh[0], i), rx = recip(wx);
     const T (&here)[3] = EUPD ? ld : car;
     const T (&xn)[3] = EUPD ? car : ld;
     auto dif = [](T a, T b, double w, double r) { return div_by((double)(EUPD ? a - b : b - a), w, r); };
@@ -578,7 +596,7 @@ __global__ __launch_bounds__(kFB) void k_cpml(RGrid g, T dt, const T* __restrict
       const CpmlFace& X = tab.f[q];
       const int pos = i - X.start;
       if ((unsigned)pos < (unsigned)X.thickness) {
-        const double p[3] = {width_u(X.p, pos), width_u(X.p, X.thickness + pos), width_u(X.p, 2 * X.thickness + pos)};
+        const double p[3] = {width_x<OFF>(X.p, pos), width_x<OFF>(X.p, X.thickness + pos), width_x<OFF>(X.p, 2 * X.thickness + pos)};
         cpml_layer<0, TP>(p, sx[q], d, aux);
         const size_t r = (size_t)pos * plane;
         put((TP*)X.psi, r, op, sx[q][0]);
@@ -673,92 +691,77 @@ __global__ __launch_bounds__(kFB) void k_conducting(int nx, int ny, int nz, int 
 // component sum in the field precision (in component order, starting from the x term),
 // the widths in double (the float64 width arrays promote) multiplied one axis at a time,
 // and nothing contracted into fused multiply-adds.  `form` is one of MX_ENERGY_*.
-// Column kernels, HBM-bound.  256^3: energy_hstep float64 270 us (307 with a thread per cell
-// and each component's loads behind the one before), 6.5 TB/s with part of it in cache,
-// float32 146 us (189); poynting 231 / 120 us (246 / 136), divergence 102 / 38 us (107 / 45).
+// HBM-bound, a thread per cell.  256^3: energy_hstep float64 303 us, float32 164 us (327 / 177
+// with the index divisions' neighbours reloaded and each component's loads behind the one
+// before; columns marching along x 343 / 188); poynting 211 / 104 us (224 / 113; columns 231 / 118).
 
-template <typename T, typename OFF>
+template <typename T>
 __global__ __launch_bounds__(kFB) void k_energy(RGrid g, int form, T dt, const T* __restrict__ f0,
                                                 const T* __restrict__ f1, const T* __restrict__ f2,
                                                 const T* __restrict__ f3, const T* __restrict__ eps, T eps_s,
-                                                const T* __restrict__ mu, T mu_s, double* __restrict__ out, int slab) {
+                                                const T* __restrict__ mu, T mu_s, double* __restrict__ out, int order) {
 #pragma clang fp contract(off)
-  const Column col = column(g, slab);
+  const Column col = column<size_t>(g, order);
   if (!col.ok) return;
-  const size_t plane = (size_t)g.ny * g.nz, nc = g.nx * plane;
-  const OFF own0 = (OFF)col.t * (OFF)sizeof(T), oout0 = (OFF)col.t * (OFF)sizeof(double);
-  const double wey = width(g.dxe[1], col.j), wez = width(g.dxe[2], col.k);
-  const double why = width(g.dxh[1], col.j), whz = width(g.dxh[2], col.k);
-#pragma unroll 1
-  for (int i = col.ib; i < col.ie; ++i) {
-    const OFF own = in_loop(own0), oout = in_loop(oout0);
-    // every load of the cell before any is used (f2, f3 and the materials only if given)
-    T a0[3], a1[3], a2[3], a3[3], me[3], mh[3];
+  const int i = col.ib, nc = g.nx * g.ny * g.nz, cell = i * g.ny * g.nz + col.t;
+  const double wex = width(g.dxe[0], i), wey = width(g.dxe[1], col.j), wez = width(g.dxe[2], col.k);
+  const double whx = width(g.dxh[0], i), why = width(g.dxh[1], col.j), whz = width(g.dxh[2], col.k);
+  // every load of the cell before any is used (f2, f3 and the materials only if given)
+  T a0[3], a1[3], a2[3], a3[3], me[3], mh[3];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      const size_t q = c * nc + i * plane;
-      a0[c] = at(f0, q, own);
-      a1[c] = at(f1, q, own);
-      a2[c] = f2 ? at(f2, q, own) : T(0);
-      a3[c] = f3 ? at(f3, q, own) : T(0);
-      me[c] = eps ? at(eps, q, own) : eps_s;
-      mh[c] = mu ? at(mu, q, own) : mu_s;
-    }
-    T se = T(0), sh = T(0);
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      T ee, hh = T(0);
-      switch (form) {
-        case MX_ENERGY_DXMUL: ee = a0[c]; hh = a1[c]; break;
-        case MX_ENERGY_HSTEP: ee = a0[c] * a2[c]; hh = a1[c] * a1[c]; break;
-        case MX_ENERGY_ESTEP: ee = a1[c] * a1[c]; hh = a0[c] * a2[c]; break;
-        case MX_ENERGY_H2E: ee = a2[c] * (a2[c] - a0[c]) / dt; hh = a1[c] * (a3[c] - a1[c]) / dt; break;
-        case MX_ENERGY_E2H: ee = a1[c] * (a3[c] - a1[c]) / dt; hh = a2[c] * (a2[c] - a0[c]) / dt; break;
-        default: ee = a0[c] * a1[c]; break;   // j0 . e1, no material
-      }
-      const T we = form == MX_ENERGY_J ? ee : ee * me[c];
-      const T wh = hh * mh[c];
-      se = c == 0 ? we : se + we;
-      sh = c == 0 ? wh : sh + wh;
-    }
-    const double ue = (double)se * width_u(g.dxe[0], i) * wey * wez;
-    put(out, i * plane, oout, form == MX_ENERGY_J ? ue : ue + (double)sh * width_u(g.dxh[0], i) * why * whz);
+  for (int c = 0; c < 3; ++c) {
+    const int q = c * nc + cell;
+    a0[c] = f0[q];
+    a1[c] = f1[q];
+    a2[c] = f2 ? f2[q] : T(0);
+    a3[c] = f3 ? f3[q] : T(0);
+    me[c] = eps ? eps[q] : eps_s;
+    mh[c] = mu ? mu[q] : mu_s;
   }
+  T se = T(0), sh = T(0);
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    T ee, hh = T(0);
+    switch (form) {
+      case MX_ENERGY_DXMUL: ee = a0[c]; hh = a1[c]; break;
+      case MX_ENERGY_HSTEP: ee = a0[c] * a2[c]; hh = a1[c] * a1[c]; break;
+      case MX_ENERGY_ESTEP: ee = a1[c] * a1[c]; hh = a0[c] * a2[c]; break;
+      case MX_ENERGY_H2E: ee = a2[c] * (a2[c] - a0[c]) / dt; hh = a1[c] * (a3[c] - a1[c]) / dt; break;
+      case MX_ENERGY_E2H: ee = a1[c] * (a3[c] - a1[c]) / dt; hh = a2[c] * (a2[c] - a0[c]) / dt; break;
+      default: ee = a0[c] * a1[c]; break;   // j0 . e1, no material
+    }
+    const T we = form == MX_ENERGY_J ? ee : ee * me[c];
+    const T wh = hh * mh[c];
+    se = c == 0 ? we : se + we;
+    sh = c == 0 ? wh : sh + wh;
+  }
+  const double ue = (double)se * wex * wey * wez;
+  out[cell] = form == MX_ENERGY_J ? ue : ue + (double)sh * whx * why * whz;
 }
 
 // s = E(+1) x H with both width-weighted (fdtd/energy.py:10-87): s_x = ey(i+1) hz - ez(i+1) hy
 // and cyclically, E taken at the next cell along the component's axis (periodic), in
 // double, stored in the field precision.
-template <typename T, typename OFF>
+template <typename T>
 __global__ __launch_bounds__(kFB) void k_poynting(RGrid g, const T* __restrict__ e, const T* __restrict__ h,
-                                                  T* __restrict__ s, int slab) {
+                                                  T* __restrict__ s, int order) {
 #pragma clang fp contract(off)
-  const Column col = column(g, slab);
+  const Column col = column<size_t>(g, order);
   if (!col.ok) return;
-  const int nx = g.nx, ny = g.ny, nz = g.nz;
-  const size_t plane = (size_t)ny * nz, nc = nx * plane;
-  const int jn = col.j + 1 == ny ? 0 : col.j + 1, kn = col.k + 1 == nz ? 0 : col.k + 1;
-  const OFF own0 = (OFF)col.t * (OFF)sizeof(T);
-  const OFF oy0 = ((OFF)jn * (OFF)nz + (OFF)col.k) * (OFF)sizeof(T);
-  const OFF oz0 = ((OFF)col.j * (OFF)nz + (OFF)kn) * (OFF)sizeof(T);
-  const double wey = width(g.dxe[1], col.j), wez = width(g.dxe[2], col.k);
-  const double why = width(g.dxh[1], col.j), whz = width(g.dxh[2], col.k);
-#pragma unroll 1
-  for (int i = col.ib; i < col.ie; ++i) {
-    const OFF own = in_loop(own0), oy = in_loop(oy0), oz = in_loop(oz0);
-    const size_t pi = i * plane, pn = (size_t)(i + 1 == nx ? 0 : i + 1) * plane;
-    const T h0 = at(h, pi, own), h1 = at(h, nc + pi, own), h2 = at(h, 2 * nc + pi, own);
-    const T eyx = at(e, nc + pn, own), ezx = at(e, 2 * nc + pn, own), ezy = at(e, 2 * nc + pi, oy), exy = at(e, pi, oy);
-    const T exz = at(e, pi, oz), eyz = at(e, nc + pi, oz);
-    const double wex = width_u(g.dxe[0], i);
-    const double hx = (double)h0 * width_u(g.dxh[0], i), hy = (double)h1 * why, hz = (double)h2 * whz;
-    const double s0 = ((double)eyx * wey) * hz - ((double)ezx * wez) * hy;
-    const double s1 = ((double)ezy * wez) * hx - ((double)exy * wex) * hz;
-    const double s2 = ((double)exz * wex) * hy - ((double)eyz * wey) * hx;
-    put(s, pi, own, (T)s0);
-    put(s, nc + pi, own, (T)s1);
-    put(s, 2 * nc + pi, own, (T)s2);
-  }
+  const int i = col.ib, nx = g.nx, ny = g.ny, nz = g.nz, plane = ny * nz, nc = nx * plane, cell = i * plane + col.t;
+  const int xn = cell + (i + 1 == nx ? -i : 1) * plane;
+  const int yn = cell + (col.j + 1 == ny ? -col.j : 1) * nz, zn = cell + (col.k + 1 == nz ? -col.k : 1);
+  const T h0 = h[cell], h1 = h[nc + cell], h2 = h[2 * nc + cell];
+  const T eyx = e[nc + xn], ezx = e[2 * nc + xn], ezy = e[2 * nc + yn], exy = e[yn], exz = e[zn], eyz = e[nc + zn];
+  const double wex = width(g.dxe[0], i), wey = width(g.dxe[1], col.j), wez = width(g.dxe[2], col.k);
+  const double hx = (double)h0 * width(g.dxh[0], i), hy = (double)h1 * width(g.dxh[1], col.j);
+  const double hz = (double)h2 * width(g.dxh[2], col.k);
+  const double s0 = ((double)eyx * wey) * hz - ((double)ezx * wez) * hy;
+  const double s1 = ((double)ezy * wez) * hx - ((double)exy * wex) * hz;
+  const double s2 = ((double)exz * wex) * hy - ((double)eyz * wey) * hx;
+  s[cell] = (T)s0;
+  s[nc + cell] = (T)s1;
+  s[2 * nc + cell] = (T)s2;
 }
 
 // ds = sum_a (s_a - s_a(previous cell along a)), unit spacing (deriv_back() without
@@ -766,7 +769,7 @@ __global__ __launch_bounds__(kFB) void k_poynting(RGrid g, const T* __restrict__
 template <typename T, typename OFF>
 __global__ __launch_bounds__(kFB) void k_poynting_div(RGrid g, const T* __restrict__ s, T* __restrict__ ds, int slab) {
 #pragma clang fp contract(off)
-  const Column col = column(g, slab);
+  const Column col = column<OFF>(g, slab);
   if (!col.ok) return;
   const int nx = g.nx, ny = g.ny, nz = g.nz;
   const size_t plane = (size_t)ny * nz, nc = nx * plane;
@@ -799,36 +802,55 @@ bool rgrid(const mx_fdtd_grid* g, RGrid* v, std::string* why) {
   return true;
 }
 
-// Launch of a column kernel: slabs of 6 planes, of 4 and then 2 while the chip has fewer
-// than 8 blocks per CU.  Slabs of 2/4/6/8/16/64 planes, E update of float64 at 256^3: 327,
-// 320, 314, 317, 323, 326 us; of float32 at 228 x 100 x 180: 28.7, 29.1, 30.0, 31.3, 34.0,
-// 42.1 us, with CPML 50.2, 43.2, 42.8, 43.5, 52.8, 107.7 us.
-struct ColumnGrid { int slab; unsigned blocks; };
-ColumnGrid column_grid(const RGrid& v) {
-  const long long pieces = ((long long)v.ny * v.nz + kFB - 1) / kFB;
+// Launch of a kernel with a thread per cell (the 64-bit form of `column`).  Work goes by XCD
+// where nine values a cell stay in the 256 MB cache, else in the order of the blocks, as the
+// memory channels like it better: Poynting flux of 100 x 110 x 120 in float64 15.3 us by XCD,
+// 20.7 plain; 256^3 float64 237 / 211 us, float32 114 / 104; energy of 256^3 float64 330 / 303 us.
+struct ColumnGrid { bool marches; int slab; unsigned blocks; };
+ColumnGrid cell_grid(const RGrid& v, int prec) {
+  const long long cells = (long long)v.nx * v.ny * v.nz, bytes = 9 * cells * (prec == MX_REAL64 ? 8 : 4);
+  const long long nwork = (cells + kFB - 1) / kFB;
+  return {false, bytes <= (256ll << 20) ? 1 : 0, (unsigned)((nwork + 7) / 8 * 8)};
+}
+
+// Launch of a column kernel: slabs of at most `deepest` planes (6, 4 or 2), shallower while
+// the chip has fewer than 8 blocks per CU.  Slabs of 2/4/6/10/16 planes, H then E update of
+// float64: 200 x 181 x 190 232.6, 233.8, 236.8, 239.0, 242.2 us, 256^3 559, 560, 554, 576, 564;
+// float32: 200 x 181 x 190 85.0, 84.2, 86.7, 89.0, 93.2, 256^3 275, 273, 278, 285, 281.  With
+// CPML, float32, slabs of 2/4/6/8: 228 x 100 x 180 50.2, 43.2, 42.8, 43.5 us.
+// A plane of fewer than kThinPlane cells leaves too much of a block without columns, and the
+// byte offsets of one, in the widest type that the kernel holds a value per cell of
+// (`prec`), may not fit 32 bits: then a thread per cell.  Columns / cells, E update of float64:
+// 2000000 x 1 x 1 887 / 30 us, 40000 x 8 x 10 50 / 43, 4000 x 16 x 15 15.4 / 14.7, 3000 x 20 x 20
+// 19.1 / 17.9, 5000 x 32 x 32 89 / 91; with CPML, float32: 8000 x 25 x 25 69 / 80, 3000 x 300 x 1 18 / 12.
+constexpr long long kThinPlane = 512;
+ColumnGrid column_grid(const RGrid& v, int prec, int deepest) {
+  const long long plane = (long long)v.ny * v.nz;
+  if (plane < kThinPlane || plane * (prec == MX_REAL64 ? 8 : 4) >= (1ll << 32)) return cell_grid(v, prec);
+  const long long pieces = (plane + kFB - 1) / kFB;
   int slab = 0;
   for (int want : {6, 4, 2}) {
+    if (want > deepest) continue;
     slab = std::min(want, v.nx);
     if (pieces * ((v.nx + slab - 1) / slab) >= 2048) break;
   }
-  const long long nwork = pieces * ((v.nx + slab - 1) / slab);
-  return {slab, (unsigned)((nwork + 7) / 8 * 8)};
-}
-// whether the byte offsets of a plane fit 32 bits (beyond: kernels with 64-bit offsets);
-// `prec` is the widest type that the kernel holds a value per cell of
-bool small_plane(const RGrid& v, int prec) {
-  return (unsigned long long)v.ny * v.nz * (prec == MX_REAL64 ? 8 : 4) < (1ull << 32);
+  return {true, slab, (unsigned)((pieces * ((v.nx + slab - 1) / slab) + 7) / 8 * 8)};
 }
 
 template <bool EUPD>
 hipError_t launch_update(const RGrid& v, int prec, double dt, const void* f, void* out, const void* mat, double mat_s,
                          hipStream_t s) {
-  const ColumnGrid cg = column_grid(v);
+  // float64 with a material field, from twice the cache on: a thread per cell.  E update,
+  // columns / cells: 170 x 171 x 172 88 / 92 us, 180^3 107 / 106, 210 x 200 x 170 139 / 129,
+  // 256^3 318 / 303, 150 x 400 x 400 462 / 426; without a material (H) 80 / 86 at 180^3, 240 / 243 at 256^3
+  // (float32 E update 152 / 150 at 256^3, 47 / 64 at 200 x 181 x 190: columns).
+  const bool cells = prec == MX_REAL64 && mat && 96ll * v.nx * v.ny * v.nz > (512ll << 20);
+  const ColumnGrid cg = cells ? cell_grid(v, prec) : column_grid(v, prec, 4);
 #define MX_UPDATE_CASE(T, OFF)                                                                                      \
   hipLaunchKernelGGL((k_fdtd_update<T, EUPD, OFF>), dim3(cg.blocks), dim3(kFB), 0, s, v, (T)dt, (const T*)f, (T*)out, \
                      (const T*)mat, (T)mat_s, cg.slab)
-  if (prec == MX_REAL64) { if (small_plane(v, prec)) MX_UPDATE_CASE(double, unsigned); else MX_UPDATE_CASE(double, size_t); }
-  else MX_UPDATE_CASE(float, unsigned);   // a float32 plane is always below 4 GiB (3 N < 2^31)
+  if (prec == MX_REAL64) { if (cg.marches) MX_UPDATE_CASE(double, unsigned); else MX_UPDATE_CASE(double, size_t); }
+  else { if (cg.marches) MX_UPDATE_CASE(float, unsigned); else MX_UPDATE_CASE(float, size_t); }
 #undef MX_UPDATE_CASE
   return hipGetLastError();
 }
@@ -855,39 +877,37 @@ hipError_t launch_conducting(const RGrid& v, int prec, int dir, int pol, int is_
   return hipGetLastError();
 }
 
-// a column kernel in the field precision, with 32-bit byte offsets where the widest plane it
-// addresses allows (a float32 plane always does: 3 N < 2^31)
-#define MX_COLUMN_LAUNCH(kern, small, ...)                                                             \
-  do {                                                                                                 \
-    const ColumnGrid cg = column_grid(v);                                                              \
-    if (prec == MX_REAL64) {                                                                           \
-      typedef double T;                                                                                \
-      if (small) hipLaunchKernelGGL((kern<T, unsigned>), dim3(cg.blocks), dim3(kFB), 0, s, v, __VA_ARGS__, cg.slab); \
-      else hipLaunchKernelGGL((kern<T, size_t>), dim3(cg.blocks), dim3(kFB), 0, s, v, __VA_ARGS__, cg.slab);         \
-    } else {                                                                                           \
-      typedef float T;                                                                                 \
-      if (small) hipLaunchKernelGGL((kern<T, unsigned>), dim3(cg.blocks), dim3(kFB), 0, s, v, __VA_ARGS__, cg.slab); \
-      else hipLaunchKernelGGL((kern<T, size_t>), dim3(cg.blocks), dim3(kFB), 0, s, v, __VA_ARGS__, cg.slab);         \
-    }                                                                                                  \
-  } while (0)
-
 hipError_t launch_energy(const RGrid& v, int prec, int form, double dt, const void* const* f, const void* eps,
                          double eps_s, const void* mu, double mu_s, double* out, hipStream_t s) {
-  MX_COLUMN_LAUNCH(k_energy, small_plane(v, MX_REAL64), form, (T)dt, (const T*)f[0], (const T*)f[1], (const T*)f[2],
-                   (const T*)f[3], (const T*)eps, (T)eps_s, (const T*)mu, (T)mu_s, out);
+  const ColumnGrid cg = cell_grid(v, prec);
+#define MX_ENERGY_CASE(T)                                                                                          \
+  hipLaunchKernelGGL(k_energy<T>, dim3(cg.blocks), dim3(kFB), 0, s, v, form, (T)dt, (const T*)f[0], (const T*)f[1], \
+                     (const T*)f[2], (const T*)f[3], (const T*)eps, (T)eps_s, (const T*)mu, (T)mu_s, out, cg.slab)
+  if (prec == MX_REAL64) MX_ENERGY_CASE(double);
+  else MX_ENERGY_CASE(float);
+#undef MX_ENERGY_CASE
   return hipGetLastError();
 }
 
 hipError_t launch_poynting(const RGrid& v, int prec, const void* e, const void* h, void* out, hipStream_t s) {
-  MX_COLUMN_LAUNCH(k_poynting, small_plane(v, prec), (const T*)e, (const T*)h, (T*)out);
+  const ColumnGrid cg = cell_grid(v, prec);
+#define MX_POYNTING_CASE(T) \
+  hipLaunchKernelGGL(k_poynting<T>, dim3(cg.blocks), dim3(kFB), 0, s, v, (const T*)e, (const T*)h, (T*)out, cg.slab)
+  if (prec == MX_REAL64) MX_POYNTING_CASE(double);
+  else MX_POYNTING_CASE(float);
+#undef MX_POYNTING_CASE
   return hipGetLastError();
 }
 
 hipError_t launch_poynting_div(const RGrid& v, int prec, const void* sv, void* ds, hipStream_t s) {
-  MX_COLUMN_LAUNCH(k_poynting_div, small_plane(v, prec), (const T*)sv, (T*)ds);
+  const ColumnGrid cg = column_grid(v, prec, 6);
+#define MX_DIV_CASE(T, OFF) \
+  hipLaunchKernelGGL((k_poynting_div<T, OFF>), dim3(cg.blocks), dim3(kFB), 0, s, v, (const T*)sv, (T*)ds, cg.slab)
+  if (prec == MX_REAL64) { if (cg.marches) MX_DIV_CASE(double, unsigned); else MX_DIV_CASE(double, size_t); }
+  else { if (cg.marches) MX_DIV_CASE(float, unsigned); else MX_DIV_CASE(float, size_t); }
+#undef MX_DIV_CASE
   return hipGetLastError();
 }
-#undef MX_COLUMN_LAUNCH
 
 // Layer table of a CPML update: faces in increasing (axis, polarity) order (the order
 // the reference accumulates in), each inside the grid, with its arrays.
@@ -915,19 +935,17 @@ bool cpml_table(const RGrid& v, const mx_cpml_layer* layers, int n, bool eupd, C
 template <bool EUPD>
 hipError_t launch_cpml(const RGrid& v, int prec, int psi_prec, double dt, const void* f, void* out,
                        const void* mat, double mat_s, const CpmlTable& tab, hipStream_t s) {
-  const ColumnGrid cg = column_grid(v);
+  // a layer's plane has at most the grid plane's cells, in the psi precision
+  const ColumnGrid cg = column_grid(v, prec == MX_REAL64 ? prec : psi_prec, 6);
 #define MX_CPML_CASE(T, TP, OFF)                                                                              \
   hipLaunchKernelGGL((k_cpml<T, TP, EUPD, OFF>), dim3(cg.blocks), dim3(kFB), 0, s, v, (T)dt, (const T*)f, (T*)out, \
                      (const T*)mat, dt / mat_s, tab, cg.slab)
-  // a layer's plane has at most the grid plane's cells, in the psi precision
-  const bool small = small_plane(v, prec == MX_REAL64 ? prec : psi_prec);
   if (prec == MX_REAL64) {
-    if (psi_prec == MX_REAL64) { if (small) MX_CPML_CASE(double, double, unsigned); else MX_CPML_CASE(double, double, size_t); }
-    else { if (small) MX_CPML_CASE(double, float, unsigned); else MX_CPML_CASE(double, float, size_t); }
-  } else if (psi_prec == MX_REAL64) {
-    if (small) MX_CPML_CASE(float, double, unsigned); else MX_CPML_CASE(float, double, size_t);
-  } else {   // a float32 plane is always below 4 GiB (3 N < 2^31)
-    MX_CPML_CASE(float, float, unsigned);
+    if (psi_prec == MX_REAL64) { if (cg.marches) MX_CPML_CASE(double, double, unsigned); else MX_CPML_CASE(double, double, size_t); }
+    else { if (cg.marches) MX_CPML_CASE(double, float, unsigned); else MX_CPML_CASE(double, float, size_t); }
+  } else {
+    if (psi_prec == MX_REAL64) { if (cg.marches) MX_CPML_CASE(float, double, unsigned); else MX_CPML_CASE(float, double, size_t); }
+    else { if (cg.marches) MX_CPML_CASE(float, float, unsigned); else MX_CPML_CASE(float, float, size_t); }
   }
 #undef MX_CPML_CASE
   return hipGetLastError();

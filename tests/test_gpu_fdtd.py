@@ -138,7 +138,7 @@ def test_updates_keep_infinities_zeros_and_nan(dtype):
 
 def _plain_step(e, h, dt, dxes, eps, mu, which):
     """One update in torch, in the fields' own precision, by the updates' expressions."""
-    w = [[torch.as_tensor(d).to(e.dtype).reshape([-1 if b == a else 1 for b in range(3)]) for a, d in enumerate(side)]
+    w = [[torch.as_tensor(d).to(e).reshape([-1 if b == a else 1 for b in range(3)]) for a, d in enumerate(side)]
          for side in dxes]
 
     def d(f, a):
@@ -147,7 +147,7 @@ def _plain_step(e, h, dt, dxes, eps, mu, which):
         return (f - torch.roll(f, 1, a)) / w[1][a]
     f = e if which == 'h' else h
     c = torch.stack([d(f[2], 1) - d(f[1], 2), d(f[0], 2) - d(f[2], 0), d(f[1], 0) - d(f[0], 1)])
-    dt = torch.tensor(dt, dtype=e.dtype)
+    dt = torch.tensor(dt, dtype=e.dtype, device=e.device)
     return (e, h - dt * c / mu) if which == 'h' else (e + dt * c / eps, h)
 
 
@@ -578,6 +578,59 @@ def test_column_kernels_at_block_and_slab_edges(dtype, shape):
     fdtd.maxwell_e(0.2, dxes)(e, h, eps)
     numpy.testing.assert_allclose(h, h1, **kw)
     numpy.testing.assert_allclose(e, e1, **kw)
+
+
+@pytest.mark.parametrize('dtype', [numpy.float64, numpy.float32])
+@pytest.mark.parametrize('shape', [(3000, 1, 1), (600, 1, 3), (9, 7, 73), (9, 8, 64), (7, 19, 27), (1, 3, 256), (13, 30, 26)])
+def test_cells_and_columns_by_plane_size(dtype, shape):
+    """The same on thin planes (a thread per cell), of 511 cells and of 512, 513 and more
+    (columns), and the CPML updates."""
+    test_column_kernels_at_block_and_slab_edges(dtype, shape)
+    test_cpml_columns_and_slabs(dtype, dtype, 1e-11 if dtype == numpy.float64 else 1e-4, shape)
+
+
+@pytest.mark.parametrize('fdt,pdt,tol', [(numpy.float64, numpy.float32, 1e-5), (numpy.float32, numpy.float64, 1e-4)])
+@pytest.mark.parametrize('shape', [(10, 90, 7), (10, 7, 90), (10, 9, 7)])
+def test_cpml_overlapping_layers_by_plane_size(fdt, pdt, tol, shape):
+    """Layers that overlap on a short axis, in columns and with a thread per cell."""
+    test_cpml_updates_match_oracle(fdt, pdt, tol, shape, fc.ALL_FACES, 4, True)
+
+
+@pytest.mark.parametrize('dtype,shape', [(torch.float64, (140, 163, 163)), (torch.float64, (141, 163, 166)),
+                                         (torch.float32, (195, 196, 196)), (torch.float64, (177, 177, 178)),
+                                         (torch.float64, (178, 177, 178))])
+def test_large_grids_on_both_sides_of_the_cache(dtype, shape):
+    """Grids just below and above the sizes where the work goes by blocks instead of by XCD, and
+    where float64 updates with a material take a thread per cell, against the same in torch."""
+    from meanas_amd import fdtd
+    gen = torch.Generator(device='cuda').manual_seed(1)
+    e, h, e2 = [torch.randn((3, *shape), dtype=dtype, device='cuda', generator=gen) for _ in range(3)]
+    eps = 1 + torch.rand((3, *shape), dtype=dtype, device='cuda', generator=gen)
+    dxes = [[0.8 + 0.4 * numpy.random.default_rng(a).random(n) for a, n in enumerate(shape)] for _ in range(2)]
+    tol = dict(rtol=1e-13, atol=1e-12) if dtype == torch.float64 else dict(rtol=1e-5, atol=1e-4)
+    torch.testing.assert_close(fdtd.energy_hstep(e, h, e2, epsilon=eps),
+                               ((e * e2 * eps).double().sum(0) + (h * h).double().sum(0)), **tol)
+    nx, ny, nz = [torch.roll(e, -1, a) for a in (1, 2, 3)]
+    torch.testing.assert_close(fdtd.poynting(e, h), torch.stack([nx[1] * h[2] - nx[2] * h[1], ny[2] * h[0] - ny[0] * h[2],
+                                                                 nz[0] * h[1] - nz[1] * h[0]]), **tol)
+    want_h = _plain_step(e, h, 0.2, dxes, None, eps, 'h')[1]
+    want_e = _plain_step(e, h, 0.2, dxes, eps, None, 'e')[0]
+    torch.testing.assert_close(fdtd.maxwell_h(0.2, dxes)(e, h.clone(), eps), want_h, **tol)
+    torch.testing.assert_close(fdtd.maxwell_e(0.2, dxes)(e.clone(), h, eps), want_e, **tol)
+
+
+def test_updates_on_a_line_of_1e8_cells():
+    """A grid of one cell across and 1.1e8 cells along x: as many blocks as a launch may have."""
+    from meanas_amd import fdtd
+    n = 110_000_000
+    f = torch.empty((3, n, 1, 1), dtype=torch.float32, device='cuda').uniform_(-1, 1)
+    e, h = torch.zeros_like(f), torch.zeros_like(f)
+    fdtd.maxwell_h(0.5)(f, h)
+    fdtd.maxwell_e(0.5)(e, f, 1.0)
+    x = f[:, :, 0, 0]
+    for got, sign, d in ((h, -0.5, torch.roll(x, -1, 1) - x), (e, 0.5, x - torch.roll(x, 1, 1))):
+        assert not got[0].any()
+        assert torch.equal(got[1, :, 0, 0], -sign * d[2]) and torch.equal(got[2, :, 0, 0], sign * d[1])
 
 
 @pytest.mark.parametrize('name', ['update', 'energy', 'poynting'])
