@@ -951,14 +951,14 @@ hipError_t launch_cpml(const RGrid& v, int prec, int psi_prec, double dt, const 
   return hipGetLastError();
 }
 
-struct StepShape { int rows, slab; };
+struct StepShape { int rows, slab; double cost; };
 long long step_tiles(const RGrid& v, int rows, int steps) {
   const int oy = rows - 2 * steps, oz = 64 - 2 * steps;
   return (long long)((v.ny + oy - 1) / oy) * ((v.nz + oz - 1) / oz);
 }
 
 // Rows and slab depth of a pass: those with the least modelled time, over all equal divisions
-// of x.  A block takes slab + 3 S - 2 iterations, each as long as its rows are many; the n
+// of x (at most 125 depths a row count, 0.5 us, once per run).  A block takes slab + 3 S - 2 iterations, each as long as its rows are many; the n
 // blocks that a CU gets (256 CUs) cost n, plus a fifth of one in float32, where two blocks
 // share a CU.  Measured at 256^3 float64, two steps: slabs 16/24/32/48/64/128 model
 // 200/196/180/208/204/264, time 611/576/542/595/572/696 us.  Float32 with 14 rows instead of
@@ -972,34 +972,28 @@ StepShape step_shape(const RGrid& v, int steps, size_t elem) {
     const char* env = getenv("MEANAS_AMD_FDTD_SLAB");
     return env ? atoi(env) : 0;
   }();
-  StepShape best{0, 0};
-  double best_cost = 0.0;
+  const int deepest = forced > 0 ? std::min(forced, kStepMaxSlab) : kStepMaxSlab;
+  const int shallowest = forced > 0 ? deepest : kStepMinSlab;
+  StepShape best{0, 0, 0.0};
   for (int rows : {kStepRows, kStepRowsMore}) {
     if (rows > kStepRows && elem != 4) continue;
     const long long tiles = step_tiles(v, rows, steps);
-    int last = 0;
-    for (int count = (v.nx + kStepMaxSlab - 1) / kStepMaxSlab; count <= v.nx; ++count) {
-      const int slab = forced > 0 ? std::min(std::min(forced, kStepMaxSlab), v.nx) : (v.nx + count - 1) / count;
-      if (slab == last) continue;
-      if (slab < kStepMinSlab && last > 0) break;
-      last = slab;
-      const long long blocks = tiles * ((v.nx + slab - 1) / slab);
-      const double n = (double)((blocks + 255) / 256) + (elem == 4 ? 0.2 : 0.0);
-      const double cost = n * (slab + 3 * steps - 2) * rows;
-      if (best.slab == 0 || cost < best_cost) {
-        best_cost = cost;
-        best = {rows, slab};
-      }
+    // the equal divisions: every slab depth that is the ceiling of nx over some count
+    for (int depth = std::min(deepest, v.nx); depth >= std::min(shallowest, v.nx); --depth) {
+      const int count = (v.nx + depth - 1) / depth, slab = (v.nx + count - 1) / count;
+      if (slab != depth && forced <= 0) continue;
+      const double n = (double)((tiles * count + 255) / 256) + (elem == 4 ? 0.2 : 0.0);
+      const double cost = n * (depth + 3 * steps - 2) * rows;
+      if (best.slab == 0 || cost < best.cost) best = {rows, depth, cost};
     }
   }
   return best;
 }
 
 template <typename T, int S>
-hipError_t launch_pass(const RGrid& v, T dt, const void* ei, const void* hi, void* eo, void* ho, const void* eps,
+hipError_t launch_pass(const RGrid& v, const StepShape& shape, T dt, const void* ei, const void* hi, void* eo, void* ho, const void* eps,
                        double eps_s, const void* mu, double mu_s, hipStream_t s) {
   static_assert(kStepMaxSlab + 5 * S - 4 <= kStepTab, "x table");
-  const StepShape shape = step_shape(v, S, sizeof(T));
   const int slab = shape.slab;
   const long long nwork = step_tiles(v, shape.rows, S) * ((v.nx + slab - 1) / slab);
   const unsigned nb = (unsigned)(((nwork + 7) / 8) * 8);
@@ -1026,22 +1020,19 @@ hipError_t launch_pass(const RGrid& v, T dt, const void* ei, const void* hi, voi
 int step_passes(int steps) { return steps / 2 + steps % 2; }
 
 // `steps` steps, (e, h) -> (e2, h2) -> (e, h) -> ... by passes
-hipError_t launch_steps(const RGrid& v, int prec, double dt, void* e, void* h, void* e2, void* h2, const void* eps,
-                        double eps_s, const void* mu, double mu_s, int steps, hipStream_t s) {
+template <typename T>
+hipError_t launch_steps(const RGrid& v, T dt, void* e, void* h, void* e2, void* h2, const void* eps, double eps_s,
+                        const void* mu, double mu_s, int steps, hipStream_t s) {
+  const StepShape two = step_shape(v, 2, sizeof(T)), one = step_shape(v, 1, sizeof(T));
   const int passes = step_passes(steps);
   for (int t = 0; t < passes; ++t) {
     void* ei = (t & 1) ? e2 : e;
     void* hi = (t & 1) ? h2 : h;
     void* eo = (t & 1) ? e : e2;
     void* ho = (t & 1) ? h : h2;
-    const bool two = 2 * t + 2 <= steps;
-    hipError_t err;
-    if (prec == MX_REAL64)
-      err = two ? launch_pass<double, 2>(v, dt, ei, hi, eo, ho, eps, eps_s, mu, mu_s, s)
-                : launch_pass<double, 1>(v, dt, ei, hi, eo, ho, eps, eps_s, mu, mu_s, s);
-    else
-      err = two ? launch_pass<float, 2>(v, (float)dt, ei, hi, eo, ho, eps, eps_s, mu, mu_s, s)
-                : launch_pass<float, 1>(v, (float)dt, ei, hi, eo, ho, eps, eps_s, mu, mu_s, s);
+    const hipError_t err = 2 * t + 2 <= steps
+                               ? launch_pass<T, 2>(v, two, dt, ei, hi, eo, ho, eps, eps_s, mu, mu_s, s)
+                               : launch_pass<T, 1>(v, one, dt, ei, hi, eo, ho, eps, eps_s, mu, mu_s, s);
     if (err != hipSuccess) return err;
   }
   return hipSuccess;
@@ -1097,7 +1088,9 @@ int mx_fdtd_run(const mx_fdtd_grid* g, int32_t prec, double dt, void* e, void* h
   void* h2 = nullptr;
   hipError_t err = hipMallocAsync(&e2, bytes, s);
   if (err == hipSuccess) err = hipMallocAsync(&h2, bytes, s);
-  if (err == hipSuccess) err = mx::launch_steps(v, prec, dt, e, h, e2, h2, eps, eps_scalar, mu, mu_scalar, steps, s);
+  if (err == hipSuccess)
+    err = prec == MX_REAL64 ? mx::launch_steps<double>(v, dt, e, h, e2, h2, eps, eps_scalar, mu, mu_scalar, steps, s)
+                            : mx::launch_steps<float>(v, (float)dt, e, h, e2, h2, eps, eps_scalar, mu, mu_scalar, steps, s);
   if (err == hipSuccess && (mx::step_passes(steps) & 1)) {   // the last pass wrote the second pair
     err = hipMemcpyAsync(e, e2, bytes, hipMemcpyDeviceToDevice, s);
     if (err == hipSuccess) err = hipMemcpyAsync(h, h2, bytes, hipMemcpyDeviceToDevice, s);

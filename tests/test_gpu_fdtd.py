@@ -111,6 +111,24 @@ def test_float32_runs_in_blocks_of_14_rows(shape, mu_kind, steps):
     assert torch.equal(et, e2) and torch.equal(ht, h2)
 
 
+@pytest.mark.parametrize('shape', [(100_003, 1, 1), (30_000, 2, 3), (129, 1, 70), (1, 1, 400)])
+@pytest.mark.parametrize('dtype', [torch.float64, torch.float32])
+def test_runs_on_long_thin_grids(shape, dtype):
+    """Runs equal the separate updates bit for bit on grids of many slabs, or of one plane."""
+    from meanas_amd import fdtd
+    gen = torch.Generator(device='cuda').manual_seed(2)
+    e, h = [torch.randn((3, *shape), dtype=dtype, device='cuda', generator=gen) for _ in range(2)]
+    eps = 1 + torch.rand((3, *shape), dtype=dtype, device='cuda', generator=gen)
+    dxes = [[0.8 + 0.4 * numpy.random.default_rng(a).random(n) for a, n in enumerate(shape)] for _ in range(2)]
+    e1, h1 = e.clone(), h.clone()
+    fdtd.run(e1, h1, eps, 0.2, dxes, steps=5)
+    me, mh = fdtd.maxwell_e(0.2, dxes), fdtd.maxwell_h(0.2, dxes)
+    for _ in range(5):
+        mh(e, h)
+        me(e, h, eps)
+    assert torch.equal(e, e1) and torch.equal(h, h1)
+
+
 @pytest.mark.parametrize('dtype', [numpy.float64, numpy.float32])
 def test_updates_keep_infinities_zeros_and_nan(dtype):
     """Infinite fields and materials, zero and NaN values divide as numpy divides them."""
