@@ -1016,21 +1016,35 @@ hipError_t launch_pass(const RGrid& v, const StepShape& shape, T dt, const void*
   return hipGetLastError();
 }
 
-// passes of a run: two steps each, a last single step if their number is odd
-int step_passes(int steps) { return steps / 2 + steps % 2; }
+// Grids of few x planes, where a pass's run-in (3 S - 2 planes a slab) is most of its work.
+// Separate updates on one plane, and on two while the fields and materials stay in the cache;
+// passes of one step on two, and in float64 with a mu field (whose two-step pass spills) on up
+// to four.  us per step, two steps a pass / one / separate: float64 1 x 1000 x 1000 55 / 47 / 35, with mu
+// 70 / 55 / 37, 1 x 4000 x 4000 698 / 640 / 539; 2 x 1000 x 1000 69 / 65 / 57, 2 x 2000 x 2000 254 / 251 / 272, with
+// mu 382 / 301 / 322; 4 x 500 x 500 33 / 33 / 36, with mu 46 / 38 / 38; 5 x 1000 x 1000 with mu 159 / 190 / 231;
+// float32 1 x 1000 x 1000 37 / 30 / 24, 2 x 1000 x 1000 43 / 34 / 34, 3 x 1000 x 1000 50 / 48 / 46.
+bool separate_updates(const RGrid& v, int prec, bool mu_field) {
+  const long long bytes = (mu_field ? 12ll : 9ll) * v.nx * v.ny * v.nz * (prec == MX_REAL64 ? 8 : 4);
+  return v.nx == 1 || (v.nx == 2 && bytes <= (256ll << 20));
+}
+bool single_steps(const RGrid& v, int prec, bool mu_field) {
+  return v.nx <= 2 || (v.nx <= 4 && prec == MX_REAL64 && mu_field);
+}
 
-// `steps` steps, (e, h) -> (e2, h2) -> (e, h) -> ... by passes
+// `steps` steps by passes of two, a last single one if their number is odd (or of one each):
+// (e, h) -> (e2, h2) -> (e, h) -> ...; *passes: how many
 template <typename T>
 hipError_t launch_steps(const RGrid& v, T dt, void* e, void* h, void* e2, void* h2, const void* eps, double eps_s,
-                        const void* mu, double mu_s, int steps, hipStream_t s) {
+                        const void* mu, double mu_s, int steps, int* passes, hipStream_t s) {
+  const bool single = single_steps(v, sizeof(T) == 8 ? MX_REAL64 : MX_REAL32, mu != nullptr);
+  *passes = single ? steps : steps / 2 + steps % 2;
   const StepShape two = step_shape(v, 2, sizeof(T)), one = step_shape(v, 1, sizeof(T));
-  const int passes = step_passes(steps);
-  for (int t = 0; t < passes; ++t) {
+  for (int t = 0; t < *passes; ++t) {
     void* ei = (t & 1) ? e2 : e;
     void* hi = (t & 1) ? h2 : h;
     void* eo = (t & 1) ? e : e2;
     void* ho = (t & 1) ? h : h2;
-    const hipError_t err = 2 * t + 2 <= steps
+    const hipError_t err = !single && 2 * t + 2 <= steps
                                ? launch_pass<T, 2>(v, two, dt, ei, hi, eo, ho, eps, eps_s, mu, mu_s, s)
                                : launch_pass<T, 1>(v, one, dt, ei, hi, eo, ho, eps, eps_s, mu, mu_s, s);
     if (err != hipSuccess) return err;
@@ -1075,7 +1089,8 @@ int mx_fdtd_run(const mx_fdtd_grid* g, int32_t prec, double dt, void* e, void* h
   if (steps == 0) return 0;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const size_t comp = (size_t)v.nx * v.ny * v.nz * (prec == MX_REAL64 ? 8 : 4), bytes = 3 * comp;
-  if (comp >= (size_t)1 << 32) {   // beyond the passes' 32-bit offsets: the separate updates
+  // (a component of 4 GiB is beyond the passes' 32-bit offsets)
+  if (comp >= (size_t)1 << 32 || mx::separate_updates(v, prec, mu != nullptr)) {
     for (int t = 0; t < steps; ++t) {
       hipError_t err = mx::launch_h(v, prec, dt, e, h, mu, mu_scalar, s);
       if (err == hipSuccess) err = mx::launch_e(v, prec, dt, e, h, eps, eps_scalar, s);
@@ -1086,12 +1101,14 @@ int mx_fdtd_run(const mx_fdtd_grid* g, int32_t prec, double dt, void* e, void* h
   // passes alternate between (e, h) and a second pair, allocated in stream order
   void* e2 = nullptr;
   void* h2 = nullptr;
+  int passes = 0;
   hipError_t err = hipMallocAsync(&e2, bytes, s);
   if (err == hipSuccess) err = hipMallocAsync(&h2, bytes, s);
   if (err == hipSuccess)
-    err = prec == MX_REAL64 ? mx::launch_steps<double>(v, dt, e, h, e2, h2, eps, eps_scalar, mu, mu_scalar, steps, s)
-                            : mx::launch_steps<float>(v, (float)dt, e, h, e2, h2, eps, eps_scalar, mu, mu_scalar, steps, s);
-  if (err == hipSuccess && (mx::step_passes(steps) & 1)) {   // the last pass wrote the second pair
+    err = prec == MX_REAL64
+              ? mx::launch_steps<double>(v, dt, e, h, e2, h2, eps, eps_scalar, mu, mu_scalar, steps, &passes, s)
+              : mx::launch_steps<float>(v, (float)dt, e, h, e2, h2, eps, eps_scalar, mu, mu_scalar, steps, &passes, s);
+  if (err == hipSuccess && (passes & 1)) {   // the last pass wrote the second pair
     err = hipMemcpyAsync(e, e2, bytes, hipMemcpyDeviceToDevice, s);
     if (err == hipSuccess) err = hipMemcpyAsync(h, h2, bytes, hipMemcpyDeviceToDevice, s);
   }
