@@ -255,7 +255,8 @@ constexpr int kStepMaxSlab = 128, kStepMinSlab = 4;
 constexpr int kStepTab = 136;    // planes of the x table: the slab and the pipeline's run-in
 enum : int { MU_ONE = 0, MU_SCALAR = 1, MU_FIELD = 2 };
 
-template <typename T, int W, int S, bool EPS, int MU>
+// OFF: byte offsets within one component
+template <typename T, typename OFF, int W, int S, bool EPS, int MU>
 __global__ __launch_bounds__(64 * W) void k_fdtd_steps(RGrid g, T dt, const T* __restrict__ e0,
                                                                const T* __restrict__ h0, T* __restrict__ e1,
                                                                T* __restrict__ h1, const T* __restrict__ eps,
@@ -282,14 +283,13 @@ __global__ __launch_bounds__(64 * W) void k_fdtd_steps(RGrid g, T dt, const T* _
   const int j = j0 + ty - S, k = k0 + tz - S;
   const bool valid = ty >= S && ty < W - S && tz >= S && tz < 64 - S && j < ny && k < nz;
   const int jw = wrap(j, ny), kw = wrap(k, nz);
-  // byte offsets within one component are 32-bit (the host keeps it below 4 GiB): an SGPR
-  // base per component and one VGPR offset per plane
-  const unsigned own = (unsigned)(jw * nz + kw) * (unsigned)sizeof(T);
-  const unsigned pbytes = (unsigned)plane * (unsigned)sizeof(T);
-  auto ld = [&](const T* f, int c, unsigned off) -> T {
+  // with 32-bit offsets an SGPR base per component and one VGPR offset per plane
+  const OFF own = (OFF)(jw * nz + kw) * (OFF)sizeof(T);
+  const OFF pbytes = (OFF)plane * (OFF)sizeof(T);
+  auto ld = [&](const T* f, int c, OFF off) -> T {
     return *(const MX_GLOBAL T*)((const MX_GLOBAL char*)(f + (size_t)c * nc) + off);
   };
-  auto st = [&](T* f, int c, unsigned off, T v) {
+  auto st = [&](T* f, int c, OFF off, T v) {
     *(MX_GLOBAL T*)((MX_GLOBAL char*)(f + (size_t)c * nc) + off) = v;
   };
 
@@ -327,7 +327,7 @@ __global__ __launch_bounds__(64 * W) void k_fdtd_steps(RGrid g, T dt, const T* _
   int pn = wrap(first, nx);    // the plane of H_0 and the materials in the next fetch
   auto fetch = [&](In& I) {
     const int p1 = pn + 1 == nx ? 0 : pn + 1;
-    const unsigned o1 = (unsigned)p1 * pbytes + own, o0 = (unsigned)pn * pbytes + own;
+    const OFF o1 = (OFF)p1 * pbytes + own, o0 = (OFF)pn * pbytes + own;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       I.e[c] = ld(e0, c, o1);
@@ -338,7 +338,7 @@ __global__ __launch_bounds__(64 * W) void k_fdtd_steps(RGrid g, T dt, const T* _
     pn = p1;
   };
 #pragma unroll
-  for (int c = 0; c < 3; ++c) Ec[0][c] = ld(e0, c, (unsigned)pn * pbytes + own);
+  for (int c = 0; c < 3; ++c) Ec[0][c] = ld(e0, c, (OFF)pn * pbytes + own);
   fetch(A);
   auto put_e = [&]() {
 #pragma unroll
@@ -418,7 +418,7 @@ __global__ __launch_bounds__(64 * W) void k_fdtd_steps(RGrid g, T dt, const T* _
     }
     const int out = first + t - kLag;   // plane of the last stage
     if (valid && out >= ib && out < ie) {
-      const unsigned o = (unsigned)out * pbytes + own;
+      const OFF o = (OFF)out * pbytes + own;
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
         st(e1, c, o, es[S - 1][c]);
@@ -990,7 +990,7 @@ StepShape step_shape(const RGrid& v, int steps, size_t elem) {
   return best;
 }
 
-template <typename T, int S>
+template <typename T, typename OFF, int S>
 hipError_t launch_pass(const RGrid& v, const StepShape& shape, T dt, const void* ei, const void* hi, void* eo, void* ho, const void* eps,
                        double eps_s, const void* mu, double mu_s, hipStream_t s) {
   static_assert(kStepMaxSlab + 5 * S - 4 <= kStepTab, "x table");
@@ -998,12 +998,17 @@ hipError_t launch_pass(const RGrid& v, const StepShape& shape, T dt, const void*
   const long long nwork = step_tiles(v, shape.rows, S) * ((v.nx + slab - 1) / slab);
   const unsigned nb = (unsigned)(((nwork + 7) / 8) * 8);
 #define MX_STEP_CASE(EPS, MU)                                                                                   \
-  hipLaunchKernelGGL((k_fdtd_steps<T, W, S, EPS, MU>), dim3(nb), dim3(64, W), 0, s, v, dt, (const T*)ei,        \
+  hipLaunchKernelGGL((k_fdtd_steps<T, OFF, W, S, EPS, MU>), dim3(nb), dim3(64, W), 0, s, v, dt, (const T*)ei,        \
                      (const T*)hi, (T*)eo, (T*)ho, (const T*)eps, (T)eps_s, (const T*)mu, (T)mu_s, slab)
   auto go = [&](auto rows) {
     constexpr int W = decltype(rows)::value;
-    if (mu) { if (eps) MX_STEP_CASE(true, MU_FIELD); else MX_STEP_CASE(false, MU_FIELD); }
-    else if (mu_s == 1.0) { if (eps) MX_STEP_CASE(true, MU_ONE); else MX_STEP_CASE(false, MU_ONE); }
+    if constexpr (S == 1 || sizeof(OFF) == 4) {   // (single_steps)
+      if (mu) {
+        if (eps) MX_STEP_CASE(true, MU_FIELD); else MX_STEP_CASE(false, MU_FIELD);
+        return;
+      }
+    }
+    if (mu_s == 1.0) { if (eps) MX_STEP_CASE(true, MU_ONE); else MX_STEP_CASE(false, MU_ONE); }
     else { if (eps) MX_STEP_CASE(true, MU_SCALAR); else MX_STEP_CASE(false, MU_SCALAR); }
   };
   if constexpr (sizeof(T) == 4) {
@@ -1027,16 +1032,18 @@ bool separate_updates(const RGrid& v, int prec, bool mu_field) {
   const long long bytes = (mu_field ? 12ll : 9ll) * v.nx * v.ny * v.nz * (prec == MX_REAL64 ? 8 : 4);
   return v.nx == 1 || (v.nx == 2 && bytes <= (256ll << 20));
 }
-bool single_steps(const RGrid& v, int prec, bool mu_field) {
-  return v.nx <= 2 || (v.nx <= 4 && prec == MX_REAL64 && mu_field);
+// `wide`: 64-bit offsets (components of 4 GiB and more), which spill more with a mu field:
+// 840 x 805 x 800 with mu 34 ms a step in passes of two, 13.6 of one (without mu 7.8 of two).
+bool single_steps(const RGrid& v, int prec, bool mu_field, bool wide) {
+  return v.nx <= 2 || (prec == MX_REAL64 && mu_field && (v.nx <= 4 || wide));
 }
 
 // `steps` steps by passes of two, a last single one if their number is odd (or of one each):
 // (e, h) -> (e2, h2) -> (e, h) -> ...; *passes: how many
-template <typename T>
+template <typename T, typename OFF>
 hipError_t launch_steps(const RGrid& v, T dt, void* e, void* h, void* e2, void* h2, const void* eps, double eps_s,
                         const void* mu, double mu_s, int steps, int* passes, hipStream_t s) {
-  const bool single = single_steps(v, sizeof(T) == 8 ? MX_REAL64 : MX_REAL32, mu != nullptr);
+  const bool single = single_steps(v, sizeof(T) == 8 ? MX_REAL64 : MX_REAL32, mu != nullptr, sizeof(OFF) == 8);
   *passes = single ? steps : steps / 2 + steps % 2;
   const StepShape two = step_shape(v, 2, sizeof(T)), one = step_shape(v, 1, sizeof(T));
   for (int t = 0; t < *passes; ++t) {
@@ -1045,8 +1052,8 @@ hipError_t launch_steps(const RGrid& v, T dt, void* e, void* h, void* e2, void* 
     void* eo = (t & 1) ? e : e2;
     void* ho = (t & 1) ? h : h2;
     const hipError_t err = !single && 2 * t + 2 <= steps
-                               ? launch_pass<T, 2>(v, two, dt, ei, hi, eo, ho, eps, eps_s, mu, mu_s, s)
-                               : launch_pass<T, 1>(v, one, dt, ei, hi, eo, ho, eps, eps_s, mu, mu_s, s);
+                               ? launch_pass<T, OFF, 2>(v, two, dt, ei, hi, eo, ho, eps, eps_s, mu, mu_s, s)
+                               : launch_pass<T, OFF, 1>(v, one, dt, ei, hi, eo, ho, eps, eps_s, mu, mu_s, s);
     if (err != hipSuccess) return err;
   }
   return hipSuccess;
@@ -1089,8 +1096,7 @@ int mx_fdtd_run(const mx_fdtd_grid* g, int32_t prec, double dt, void* e, void* h
   if (steps == 0) return 0;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const size_t comp = (size_t)v.nx * v.ny * v.nz * (prec == MX_REAL64 ? 8 : 4), bytes = 3 * comp;
-  // (a component of 4 GiB is beyond the passes' 32-bit offsets)
-  if (comp >= (size_t)1 << 32 || mx::separate_updates(v, prec, mu != nullptr)) {
+  if (mx::separate_updates(v, prec, mu != nullptr)) {
     for (int t = 0; t < steps; ++t) {
       hipError_t err = mx::launch_h(v, prec, dt, e, h, mu, mu_scalar, s);
       if (err == hipSuccess) err = mx::launch_e(v, prec, dt, e, h, eps, eps_scalar, s);
@@ -1105,9 +1111,11 @@ int mx_fdtd_run(const mx_fdtd_grid* g, int32_t prec, double dt, void* e, void* h
   hipError_t err = hipMallocAsync(&e2, bytes, s);
   if (err == hipSuccess) err = hipMallocAsync(&h2, bytes, s);
   if (err == hipSuccess)
-    err = prec == MX_REAL64
-              ? mx::launch_steps<double>(v, dt, e, h, e2, h2, eps, eps_scalar, mu, mu_scalar, steps, &passes, s)
-              : mx::launch_steps<float>(v, (float)dt, e, h, e2, h2, eps, eps_scalar, mu, mu_scalar, steps, &passes, s);
+    err = prec == MX_REAL32
+              ? mx::launch_steps<float, unsigned>(v, (float)dt, e, h, e2, h2, eps, eps_scalar, mu, mu_scalar, steps, &passes, s)
+          : comp < (size_t)1 << 32
+              ? mx::launch_steps<double, unsigned>(v, dt, e, h, e2, h2, eps, eps_scalar, mu, mu_scalar, steps, &passes, s)
+              : mx::launch_steps<double, size_t>(v, dt, e, h, e2, h2, eps, eps_scalar, mu, mu_scalar, steps, &passes, s);
   if (err == hipSuccess && (passes & 1)) {   // the last pass wrote the second pair
     err = hipMemcpyAsync(e, e2, bytes, hipMemcpyDeviceToDevice, s);
     if (err == hipSuccess) err = hipMemcpyAsync(h, h2, bytes, hipMemcpyDeviceToDevice, s);
