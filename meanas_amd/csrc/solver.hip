@@ -157,17 +157,26 @@ int op_kind(const mx_operator& op) { return mat_kind(view_of<double>(op).flags);
 //   64^3 x4 89 / 77, x8 158 / 151, 72^3 x4 122 / 134: the line is at 512 tiles (64^3);
 //   partly empty tiles (padded / cells): 12^3 (2.4) 168 / 115, 25^3 (2.1) 157 / 154,
 //   33^3 (1.8) 133 / 137, 41^3 (1.6) 116 / 126, 43^3 (1.4) 115 / 117, 37^3 (1.3) 127 / 121,
-//   52^3 (1.2) 121 / 125, 61^3 (1.15) 144 / 150, 63^3 (1.05) 152 / 159: any up to 72 tiles, at
-//   most 1.4 up to 216, at most 1.04 above.
+//   52^3 (1.2) 121 / 125, 61^3 (1.15) 144 / 150, 63^3 (1.05) 152 / 159: any up to 72 tiles (but
+//   for the next line), at most 1.4 up to 216, at most 1.04 above.
+// Grids that are short along x or y and long along z leave the tiles empty and fill the three
+// launches' rows of 64 lanes.  With R = tile slots / lanes of those rows, batches of 2048 tiles,
+// three launches / one: 1x64x64 (64 tiles, R 8) 36 / 45, 64x1x64 41 / 47, 1x32x64 (32, 8) 44 / 52, 2x64x64
+// (64, 4) 45 / 48, 9x9x128 (64, 3.2) 52 / 56, 20x20x62 (72, 1.4) 74 / 83, 12x32x60 (64, 1.3) 78 / 90;
+// 13x20x62 (48, 1.5) 78 / 79, 5x48x64 (48, 1.6) 77 / 68, 4x32x64 (32, 2) 69 / 63, 1x32x32 (16, 4) 64 / 66, 1x16x16 (4, 4)
+// 168 / 146, 25^3 (64, 0.8) 75 / 61; along z, 64x64x1 (64, 0.1) x64 287 / 89.  The line is at tiles x R = 80.
+// Alone the grids that it turns away would take 10 us instead of 23.
 // What that line gives away: alone 60^3 would take 22 us instead of 39, 52^3 21 instead of 33.
 // What it costs: an odd batch of 5 or more near the upper line ends with a group of one
 // system (48x48x95 x9 168 / 177, 64^3 x7 139 / 138, x5 107 / 101).
-constexpr int kIterTiles = 512, kIterFillTiles = 216, kIterAnyFill = 72;
+constexpr int kIterTiles = 512, kIterFillTiles = 216, kIterAnyFill = 72, kIterFlat = 80;
 bool one_launch(const mx_operator& op, int mode) {
   if (mode != MX_FP64) return false;
   const long long tiles = iter_blocks(op.nx, op.ny, op.nz);
   const long long padded = tiles * kIterTileCells * 100, cells = ncell_of(op);
-  return tiles <= kIterAnyFill || (tiles <= kIterFillTiles && padded <= 140 * cells) ||
+  const long long lanes = (long long)op.nx * op.ny * ((op.nz + 63) / 64 * 64);
+  if (tiles <= kIterAnyFill) return tiles * tiles * kIterTileCells <= kIterFlat * lanes;
+  return (tiles <= kIterFillTiles && padded <= 140 * cells) ||
          (tiles <= kIterTiles && padded <= 104 * cells);
 }
 // Iterations per chunk of a batch of such systems

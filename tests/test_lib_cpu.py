@@ -320,3 +320,17 @@ def test_wave_operators_refuse_host_tensors():
               sources.e_boundary_source(eps, 0.3, dxes, eps, device='cpu')):
         with pytest.raises(ValueError, match='CUDA tensor'):
             f(v)
+
+
+@pytest.mark.parametrize('shape,one', [((16, 16, 16), True), ((64, 64, 1), True), ((25, 25, 25), True), ((64, 64, 64), True),
+                                       ((64, 1, 64), False), ((1, 64, 64), False), ((2, 64, 64), False), ((20, 20, 62), False),
+                                       ((5, 48, 64), True), ((60, 60, 60), False), ((72, 72, 72), False)])
+def test_which_grids_run_one_launch_an_iteration(shape, one):
+    """The workspace of a complex128 system tells its form: five vectors for three launches, eight
+    for one.  Grids that leave the tiles empty and fill the three launches' rows keep those."""
+    from meanas_amd import _lib
+    op = _lib.MxOperator(*shape, 0, 0.0, 0.0, None, None, None, None, None, None, None)
+    vector = 3 * 16 * int(numpy.prod(shape))
+    tables = 300_000   # states and partial sums: below this, whatever the grid
+    got = _lib.lib().mx_work_bytes(ctypes.byref(op), _lib.MX_FP64)
+    assert (8 if one else 5) * vector <= got < (8 if one else 5) * vector + tables
