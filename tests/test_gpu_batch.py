@@ -439,3 +439,53 @@ def test_server_matches_generic():
     E = solvers.generic(r.omega, r.dxes, r.J, r.epsilon, matrix_solver='cocg_fp64',
                         matrix_solver_opts=dict(rtol=1e-9))
     assert numpy.linalg.norm(res.E - E) <= 1e-7 * numpy.linalg.norm(E)
+
+
+# ---- the three-launch form of a complex128 batch -------------------------------------
+THREE_LAUNCH = (33, 33, 17)   # 75 tiles half empty: too many for one launch per iteration
+
+
+@pytest.mark.parametrize('check', ['multi_rhs', 'merged', 'kept_plans'])
+def test_three_launch_systems(check, monkeypatch):
+    """The checks above whose small grids run one launch per iteration, on a grid that runs
+    three: batch equal to alone, merged finishing launches, kept plans."""
+    from meanas_amd import _lib
+    from meanas_amd.fdfd.device import DeviceOperator
+    small = small_aniso
+    omega, dxes, eps, _ = small(THREE_LAUNCH, 1)
+    op = DeviceOperator(omega, dxes, eps)
+    assert op.work_bytes(_lib.MX_FP64) < 7 * 16 * op.n3   # five vectors, not eight
+    monkeypatch.setitem(globals(), 'small_aniso', lambda nrhs=4: small(THREE_LAUNCH, nrhs))
+    if check == 'multi_rhs':
+        test_multi_rhs_batch('fp64')
+    elif check == 'merged':
+        test_merged_finishing_equals_separate('aniso_batch', monkeypatch)
+    else:
+        test_kept_plans_equal_fresh_plans(monkeypatch)
+
+
+def test_three_launch_system_that_loses_track(monkeypatch):
+    """A near-static system of three launches loses track and continues in the classic form:
+    the same bits with merged and separate finishing launches, and from a kept plan."""
+    import torch
+    from meanas_amd import _lib
+    from meanas_amd.fdfd.device import DeviceOperator, solve_batch
+    omega = 1 / 1500
+    eps = numpy.ones((3, *THREE_LAUNCH))
+    eps[:, 2:20, 2:9, 2] = 2.5
+    dxes = [[numpy.full(n, 1.5) for n in THREE_LAUNCH] for _ in range(2)]
+    J = numpy.zeros((3, *THREE_LAUNCH), dtype=complex)
+    J[:, 3, 3, 3] = 1 + 1j
+    J[:, 1, 1, 1] = 1 - 1j
+    op = DeviceOperator(omega, dxes, eps.ravel())
+    b = op.map(_lib.MX_MAP_RHS, torch.from_numpy(J.ravel()).cuda(), coef=-1j * omega)
+    x = torch.zeros_like(b)
+    work = torch.empty(op.work_bytes(_lib.MX_FP64), dtype=torch.uint8, device=b.device)
+    runs = []
+    for merged in ('1', '1', '0', '0'):
+        monkeypatch.setenv('MEANAS_AMD_MERGED_FIN', merged)
+        x.zero_()
+        st = solve_batch([op], [dict(op=0, b=b, x=x, work=work, rtol=1e-11, maxiter=1500)], mode=_lib.MX_FP64)
+        runs.append((x.clone(), st[0]))
+    for y, st in runs[1:]:
+        assert torch.equal(y, runs[0][0]) and st == runs[0][1]
