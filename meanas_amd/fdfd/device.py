@@ -4,7 +4,8 @@ A `DeviceOperator` holds, in HBM, everything the kernels need to apply the
 symmetrised wave operator A = Pl e_full Pr of meanas.fdfd.solvers.generic
 (reference fdfd/solvers.py:116-125, fdfd/operators.py:40-123) matrix-free:
   * a per-axis coefficient table: fa, fb (scaled forward differences), se, sh
-    (square roots of the E- and H-grid widths, i.e. the separable factors of p);
+    (square roots of the E- and H-grid widths, i.e. the separable factors of p), and the
+    widths themselves (for the unscaled operator);
   * epsilon, stored once if the three components are equal (isotropic) and as a real
     array if it has no imaginary part;
   * 1/mu (optional), with the same compaction;
@@ -82,7 +83,8 @@ def operator_flags(shape, epsilon, mu=None, pec=None, pmc=None) -> int:
 def device_bytes(shape, flags: int, mode: int) -> int:
     """HBM bytes one solve of this operator holds: the per-axis tables and the materials
     in both precisions, the mask, b and x (complex128) plus the source upload, and the
-    solver workspace (mx_work_bytes, a host query)."""
+    solver workspace (mx_work_bytes, a host query).  The cell widths (32 bytes a plane of
+    each axis) are not counted."""
     nx, ny, nz = (int(v) for v in shape)
     n = nx * ny * nz
 
@@ -126,9 +128,16 @@ class DeviceOperator:
         self.device = torch.device(device)
         flags = 0
 
-        coef = coefficient_table(dxes)
-        self.coef64 = _to_device(coef.view(numpy.float64), torch.float64, self.device)
-        self.coef32 = _to_device(coef.astype(numpy.complex64).view(numpy.float32), torch.float32, self.device)
+        # the coefficients in both precisions and the cell widths, in one upload
+        coef = coefficient_table(dxes).view(numpy.float64)
+        coef32 = coef.astype(numpy.float32)
+        widths = numpy.concatenate([numpy.asarray(d, dtype=numpy.complex128).reshape(-1) for side in dxes for d in side])
+        tables = _to_device(numpy.concatenate([coef.reshape(-1), widths.view(numpy.float64),
+                                               coef32.reshape(-1).view(numpy.float64)]), torch.float64, self.device)
+        n = coef.shape[0]   # nx + ny + nz
+        self.coef64 = tables[:8 * n].view(n, 8)
+        self.widths = tables[8 * n:12 * n]
+        self.coef32 = tables[12 * n:].view(torch.float32).view(n, 8)
 
         eps, cplx, aniso = _material(epsilon, self.ncell, 'epsilon')
         flags |= (_lib.MX_EPS_COMPLEX if cplx else 0) | (_lib.MX_EPS_ANISO if aniso else 0)
@@ -159,6 +168,13 @@ class DeviceOperator:
         self.desc = _lib.MxOperator(nx, ny, nz, flags, w2.real, w2.imag,
                                     ptr(self.coef32), ptr(self.coef64), ptr(self.eps32), ptr(self.eps64),
                                     ptr(self.inv_mu32), ptr(self.inv_mu64), ptr(self.mask))
+
+    def grid_desc(self) -> '_lib.MxGrid':
+        """The mx_grid of this operator's cell widths."""
+        nx, ny, nz = self.shape
+        ptrs = [self.widths.data_ptr() + 16 * k for k in (0, nx, nx + ny)]
+        side = 16 * (nx + ny + nz)
+        return _lib.MxGrid(nx, ny, nz, 0, (ctypes.c_void_p * 3)(*ptrs), (ctypes.c_void_p * 3)(*[p + side for p in ptrs]))
 
     def _pair(self, arr: numpy.ndarray, is_complex: bool):
         if is_complex:

@@ -253,13 +253,13 @@ class _A0:
     def __init__(self, omega, dxes, epsilon, mu, pec, pmc, device, reversed: bool = False):
         self.op = DeviceOperator(omega, dxes, numpy.asarray(epsilon).reshape(-1), mu=_vec_or_none(mu),
                                  pec=_vec_or_none(pec), pmc=_vec_or_none(pmc), device=device)
-        self.grid = _Grid(dxes, device)
+        self.grid = self.op.grid_desc()
         self.reversed = 1 if reversed else 0
 
     def __call__(self, x: torch.Tensor) -> torch.Tensor:
         self.op._check_vec(x, torch.complex128)
         y = torch.empty_like(x)
-        _lib.check(_lib.lib().mx_wave(ctypes.byref(self.op.desc), ctypes.byref(self.grid.desc), self.reversed,
+        _lib.check(_lib.lib().mx_wave(ctypes.byref(self.op.desc), ctypes.byref(self.grid), self.reversed,
                                       x.data_ptr(), y.data_ptr(), torch_stream_handle()), 'mx_wave')
         return y
 

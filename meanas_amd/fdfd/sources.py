@@ -26,7 +26,7 @@ import torch
 
 from .. import _lib
 from .device import DeviceOperator, grid_shape, torch_stream_handle
-from .functional import _flat, _Grid
+from .functional import _flat
 
 
 def _field_mask(mask, n3: int, ncell: int) -> numpy.ndarray:
@@ -65,7 +65,7 @@ def _masked_source(omega, dxes, epsilon, mu, device, q, keep) -> Callable:
     """`f(E) -> keep (A0 q E - q A0 E) / (-i omega)` for the 3N host masks q and keep (or
     None), one pass over the field."""
     op = DeviceOperator(omega, dxes, epsilon, mu=mu, device=device)
-    grid = _Grid(dxes, device)
+    grid = op.grid_desc()
     q = torch.from_numpy(q).to(op.device)
     keep = None if keep is None else torch.from_numpy(keep).to(op.device)
     c = 1.0 / (-1j * complex(omega))
@@ -74,7 +74,7 @@ def _masked_source(omega, dxes, epsilon, mu, device, q, keep) -> Callable:
         et, like = _to_dev(e, op)
         op._check_vec(et, torch.complex128)
         j = torch.empty_like(et)
-        _lib.check(_lib.lib().mx_wave_source(ctypes.byref(op.desc), ctypes.byref(grid.desc), q.data_ptr(),
+        _lib.check(_lib.lib().mx_wave_source(ctypes.byref(op.desc), ctypes.byref(grid), q.data_ptr(),
                                              None if keep is None else keep.data_ptr(), c.real, c.imag,
                                              et.data_ptr(), j.data_ptr(), torch_stream_handle()), 'mx_wave_source')
         return _from_dev(j, like)
