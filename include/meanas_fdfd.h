@@ -267,10 +267,11 @@ int mx_fdtd_h(const mx_fdtd_grid* g, int32_t prec, double dt, const void* e, voi
 int mx_fdtd_e(const mx_fdtd_grid* g, int32_t prec, double dt, void* e, const void* h, const void* eps,
               double eps_scalar, void* stream);
 /* `steps` leapfrog steps: maxwell_h then maxwell_e, as the reference's update loop
- * (meanas/test/test_fdtd.py:215-233) runs them, without sources.  Each step is one fused
- * pass that gives the same bits as mx_fdtd_h followed by mx_fdtd_e; the passes alternate
- * between (e, h) and a second pair of fields that the call allocates and frees in stream
- * order (hipMallocAsync, 2 x 3N values), and the result ends in (e, h). */
+ * (meanas/test/test_fdtd.py:215-233) runs them, without sources, with the same bits as
+ * mx_fdtd_h followed by mx_fdtd_e.  A pass does two steps (a last odd one, and small or
+ * very large cases, one); passes alternate between (e, h) and a second pair of fields that
+ * the call allocates and frees in stream order (hipMallocAsync, 2 x 3N values), and the
+ * result ends in (e, h).  Grids of one x plane, or two small ones, run the two updates. */
 int mx_fdtd_run(const mx_fdtd_grid* g, int32_t prec, double dt, void* e, void* h, const void* eps,
                 double eps_scalar, const void* mu, double mu_scalar, int32_t steps, void* stream);
 
@@ -347,7 +348,8 @@ int mx_fdtd_poynting_divergence(const mx_fdtd_grid* g, int32_t prec, const void*
  * us_out[0] operator apply (COCG epilogue), [1] its finishing kernel, [2] the vector
  * update, [3] its finishing kernel, [4] the direction update of the classic form
  * (a no-op launch for MX_FP64 systems in the fused form).  Fills min(n_out, 5) entries.
- * x and the workspace are overwritten. */
+ * A small MX_FP64 system that mx_solve runs with one launch per iteration is timed in this
+ * form all the same.  x and the workspace are overwritten. */
 int mx_time_kernels(const mx_operator* op, const mx_system* sys, const mx_options* opt, int32_t reps,
                     double* us_out, int32_t n_out, void* stream);
 

@@ -301,7 +301,10 @@ __global__ __launch_bounds__(64 * TY, (kWavesPerSimd<T, MK>)) void k_apply(const
     for (int c = 0; c < 3; ++c) epsv[c] = epsn[SM ? 0 : c];
     const FaFb<T> cxi = coef_u(cx, i);
     const cplx<T> fa_xm = coef_u(cx, wrapi(i - 1, nx)).fa;
-    __syncthreads();   // plane i is in LDS; the previous step's reads of sH are done
+    // plane i is in LDS; the previous step's reads of sH are done.  (The barrier heads the loop
+    // body, where a compiler has been seen to leave out the wait for LDS writes: here the reads of
+    // sH after commit() in the step before, which wait for it, stand between.)
+    __syncthreads();
 
     const int r = ty + 1, q = tz + 1;
     cplx<T> ec[3] = {e_(0, r, q), e_(1, r, q), e_(2, r, q)};

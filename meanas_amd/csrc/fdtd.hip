@@ -6,8 +6,9 @@
 // differences (f[n+1] - f[n]) / dx_e[n] and backward differences (f[n] - f[n-1]) / dx_h[n],
 // unit widths when the grid gives none.  Materials divide, as the reference does.
 //
-// The updates, the CPML and the energy kernels march along x, a thread per (y, z) column
-// (see Column); runs of several steps pipeline two steps per pass (k_fdtd_steps).
+// The updates, the CPML and the divergence march along x, a thread per (y, z) column, or have a
+// thread per cell, as energy and flux do (see Column); runs of several steps pipeline two steps
+// per pass (k_fdtd_steps).
 #include <algorithm>
 #include <cstdlib>
 #include <string>
@@ -444,9 +445,10 @@ __global__ __launch_bounds__(64 * W) void k_fdtd_steps(RGrid g, T dt, const T* _
       }
     }
     put_e();
-    // the barrier ends the step: as the first instruction of the loop it came without the
-    // wait for the LDS writes of the step before (read in the assembly of this build), and
-    // a row's old values were read now and then
+    // the barrier ends the step, in straight line with the LDS writes before it.  A form of this
+    // kernel with the barrier as the loop's first instruction was compiled without the wait for
+    // the writes on the back edge (seen in its assembly), and a row's old values were read now
+    // and then; in the present build every barrier of the library comes after its wait
     __syncthreads();
   };
   int t = 0;
@@ -459,7 +461,7 @@ __global__ __launch_bounds__(64 * W) void k_fdtd_steps(RGrid g, T dt, const T* _
 }
 
 // ---- convolutional PML (fdtd/pml.py:96-230) ---------------------------------------
-// One thread per cell.  The six derivatives d_a f_c (a != c) use dx_h along every axis.
+// The six derivatives d_a f_c (a != c) use dx_h along every axis.
 // Each layer the cell lies in (in the table's order: axis 0..2, polarity -1 then +1)
 // scales the two derivatives along its axis by p2, advances the cell's psi_u, psi_v
 // (u < v the components other than the axis) with p0 and p1, stores them in the psi
@@ -691,9 +693,9 @@ __global__ __launch_bounds__(kFB) void k_conducting(int nx, int ny, int nz, int 
 // component sum in the field precision (in component order, starting from the x term),
 // the widths in double (the float64 width arrays promote) multiplied one axis at a time,
 // and nothing contracted into fused multiply-adds.  `form` is one of MX_ENERGY_*.
-// HBM-bound, a thread per cell.  256^3: energy_hstep float64 303 us, float32 164 us (327 / 177
-// with the index divisions' neighbours reloaded and each component's loads behind the one
-// before; columns marching along x 343 / 188); poynting 211 / 104 us (224 / 113; columns 231 / 118).
+// HBM-bound, a thread per cell, every load of a cell before any is used.  256^3: energy_hstep
+// float64 303 us, float32 162 us (327 / 177 with each component's loads behind the one before;
+// columns marching along x 343 / 188); poynting 211 / 104 us (224 / 113; columns 231 / 118).
 
 template <typename T>
 __global__ __launch_bounds__(kFB) void k_energy(RGrid g, int form, T dt, const T* __restrict__ f0,

@@ -182,8 +182,9 @@ bool one_launch(const mx_operator& op, int mode) {
 // Iterations per chunk of a batch of such systems
 constexpr int kOneLaunchChunk = 32;
 
-// One finishing launch per fused iteration (default); MEANAS_AMD_MERGED_FIN=0 launches
-// the post-apply and post-update finishing kernels separately (same results).
+// One finishing launch per fused iteration of three launches (default); MEANAS_AMD_MERGED_FIN=0
+// launches the post-apply and post-update finishing kernels separately (same results).
+// One-launch iterations have none.
 bool merged_fin_enabled() {
   const char* v = getenv("MEANAS_AMD_MERGED_FIN");
   return !(v && v[0] == '0');

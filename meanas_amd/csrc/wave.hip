@@ -238,8 +238,8 @@ __global__ __launch_bounds__(64 * ROWS) void k_wave(OpView<double> op, Widths wd
     take(cur);
     M = Mn;
     p = p1;
-    // the barrier ends the step, in straight line with the LDS writes (at the head of a
-    // loop this compiler leaves out the wait for them)
+    // the barrier ends the step, in straight line with the LDS writes (k_fdtd_steps, fdtd.hip,
+    // says why)
     __syncthreads();
   };
   int t = 0;

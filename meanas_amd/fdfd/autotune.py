@@ -13,6 +13,9 @@ memory and in a JSON cache file.  Shapes within 3% of the fastest (timing noise)
 ranked by a fixed preference (4-row tiles, then the deepest slab), so that near-ties
 resolve the same way on every box.
 
+A small complex128 system that runs one launch per iteration uses its tiling for the
+residual replacements only.
+
 A system's block partition -- and so the order of its reductions -- depends on that
 system alone (its shape and materials through this table), never on the rest of a
 batch, so a system gives the same bits alone and in any batch.

@@ -392,7 +392,9 @@ KERNEL_NAMES = ('apply', 'fin_apply', 'update', 'fin_update', 'pupdate')
 def time_kernels(op: DeviceOperator, b: torch.Tensor, mode: int = _lib.MX_FP64, reps: int = 50,
                  slab: int | None = None, stream=None, tile_rows: int = 0, form: str = 'auto') -> dict:
     """Average microseconds per launch of each kernel of one solver iteration
-    (`mx_time_kernels`), timed with HIP events on `stream` on the system A x = b.
+    (`mx_time_kernels`), timed with HIP events on `stream` on the system A x = b.  A small
+    complex128 system that a solve runs with one launch per iteration is timed in the form of
+    separate launches all the same.
     The tiling is the one a solve of this operator uses (the autotuned tile height and slab
     depth unless given)."""
     op._check_vec(b, torch.complex128)
