@@ -693,9 +693,10 @@ __global__ __launch_bounds__(kFB) void k_conducting(int nx, int ny, int nz, int 
 // component sum in the field precision (in component order, starting from the x term),
 // the widths in double (the float64 width arrays promote) multiplied one axis at a time,
 // and nothing contracted into fused multiply-adds.  `form` is one of MX_ENERGY_*.
+
 // HBM-bound, a thread per cell, every load of a cell before any is used.  256^3: energy_hstep
-// float64 303 us, float32 162 us (327 / 177 with each component's loads behind the one before;
-// columns marching along x 343 / 188); poynting 211 / 104 us (224 / 113; columns 231 / 118).
+// with widths float64 314 us, float32 163 us (358 / 208 with each component's loads behind the
+// one before; columns marching along x 345 / 189), without widths 303 / 162 us (327 / 177; 343 / 188).
 
 template <typename T>
 __global__ __launch_bounds__(kFB) void k_energy(RGrid g, int form, T dt, const T* __restrict__ f0,
@@ -744,26 +745,39 @@ __global__ __launch_bounds__(kFB) void k_energy(RGrid g, int form, T dt, const T
 // s = E(+1) x H with both width-weighted (fdtd/energy.py:10-87): s_x = ey(i+1) hz - ez(i+1) hy
 // and cyclically, E taken at the next cell along the component's axis (periodic), in
 // double, stored in the field precision.
-template <typename T>
+// HBM-bound.  With widths in columns, which load the y and z ones once: 256^3 float64 235 us,
+// float32 120 us (256 / 134 before; a thread per cell 254 / 127); without, a thread per cell:
+// 211 / 104 us (224 / 113; columns 231 / 118).
+template <typename T, typename OFF>
 __global__ __launch_bounds__(kFB) void k_poynting(RGrid g, const T* __restrict__ e, const T* __restrict__ h,
-                                                  T* __restrict__ s, int order) {
+                                                  T* __restrict__ s, int slab) {
 #pragma clang fp contract(off)
-  const Column col = column<size_t>(g, order);
+  const Column col = column<OFF>(g, slab);
   if (!col.ok) return;
-  const int i = col.ib, nx = g.nx, ny = g.ny, nz = g.nz, plane = ny * nz, nc = nx * plane, cell = i * plane + col.t;
-  const int xn = cell + (i + 1 == nx ? -i : 1) * plane;
-  const int yn = cell + (col.j + 1 == ny ? -col.j : 1) * nz, zn = cell + (col.k + 1 == nz ? -col.k : 1);
-  const T h0 = h[cell], h1 = h[nc + cell], h2 = h[2 * nc + cell];
-  const T eyx = e[nc + xn], ezx = e[2 * nc + xn], ezy = e[2 * nc + yn], exy = e[yn], exz = e[zn], eyz = e[nc + zn];
-  const double wex = width(g.dxe[0], i), wey = width(g.dxe[1], col.j), wez = width(g.dxe[2], col.k);
-  const double hx = (double)h0 * width(g.dxh[0], i), hy = (double)h1 * width(g.dxh[1], col.j);
-  const double hz = (double)h2 * width(g.dxh[2], col.k);
-  const double s0 = ((double)eyx * wey) * hz - ((double)ezx * wez) * hy;
-  const double s1 = ((double)ezy * wez) * hx - ((double)exy * wex) * hz;
-  const double s2 = ((double)exz * wex) * hy - ((double)eyz * wey) * hx;
-  s[cell] = (T)s0;
-  s[nc + cell] = (T)s1;
-  s[2 * nc + cell] = (T)s2;
+  const int nx = g.nx, ny = g.ny, nz = g.nz;
+  const size_t plane = (size_t)ny * nz, nc = nx * plane;
+  const int jn = col.j + 1 == ny ? 0 : col.j + 1, kn = col.k + 1 == nz ? 0 : col.k + 1;
+  const OFF own0 = (OFF)col.t * (OFF)sizeof(T);
+  const OFF oy0 = ((OFF)jn * (OFF)nz + (OFF)col.k) * (OFF)sizeof(T);
+  const OFF oz0 = ((OFF)col.j * (OFF)nz + (OFF)kn) * (OFF)sizeof(T);
+  const double wey = width(g.dxe[1], col.j), wez = width(g.dxe[2], col.k);
+  const double why = width(g.dxh[1], col.j), whz = width(g.dxh[2], col.k);
+#pragma unroll 1
+  for (int i = col.ib; i < col.ie; ++i) {
+    const OFF own = in_loop(own0), oy = in_loop(oy0), oz = in_loop(oz0);
+    const size_t pi = i * plane, pn = (size_t)(i + 1 == nx ? 0 : i + 1) * plane;
+    const T h0 = at(h, pi, own), h1 = at(h, nc + pi, own), h2 = at(h, 2 * nc + pi, own);
+    const T eyx = at(e, nc + pn, own), ezx = at(e, 2 * nc + pn, own), ezy = at(e, 2 * nc + pi, oy), exy = at(e, pi, oy);
+    const T exz = at(e, pi, oz), eyz = at(e, nc + pi, oz);
+    const double wex = width_x<OFF>(g.dxe[0], i);
+    const double hx = (double)h0 * width_x<OFF>(g.dxh[0], i), hy = (double)h1 * why, hz = (double)h2 * whz;
+    const double s0 = ((double)eyx * wey) * hz - ((double)ezx * wez) * hy;
+    const double s1 = ((double)ezy * wez) * hx - ((double)exy * wex) * hz;
+    const double s2 = ((double)exz * wex) * hy - ((double)eyz * wey) * hx;
+    put(s, pi, own, (T)s0);
+    put(s, nc + pi, own, (T)s1);
+    put(s, 2 * nc + pi, own, (T)s2);
+  }
 }
 
 // ds = sum_a (s_a - s_a(previous cell along a)), unit spacing (deriv_back() without
@@ -806,8 +820,9 @@ bool rgrid(const mx_fdtd_grid* g, RGrid* v, std::string* why) {
 
 // Launch of a kernel with a thread per cell (the 64-bit form of `column`).  Work goes by XCD
 // where nine values a cell stay in the 256 MB cache, else in the order of the blocks, as the
-// memory channels like it better: Poynting flux of 100 x 110 x 120 in float64 15.3 us by XCD,
-// 20.7 plain; 256^3 float64 237 / 211 us, float32 114 / 104; energy of 256^3 float64 330 / 303 us.
+// memory channels like it better: Poynting flux without widths of 100 x 110 x 120 in float64
+// 15.3 us by XCD, 20.7 plain; 256^3 float64 237 / 211 us, float32 114 / 104; energy of 256^3 float64
+// 330 / 303 us.
 struct ColumnGrid { bool marches; int slab; unsigned blocks; };
 ColumnGrid cell_grid(const RGrid& v, int prec) {
   const long long cells = (long long)v.nx * v.ny * v.nz, bytes = 9 * cells * (prec == MX_REAL64 ? 8 : 4);
@@ -892,11 +907,13 @@ hipError_t launch_energy(const RGrid& v, int prec, int form, double dt, const vo
 }
 
 hipError_t launch_poynting(const RGrid& v, int prec, const void* e, const void* h, void* out, hipStream_t s) {
-  const ColumnGrid cg = cell_grid(v, prec);
-#define MX_POYNTING_CASE(T) \
-  hipLaunchKernelGGL(k_poynting<T>, dim3(cg.blocks), dim3(kFB), 0, s, v, (const T*)e, (const T*)h, (T*)out, cg.slab)
-  if (prec == MX_REAL64) MX_POYNTING_CASE(double);
-  else MX_POYNTING_CASE(float);
+  bool widths = false;
+  for (int a = 0; a < 3; ++a) widths = widths || v.dxe[a] || v.dxh[a];
+  const ColumnGrid cg = widths ? column_grid(v, prec, 6) : cell_grid(v, prec);
+#define MX_POYNTING_CASE(T, OFF)                                                                                        \
+  hipLaunchKernelGGL((k_poynting<T, OFF>), dim3(cg.blocks), dim3(kFB), 0, s, v, (const T*)e, (const T*)h, (T*)out, cg.slab)
+  if (prec == MX_REAL64) { if (cg.marches) MX_POYNTING_CASE(double, unsigned); else MX_POYNTING_CASE(double, size_t); }
+  else { if (cg.marches) MX_POYNTING_CASE(float, unsigned); else MX_POYNTING_CASE(float, size_t); }
 #undef MX_POYNTING_CASE
   return hipGetLastError();
 }

@@ -672,6 +672,11 @@ def test_large_grids_on_both_sides_of_the_cache(dtype, shape):
     nx, ny, nz = [torch.roll(e, -1, a) for a in (1, 2, 3)]
     torch.testing.assert_close(fdtd.poynting(e, h), torch.stack([nx[1] * h[2] - nx[2] * h[1], ny[2] * h[0] - ny[0] * h[2],
                                                                  nz[0] * h[1] - nz[1] * h[0]]), **tol)
+    w = [[torch.as_tensor(d).cuda().reshape([-1 if b == a else 1 for b in range(3)]) for a, d in enumerate(side)] for side in dxes]
+    hw = [h[a].double() * w[1][a] for a in range(3)]
+    flux = [nx[1] * w[0][1] * hw[2] - nx[2] * w[0][2] * hw[1], ny[2] * w[0][2] * hw[0] - ny[0] * w[0][0] * hw[2],
+            nz[0] * w[0][0] * hw[1] - nz[1] * w[0][1] * hw[0]]
+    torch.testing.assert_close(fdtd.poynting(e, h, dxes), torch.stack(flux).to(dtype), **tol)
     want_h = _plain_step(e, h, 0.2, dxes, None, eps, 'h')[1]
     want_e = _plain_step(e, h, 0.2, dxes, eps, None, 'e')[0]
     torch.testing.assert_close(fdtd.maxwell_h(0.2, dxes)(e, h.clone(), eps), want_h, **tol)
