@@ -97,7 +97,7 @@ def test_merged_finishing_equals_separate(case, monkeypatch):
         assert all(s['status'] == 'converged' for s in sm), sm
 
 
-def test_given_check_interval_stands_beside_the_automatic_chunk():
+def test_given_check_interval_stands_beside_the_automatic_chunk(monkeypatch):
     """A batch of one-launch systems runs chunks of 32 iterations unless told otherwise; the
     caller's check_every stands with them.  Options that resolve alike share a kept plan."""
     import torch
@@ -108,6 +108,7 @@ def test_given_check_interval_stands_beside_the_automatic_chunk():
     b = op.map(_lib.MX_MAP_RHS, torch.from_numpy(Js[0]).cuda(), coef=-1j * omega)
     x = torch.zeros_like(b)
     work = torch.empty(op.work_bytes(_lib.MX_FP64), dtype=torch.uint8, device=b.device)
+    monkeypatch.setenv('MEANAS_AMD_PLAN_CACHE', '1')
 
     def reused(**options):
         before = _lib.lib().mx_solve_plan_reuses()
